@@ -2,15 +2,12 @@
 // and the C write-side block packing, for gfx950.
 //
 // Decode is two launches:
-//   k_lz4_streams   one 64-lane wavefront per LZ4 stream.  The token stream is
-//                   parsed uniformly by all lanes (every lane holds the same
-//                   ip/op, loads of one address are broadcast), literal runs
-//                   and matches are copied by the 64 lanes together.  A match
-//                   copies out[op+i] = out[op-off + (i mod off)], so every
-//                   source byte precedes op and one match never depends on
-//                   itself; stores of earlier sequences are made visible with
-//                   a workgroup-scope release/acquire only when the match
-//                   source overlaps bytes stored since the last such fence.
+//   k_lz4_streams   one workgroup per LZ4 stream, of 8, 4 or 1 wavefronts by
+//                   the number of streams.  Input positions are decoded as
+//                   sequence headers all at once, the sequences really there
+//                   are picked out by following them from every start, and
+//                   output bytes are produced one a lane, whatever sequences
+//                   they belong to.
 //   k_unfilter      one workgroup per block: gathers each element's bytes from
 //                   its byte planes (byte shuffle) or bit planes (bitshuffle,
 //                   8x8 bit-matrix transposes), and writes the element into its
@@ -21,9 +18,11 @@
 // chunks).
 #include "iamx_internal.h"
 
-#include <stdlib.h>
 
 namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));  // at any address
 
 // Delta-swap transpose of an 8x8 bit matrix held in a uint64 (row r = byte r,
 // column c = bit c): bit 8r+c moves to bit 8c+r (Hacker's Delight, 7-3).
@@ -42,386 +41,704 @@ __device__ __forceinline__ uint32_t rdlane(uint32_t v, int32_t l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
 }
 
-// One wavefront per LZ4 stream.
-//   input   the wave keeps 1 KiB of the compressed stream in four VGPRs (lane
-//           l of w[k] holds bytes wb+256k+4l..+3); sequence headers are parsed
-//           uniformly with readlane, so the serial token chain does not wait
-//           on memory.  The window slides by 256 bytes, loading w[3] two slides
-//           before it is read, or jumps after a long literal run.
-//   output  decoded bytes go to an LDS ring of RING bytes and reach the
-//           stream's scratch slot in dword stores whenever RING/2 bytes are
-//           pending.  Literal runs longer than 64 bytes are copied global ->
-//           global in 16-byte groups per lane (dword loads realigned with
-//           alignbyte) and also written to the ring in order.
-//   matches with offset <= RING-64 are copied ring -> ring, 64 bytes per step,
-//           each lane reading `off * ceil((lane+1)/off)` bytes back (`off`
-//           back when off >= 64), so a step never reads what it writes.
-//           Farther matches read the flushed stream back from global memory,
-//           after a workgroup fence if it was stored since the last fence.
-//   fast path  the headers of the next 64 input positions are decoded one
-//           per lane; the walk over them reads each sequence's fields with
-//           readlane and copies its literals and match with all 64 lanes.
-// Ring steps store all 64 lanes: bytes past the sequence land on positions
-// that are written again before anything reads them, and the slots they take
-// belong to positions more than RING-64 bytes back, which no later match
-// reads and which were flushed (at most RING/2 + 400 bytes are ever pending).
-// With a 4 KiB ring the kernel fits 54 VGPRs: 8 wavefronts per SIMD, 32 per CU.
-template <int RING>
+__device__ __forceinline__ uint32_t lds_u32(const uint8_t *p) {  // any alignment
+  typedef uint32_t u32_any __attribute__((aligned(1)));
+  return *reinterpret_cast<const u32_any *>(p);
+}
+
+__device__ __forceinline__ int32_t bperm(int32_t l, int32_t v) {  // v of lane l & 63
+  return __builtin_amdgcn_ds_bpermute(l << 2, v);
+}
+
+// bits of m below this lane, added to v
+__device__ __forceinline__ int32_t bits_below(uint64_t m, int32_t v) {
+  return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)v));
+}
+
+// Inclusive prefix sum over the 64 lanes (DPP row shifts, then row broadcasts).
+__device__ __forceinline__ int32_t wave_inclusive_sum(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
+// Workgroup barrier that orders LDS only: global loads and stores in flight
+// stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Sizes of a stream decoder of NW wavefronts (NW > 1: one window of 64 input
+// positions per wavefront and round).
+template <int NW>
+struct Lz4Geom {
+  static constexpr int kThreads = 64 * NW;
+  static constexpr int kRing = 4096 * NW;         // output history, bytes
+  static constexpr int kOut = 256 * NW;           // most output bytes of a round
+  static constexpr int kStep = kOut;              // output bytes of a step of the general path
+  static constexpr int kStageWords = 16 * NW + 24;  // input of a round: 64 NW positions and what the last ones reach
+  static constexpr int kStage = 4 * kStageWords;
+  static constexpr int kSeqs = 22 * NW;           // a sequence takes at least 3 input bytes
+  // LDS: ring, two stages, sequence table, first-output-byte bits, source
+  // records of an output step, window exits, window totals, the cut
+  static constexpr int kTabAt = kRing + 2 * kStage;
+  static constexpr int kBitsAt = kTabAt + 8 * kSeqs;
+  static constexpr int kRecAt = kBitsAt + kOut / 8;
+  static constexpr int kExitAt = kRecAt + 4 * kThreads;
+  static constexpr int kTotAt = kExitAt + kThreads;
+  static constexpr int kCutAt = kTotAt + ((4 * NW + 7) & ~7);
+  static constexpr int kLds = kCutAt + 8;
+  static_assert(kOut >= 59 + 273, "a round holds any one sequence");
+};
+
+// One wavefront: three windows of 63 positions a round, at most 64 sequences.
+template <>
+struct Lz4Geom<1> {
+  static constexpr int kThreads = 64;
+  static constexpr int kRing = 4096;
+  static constexpr int kOut = 1024;
+  static constexpr int kStep = 512;
+  static constexpr int kStage = 1024;  // a ring, its first bytes repeated after its end
+  static constexpr int kSeqs = 64;
+  static constexpr int kTabAt = kRing + kStage + 16;
+  static constexpr int kBitsAt = kTabAt + 8 * kSeqs;
+  static constexpr int kListAt = kBitsAt + kOut / 8;
+  static constexpr int kLds = kListAt + 2 * kSeqs;
+};
+
+// One LZ4 stream by one workgroup of NW wavefronts.  The state (input and
+// output position, what is flushed) is uniform over the workgroup: every
+// wavefront derives it from the same LDS words.
+//
+// Rounds.  A round takes the 64 NW input positions from `base`, whatever the
+// sequences in them, so its input is staged in LDS one round ahead.
+//   headers  thread t decodes the sequence that would start at position base
+//            + t.  Sequences of at most 63 input bytes, 59 literals and 273
+//            match bytes inside the stream are decoded by rounds (`ok`).
+//   reach    each wavefront follows the sequences of its 64-position window
+//            from all 64 starts at once, by pointer doubling (at most 21
+//            hops): the set of starts passed, and where the chain leaves the
+//            window or stops at a sequence that is not ok.  None of this needs
+//            to know where the window is entered.
+//   chain    the windows' exits are then followed from the round's entry, one
+//            lookup per window, and each wavefront picks its set of starts.
+//   scan     prefix sums of the sequences' output lengths, over the lanes and
+//            over the windows, give every sequence's first output byte; the
+//            round is cut before the first one that does not fit.
+//   table    the starts store their fields in LDS in sequence order and set
+//            the bit of their first output byte.
+//   output   one byte a thread, two at a time, whatever sequences they belong
+//            to: a thread finds its sequence by counting the bits up to its
+//            byte and takes a literal from the stage or a match byte from the
+//            ring (from the flushed output when the offset passes it).  A
+//            match that overlaps itself reads from the bytes before it.  A
+//            source written in the same step is a lower byte: the threads
+//            leave their byte, or the number of their source byte, in LDS and
+//            follow the numbers until they find a byte.
+// What bounds it is the chain from round to round (about 6000 cycles for 4
+// windows: header reads, 5 hops of pointer doubling, the exits, the scans, the
+// table, the sources), so its time falls with the windows a round takes: a
+// 250 KB bitshuffled float32 stream takes 537 us with one wavefront, 289 with
+// 4, 235 with 8; one sequence after the other, with 64 lanes copying each,
+// took 783.  Of a launch of 6400 such streams, 0.35 ms are their literal runs
+// crossing HBM at 4.8 TB/s.
+//
+// What a round cannot hold (long literal runs, matches of more than 273
+// bytes, the stream's end) is decoded one sequence at a time by the general
+// path, with all threads copying.
+//
+// Output bytes go to an LDS ring and reach the stream's scratch slot in
+// 16-byte stores whenever a quarter of the ring is pending.  An offset of more
+// than kNear reads the slot back from global memory: such a source is at least
+// 15/16 of the ring back, at most 5/16 of the ring is pending or was flushed
+// last, and the stores of the flush before that were waited for by every
+// wavefront before a barrier that precedes the read.
+template <int NW>
 __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__restrict__ scratch, int *status,
-                                           uint8_t *ring) {
-  constexpr int32_t RM = RING - 1;
-  constexpr int32_t NEAR = RING - 64;
-  constexpr int32_t FLUSH_AT = RING / 2;
-  constexpr int kRunUnroll = 4;  // 16-byte groups in flight per lane in a long literal run
-  const int lane = threadIdx.x;
+                                           uint8_t *lds) {
+  using G = Lz4Geom<NW>;
+  constexpr int32_t NT = G::kThreads;
+  constexpr int32_t RING = G::kRing, RM = RING - 1;
+  constexpr int32_t NEAR = RING - G::kStep;
+  constexpr int32_t FLUSH_AT = RING / 4;
+  uint8_t *ring = lds;
+  uint8_t *stage = lds + RING;
+  uint64_t *tab = reinterpret_cast<uint64_t *>(lds + G::kTabAt);
+  uint32_t *obits = reinterpret_cast<uint32_t *>(lds + G::kBitsAt);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint64_t abase = job.src & ~3ull;  // input positions are relative to this aligned address
   const IAMX_GLOBAL uint32_t *__restrict__ sw = iamx::gptr<const uint32_t>(abase);
   const IAMX_GLOBAL uint8_t *__restrict__ sb = iamx::gptr<const uint8_t>(abase);
   IAMX_GLOBAL uint8_t *dst = iamx::gptr<uint8_t>((uint64_t)(scratch + job.dst_off));
   IAMX_GLOBAL uint32_t *dstw = iamx::gptr<uint32_t>((uint64_t)(scratch + job.dst_off));
-  const uint32_t *ring32 = reinterpret_cast<const uint32_t *>(ring);
-  uint32_t *ring32w = reinterpret_cast<uint32_t *>(ring);
+  const bool wide = ((uint64_t)(scratch + job.dst_off) & 15) == 0;  // 16-byte stores of the slot
   const int32_t iend = (int32_t)(job.src & 3) + job.csize;
   const int32_t oend = job.nbytes;
   const int32_t lastw = (iend - 1) >> 2;  // last word holding stream bytes
 
-  // window words past the stream repeat its last word (never parsed)
-  auto ld_word = [&](int32_t pos) -> uint32_t { return sw[min(pos >> 2, lastw)]; };
-  int32_t wb = 0;
-  uint32_t w0 = ld_word(4 * lane), w1 = ld_word(256 + 4 * lane), w2 = ld_word(512 + 4 * lane),
-           w3 = ld_word(768 + 4 * lane);
-  auto jump = [&](int32_t pos) {
-    wb = pos & ~3;
-    w0 = ld_word(wb + 4 * lane);
-    w1 = ld_word(wb + 256 + 4 * lane);
-    w2 = ld_word(wb + 512 + 4 * lane);
-    w3 = ld_word(wb + 768 + 4 * lane);
+  // word i of the input from pos; words past the stream repeat its last word
+  // (never parsed)
+  auto ld_word = [&](int32_t pos, int32_t i) -> uint32_t { return sw[min((pos >> 2) + i, lastw)]; };
+  int32_t ip = (int32_t)(job.src & 3), op = 0, flushed = 0, flush_at = FLUSH_AT;
+  // this wavefront's memory operations so far are complete
+  auto drain = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
   };
-  // make `pos - wb < 256`; positions only move forward
-  auto refill = [&](int32_t pos) {
-    const int32_t q = pos - wb;
-    if (q >= 256) {
-      if (q < 512) {
-        w0 = w1;
-        w1 = w2;
-        w2 = w3;
-        wb += 256;
-        w3 = ld_word(wb + 768 + 4 * lane);
-      } else {
-        jump(pos);
-      }
-    }
-  };
-  // byte at input position pos, wb <= pos < wb + 512 (uniform)
-  auto rbyte = [&](int32_t pos) -> uint32_t {
-    const int32_t q = pos - wb;
-    const uint32_t w = q < 256 ? rdlane(w0, q >> 2) : rdlane(w1, (q >> 2) - 64);
-    return (w >> ((q & 3) << 3)) & 0xffu;
-  };
-  int32_t ip = (int32_t)(job.src & 3), op = 0, flushed = 0, fenced = 0, flush_at = FLUSH_AT;
-  // store the whole dwords of ring bytes [flushed, cur) to the slot; a dword
-  // is stored again only with the same bytes below `flushed`
+  // store the whole 16-byte groups (as dwords where the slot is not 16-byte
+  // aligned) of ring bytes [flushed, cur) to the slot; flushed stays a
+  // multiple of 16
   auto flush = [&](int32_t cur) {
-    for (int32_t p = flushed + 4 * lane; p + 4 <= cur; p += 256) dstw[p >> 2] = ring32[(p & RM) >> 2];
-    flushed = __builtin_amdgcn_readfirstlane(cur & ~3);  // uniform; keeps it in an SGPR
-    flush_at = flushed + FLUSH_AT;
-  };
-
-  // Adds the length continuation bytes from ip on (255s, then one below 255)
-  // to v, 64 input bytes a step (a ballot finds the last one); false when the
-  // stream ends first or the length exceeds the block.
-  auto read_len = [&](int32_t &v) -> bool {
-    for (;;) {
-      refill(ip);
-      const int32_t q = ip - wb + lane;  // < 320
-      const int32_t d = (q >> 2) & 63;
-      const uint32_t a0 = (uint32_t)__shfl((int)w0, d, 64), a1 = (uint32_t)__shfl((int)w1, d, 64);
-      const uint32_t b = ((q < 256 ? a0 : a1) >> ((q & 3) << 3)) & 255u;
-      const uint64_t stop = __ballot(ip + lane < iend && b != 255u);
-      if (stop) {
-        const int32_t t = (int32_t)__builtin_ctzll(stop);
-        v += 255 * t + (int32_t)rdlane(b, t);
-        ip += t + 1;
-        return true;
-      }
-      if (iend - ip < 64) return false;
-      v += 255 * 64;
-      ip += 64;
-      if (v > oend) return false;
+    if (NW > 1) drain();  // the stores of the flush before this one
+    if (wide) {
+      for (int32_t p = flushed + 16 * tid; p + 16 <= cur; p += 16 * NT)
+        *iamx::gptr<u32x4>((uint64_t)(dst + p)) = *reinterpret_cast<const u32x4 *>(ring + (p & RM));
+    } else {
+      for (int32_t p = flushed + 4 * tid; p + 4 <= (cur & ~15); p += 4 * NT)
+        dstw[p >> 2] = *reinterpret_cast<const uint32_t *>(ring + (p & RM));
     }
+    flushed = __builtin_amdgcn_readfirstlane(cur & ~15);
+    flush_at = flushed + FLUSH_AT;
   };
 
   int bad = 0;
   for (;;) {
-    refill(ip);
-    // Fast section (refill() above keeps ip - wb < 256).  Lane l decodes the
-    // header of the sequence that would start at window position qs + l (the
-    // window bytes are gathered with ds_bpermute): literal count, offset,
-    // match length, and a control word: the header length plus literals
-    // (`adv`) when the sequence can be decoded here, bit 31 when the walk
-    // stops before it, bit 30 when the general path below must decode it.
-    // Decoded here: up to 59 literals (read from w0/w1) and a match of
-    // 4..273 bytes (at most one length byte each), an offset within the
-    // output so far, the sequence inside the stream and at most 63 bytes
-    // long, and the next header still among the 64 positions.  The walk
-    // then costs one readlane per field, and it stops once the output
-    // position passes `olim`: 333 bytes (the most one sequence here writes)
-    // short of the slot end, and below the next flush.
-    {
-      const int32_t olim = min(oend - 333, flush_at - 1);
-      while (op <= olim) {
-        const int32_t qs = ip - wb;
-        const int32_t r = qs + lane;  // <= 318
-        auto gather = [&](int32_t d) -> uint32_t {  // window dword d < 128
-          const uint32_t a0 = (uint32_t)__shfl((int)w0, d & 63, 64);
-          const uint32_t a1 = (uint32_t)__shfl((int)w1, d & 63, 64);
-          return d < 64 ? a0 : a1;
-        };
-        const uint32_t h = __builtin_amdgcn_alignbyte(gather((r >> 2) + 1), gather(r >> 2), (uint32_t)(r & 3));
+    // ---- rounds
+    bool general = false;
+    if constexpr (NW == 1) {
+      constexpr int32_t SM = G::kStage - 1, WIN = 63, NEAR1 = RING - 64;
+      uint16_t *list = reinterpret_cast<uint16_t *>(lds + G::kListAt);
+      uint32_t *stage32 = reinterpret_cast<uint32_t *>(stage);
+      // 256 input bytes from pos, a multiple of 256, into the stage
+      auto put_stage = [&](int32_t pos, uint32_t w) {
+        const int32_t at = (pos & SM) >> 2;
+        stage32[at + lane] = w;
+        if (at == 0 && lane < 4) stage32[G::kStage / 4 + lane] = w;
+        __builtin_amdgcn_wave_barrier();
+      };
+      int32_t have = (ip & ~255) + 768;  // the stage holds the input from ip up to here
+      {
+        const uint32_t a = ld_word(have - 768, lane), b = ld_word(have - 512, lane), c = ld_word(have - 256, lane);
+        put_stage(have - 768, a);
+        put_stage(have - 512, b);
+        put_stage(have - 256, c);
+      }
+      for (;;) {
+        // a round reads at most 384 bytes from ip (three windows entered 125
+        // apart, and what the last one's sequences reach); one window's worth
+        // less than it loads ahead is usual
+        while (have < ip + 384) {
+          put_stage(have, ld_word(have, lane));
+          have += 256;
+        }
+        const bool more = have - ip < 768;
+        uint32_t ahead = 0;
+        if (more) ahead = ld_word(have, lane);
+        if (lane < G::kOut / 32) obits[lane] = 0;
+        // walk: the starts of up to three windows, listed by position
+        int32_t n = 0, at = ip;  // sequences so far, the next one's position
+        bool stopped = false;
+#pragma unroll 1
+        for (int w = 0; w < 3; w++) {
+          const uint32_t h = lds_u32(stage + ((at + lane) & SM));
+          const uint32_t hl = (h >> 4) & 15u, lb = (h >> 8) & 255u;
+          const int32_t adv = 3 + (int32_t)hl + (hl == 15 ? (int32_t)lb + 1 : 0) + ((h & 15u) == 15 ? 1 : 0);
+          const bool ok = ((adv <= 63) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
+          const int32_t to = ok ? min(lane + adv, WIN) : lane;
+          const int32_t to2 = bperm(to, to);
+          uint64_t starts = 0;
+          int32_t l = 0, t1;
+          do {
+            t1 = (int32_t)rdlane((uint32_t)to, l);
+            starts |= (1ull << l) | (1ull << t1);
+            l = (int32_t)rdlane((uint32_t)to2, l);
+          } while (l != t1);
+          stopped = l < WIN;
+          starts &= __ballot(ok);
+          if (starts == 0) break;
+          const int32_t k = bits_below(starts, n);
+          if (((starts >> lane) & 1ull) && k < G::kSeqs) list[k] = (uint16_t)(at - ip + lane);
+          n += __builtin_popcountll(starts);
+          const int32_t last = 63 - __builtin_clzll(starts);
+          at += last + (int32_t)rdlane((uint32_t)adv, last);
+          if (stopped || n >= G::kSeqs) break;
+        }
+        if (n == 0) {
+          general = true;
+          break;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // lane k takes sequence k
+        const int32_t pos = ip + (int32_t)list[lane];
+        const uint32_t h = lds_u32(stage + (pos & SM));
         const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
         const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
-        const uint32_t hlit = hl + (lext ? lb : 0u);
-        const uint32_t hlsrc = 1 + lext;  // literals start this far after the token
-        // offset field: <= 318 + 2 + 58 when the sequence is decoded here, and
-        // only read through lane indexes taken mod 64 otherwise
-        const int32_t r2 = r + (int32_t)(hlsrc + hlit);
-        const uint32_t h2 = __builtin_amdgcn_alignbyte(gather((r2 >> 2) + 1), gather(r2 >> 2), (uint32_t)(r2 & 3));
-        const uint32_t hoff = h2 & 0xffffu, he = (h2 >> 16) & 255u;
-        const uint32_t ext = hm == 15 ? 1u : 0u;
-        const uint32_t hml = hm + 4 + (ext ? he : 0u);
-        const int32_t adv = 3 + (int32_t)(lext + hlit + ext);
-        // (bitwise: one vector compare chain, no branches)
-        const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) & ((int32_t)hoff <= op) &
-                         (adv <= 63) & (adv <= iend - wb - r)) != 0;
-        const uint32_t ctl = ok ? (lane + adv <= 63 ? (uint32_t)adv : 0x80000000u) : 0xC0000000u;
-        // 1/off rounded up by 16 ulps: floor((lane + off) * rcp) is exact for
-        // lane < 64, off < 64
-        const uint32_t hrcp = __float_as_uint(__builtin_amdgcn_rcpf((float)hoff)) + 16u;
-        int32_t l = 0;
-        uint32_t c = rdlane(ctl, 0);
-        while ((int32_t)(c | (uint32_t)(olim - op)) >= 0) {
-          const int32_t lit = (int32_t)rdlane(hlit, l);
-          const int32_t off = (int32_t)rdlane(hoff, l);
-          const int32_t ml = (int32_t)rdlane(hml, l);
-          const int32_t o2 = op + lit;
-          if (lit) {
-            const int32_t q = r + l + (int32_t)rdlane(hlsrc, l);  // window position of literal byte `lane`, <= 383
-            const int32_t d = (q >> 2) & 63;
-            const uint32_t a0 = (uint32_t)__shfl((int)w0, d, 64), a1 = (uint32_t)__shfl((int)w1, d, 64);
-            ring[(op + lane) & RM] = (uint8_t)((q < 256 ? a0 : a1) >> ((q & 3) << 3));
-            __builtin_amdgcn_wave_barrier();
+        const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
+        const int32_t src = pos + 1 + (int32_t)lext;  // first literal
+        const uint32_t h2 = lds_u32(stage + ((src + lit) & SM));
+        const int32_t hoff = (int32_t)(h2 & 0xffffu);
+        const uint32_t he = (h2 >> 16) & 255u;
+        const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
+        const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
+        const bool mine = lane < n;
+        const int32_t oinc = wave_inclusive_sum(mine ? len : 0);
+        const int32_t os = oinc - len;  // this sequence's first output byte, from op
+        // the first sequence that does not fit, or ends in a second length byte
+        const bool hard = (((ext != 0) & (he == 255)) | (hoff < 1) | (hoff > op + os + lit) | (oinc > oend - op)) != 0;
+        const uint64_t cutm = __ballot(mine & (hard | (oinc > G::kOut)));
+        const uint64_t hardm = __ballot(hard);
+        int32_t nseq = min(n, G::kSeqs);
+        if (cutm) {
+          nseq = __builtin_ctzll(cutm);
+          stopped = ((hardm >> nseq) & 1ull) != 0;
+          at = (int32_t)rdlane((uint32_t)pos, nseq);
+          if (nseq == 0) {
+            general = true;
+            break;
           }
-          // the first 64-byte step is peeled: most matches are one step
-          if (off > NEAR) {
-            // every source byte lies more than RING - 64 bytes back, and at
-            // most RING/2 + 395 bytes are pending, so all of them were flushed
-            const int32_t gend = o2 + ((ml + 63) & ~63) - off;
-            if (gend > fenced) {
-              __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-              fenced = flushed;
-            }
-            const int32_t d0 = o2 + lane;
-            ring[d0 & RM] = dst[d0 - off];
-            __builtin_amdgcn_wave_barrier();
-            for (int32_t k = 64; k < ml; k += 64) {
-              ring[(d0 + k) & RM] = dst[d0 + k - off];
-              __builtin_amdgcn_wave_barrier();
-            }
-          }
-          if (off <= NEAR) {
-            int32_t back = off;  // off * ceil((lane + 1) / off)
-            if (off < 64) {
-              const float rc = __uint_as_float(rdlane(hrcp, l));
-              back = (int32_t)__umul24((uint32_t)((float)(lane + off) * rc), (uint32_t)off);
-            }
-            const int32_t d0 = o2 + lane, s0 = d0 - back;
-            const uint8_t v = ring[s0 & RM];
-            __builtin_amdgcn_wave_barrier();
-            ring[d0 & RM] = v;
-            __builtin_amdgcn_wave_barrier();
-            for (int32_t k = 64; k < ml; k += 64) {
-              const uint8_t v2 = ring[(s0 + k) & RM];
-              __builtin_amdgcn_wave_barrier();
-              ring[(d0 + k) & RM] = v2;
-              __builtin_amdgcn_wave_barrier();
-            }
-          }
-          op = o2 + ml;
-          l += (int32_t)c;
-          c = rdlane(ctl, l);
+        } else if (n > G::kSeqs) {
+          stopped = false;
+          at = (int32_t)rdlane((uint32_t)(src + lit), 63) + 2 + (int32_t)rdlane(ext, 63);
         }
-        ip = wb + qs + l;
-        if (op > olim || (c & 0x40000000u)) break;  // a flush, or a sequence for the general path
-        refill(ip);  // the walk left the 64 positions: the next ones
+        const int32_t total = (int32_t)rdlane((uint32_t)oinc, nseq - 1);
+        if (lane < nseq) {
+          // byte x of the output is a literal below `os + lit`
+          tab[lane] = (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
+          atomicOr(obits + (os >> 5), 1u << (os & 31));
+        }
+        __builtin_amdgcn_wave_barrier();
+        const uint64_t ob = lane < G::kOut / 64 ? reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)] : 0ull;
+        int32_t before = -1;  // sequences that start in earlier steps, less one
+        auto entry_of = [&](int32_t x0) -> uint64_t {
+          const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), x0 >> 6) << 32) | rdlane((uint32_t)ob, x0 >> 6);
+          const int32_t k = bits_below(m >> 1, before + (int32_t)(m & 1));  // the last start at or before its byte
+          before += __builtin_popcountll(m);
+          return tab[k];
+        };
+        uint64_t e = entry_of(0);
+        for (int32_t x0 = 0;;) {
+          const int32_t x = x0 + lane;
+          const uint32_t elo = (uint32_t)e;
+          const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
+          int32_t off = (int32_t)(elo >> 16);
+          const int32_t lat = RING + ((x + (int32_t)(uint32_t)(e >> 32)) & SM);
+          int32_t sp = op + x - off;
+          // a source past the ring, inside the match itself or inside this step
+          const bool odd = (im >= 0) & (x < total) & ((off > NEAR1) | (off <= max(im, lane)));
+          const int32_t x1 = x0 + 64;
+          uint32_t v;
+          if (__ballot(odd)) {
+            if (__ballot(odd & (im >= off))) {
+              // (im + 1/2) / off is at least 1/546 away from a whole number
+              const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
+              if (im >= off) off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
+              sp = op + x - off;
+            }
+            v = lds[im < 0 ? lat : sp & RM];
+            if (x1 < total) e = entry_of(x1);
+            const bool far = odd & (off > NEAR1);
+            // at most FLUSH_AT + 64 bytes are pending, so a far source was
+            // flushed, by this wavefront's own stores
+            if (far) v = dst[sp];
+            const bool dep = odd & (off <= lane);
+            if (__ballot(dep)) {
+              // bit 6: the lane has its own byte
+              int32_t code = dep ? lane - off : lane | 64;
+              do {
+                code = bperm(code, code);
+              } while (__ballot(code < 64));
+              v = (uint32_t)bperm(code, (int32_t)v);
+            }
+            asm volatile("" : "+v"(v));  // a far byte has arrived
+          } else {
+            v = lds[im < 0 ? lat : sp & RM];
+            if (x1 < total) e = entry_of(x1);
+          }
+          __builtin_amdgcn_wave_barrier();
+          ring[(op + x) & RM] = (uint8_t)v;
+          __builtin_amdgcn_wave_barrier();
+          const int32_t cur = op + min(total, x1);
+          if (cur >= flush_at) flush(cur);
+          if (x1 >= total) break;
+          x0 = x1;
+        }
+        op += total;
+        ip = at;
+        if (stopped) {
+          general = true;
+          break;
+        }
+        if (more) {
+          put_stage(have, ahead);
+          have += 256;
+        }
+      }
+    } else {
+      volatile uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
+      uint8_t *exits = lds + G::kExitAt;
+      uint32_t *tot = reinterpret_cast<uint32_t *>(lds + G::kTotAt);
+      unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
+      int32_t base = ip, entry = 0, buf = 0;
+      if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage)[tid] = ld_word(base, tid);
+      lds_barrier();
+      for (;;) {
+        const int32_t nbase = base + 64 * NW;
+        uint32_t ahead = 0;  // the next round's input, on its way until the end of this one
+        if (tid < G::kStageWords) ahead = ld_word(nbase, tid);
+        if (tid < G::kOut / 32) obits[tid] = 0;
+        if (tid == 0) *cut = ~0ull;
+        // headers
+        const uint8_t *st = stage + buf * G::kStage + (base & 3);
+        const uint32_t h = lds_u32(st + tid);
+        const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
+        const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
+        const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
+        const int32_t src = tid + 1 + (int32_t)lext;  // first literal, from base
+        const uint32_t h2 = lds_u32(st + min(src + lit, G::kStage - 8));
+        const int32_t hoff = (int32_t)(h2 & 0xffffu);
+        const uint32_t he = (h2 >> 16) & 255u;
+        const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
+        const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
+        const int32_t adv = 3 + lit + (int32_t)(lext + ext);
+        // (bitwise: one vector compare chain, no branches)
+        const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) & (adv <= 63) &
+                         (adv <= iend - base - tid)) != 0;
+        const uint64_t okm = __ballot(ok);
+        // reach: 64 and more is a position of the next window; a start that is
+        // not ok leads to itself
+        int32_t to = ok ? lane + adv : lane;
+        uint32_t rlo = lane < 32 ? 1u << lane : 0u, rhi = lane < 32 ? 0u : 1u << (lane - 32);
+#pragma unroll
+        for (int t = 0; t < 5; t++) {
+          const int32_t f = bperm(to, to);
+          const uint32_t flo = (uint32_t)bperm(to, (int32_t)rlo), fhi = (uint32_t)bperm(to, (int32_t)rhi);
+          const bool in = to < 64;
+          rlo |= in ? flo : 0u;
+          rhi |= in ? fhi : 0u;
+          to = in ? f : to;
+        }
+        exits[tid] = (uint8_t)to;
+        lds_barrier();
+        // chain
+        uint32_t ex[(NW + 3) / 4];
+#pragma unroll
+        for (int v = 0; v < (NW + 3) / 4; v++) ex[v] = reinterpret_cast<const uint32_t *>(exits)[(64 * v + lane) & (16 * NW - 1)];
+        int32_t e = entry, mine_at = 64, stop = -1;
+#pragma unroll
+        for (int v = 0; v < NW; v++) {
+          if (stop < 0) {
+            if (v == wave) mine_at = e;
+            const int32_t x = (int32_t)((rdlane(ex[v / 4], 16 * (v & 3) + (e >> 2)) >> (8 * (e & 3))) & 255u);
+            if (x < 64) stop = 64 * v + x;
+            e = x - 64;
+          }
+        }
+        if (stop == entry) {  // the first sequence is not one for a round
+          ip = base + entry;
+          general = true;
+          break;
+        }
+        const uint64_t starts =
+            mine_at < 64 ? (((uint64_t)rdlane(rhi, mine_at) << 32) | rdlane(rlo, mine_at)) & okm : 0ull;
+        // scan
+        const bool mine = ((starts >> lane) & 1ull) != 0;
+        int32_t oinc = wave_inclusive_sum(mine ? len : 0);
+        if (lane == 0) tot[wave] = rdlane((uint32_t)oinc, 63) | ((uint32_t)__builtin_popcountll(starts) << 20);
+        lds_barrier();
+        const int32_t tsum = wave_inclusive_sum(lane < NW ? (int32_t)tot[lane & (NW - 1)] : 0);
+        const uint32_t prev = wave ? rdlane((uint32_t)tsum, wave - 1) : 0u;  // of the windows before
+        int32_t total = (int32_t)(rdlane((uint32_t)tsum, NW - 1) & 0xfffffu);
+        oinc += (int32_t)(prev & 0xfffffu);
+        const int32_t os = oinc - len;  // this sequence's first output byte, from op
+        if (mine) {
+          const bool hard = (oinc > oend - op) | (hoff > op + os + lit);
+          if (hard | (oinc > G::kOut)) {
+            atomicMin(cut, ((unsigned long long)tid << 32) | ((uint32_t)os << 1) | (hard ? 1u : 0u));
+          } else {
+            // table: byte x of the output is a literal below `os + lit`
+            tab[bits_below(starts, (int32_t)(prev >> 20))] =
+                (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
+            atomicOr(obits + (os >> 5), 1u << (os & 31));
+          }
+        }
+        lds_barrier();
+        const uint64_t c = *cut;
+        const uint32_t clo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)c),
+                       chi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(c >> 32));
+        const bool is_cut = chi != ~0u;
+        if (is_cut) {
+          total = (int32_t)(clo >> 1);
+          stop = (int32_t)chi;
+          general = (clo & 1u) != 0;
+          if (total == 0) {  // the first sequence itself (never for its length alone)
+            ip = base + stop;
+            general = true;
+            break;
+          }
+        } else {
+          general = stop >= 0;
+        }
+        // output: lane q of a wavefront holds the bits of bytes 64 q .. 64 q + 63
+        // and the number of sequences that start before them
+        const uint64_t ob = lane < G::kOut / 64 ? reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)] : 0ull;
+        const int32_t own = __builtin_popcountll(ob);
+        const int32_t before = wave_inclusive_sum(own) - own;
+        for (int32_t x0 = 0; x0 < total; x0 += 2 * NT) {
+          uint32_t v[2] = {0, 0};
+          int32_t from[2];
+          bool dep[2] = {false, false};
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int32_t xw = x0 + NT * u + 64 * wave;
+            if (xw < total) {
+              const int32_t x = xw + lane;
+              const int32_t q = xw >> 6;
+              const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), q) << 32) | rdlane((uint32_t)ob, q);
+              // the last sequence that starts at or before this byte
+              const uint64_t en =
+                  tab[bits_below(m >> 1, (int32_t)rdlane((uint32_t)before, q) - 1 + (int32_t)(m & 1))];
+              const uint32_t elo = (uint32_t)en;
+              const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
+              int32_t off = (int32_t)(elo >> 16);
+              const bool live = (im >= 0) & (x < total);
+              const bool far = live & (off > NEAR);
+              if (__ballot(live & (im >= off))) {
+                // (im + 1/2) / off is at least 1/546 away from a whole number
+                const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
+                if (im >= off) off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
+              }
+              const int32_t sp = x - off;  // source byte of a match, from op
+              const int32_t lat = (int32_t)(st - lds) + x + (int32_t)(uint32_t)(en >> 32);
+              v[u] = lds[im < 0 ? lat : (op + sp) & RM];
+              if (__ballot(far)) {
+                if (far) v[u] = dst[op + sp];
+              }
+              dep[u] = live & (sp >= x0);
+              from[u] = sp - x0;
+              rec[NT * u + tid] = (uint16_t)(dep[u] ? (uint32_t)from[u] : 0x8000u | v[u]);
+            }
+          }
+          lds_barrier();
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            while (__ballot(dep[u])) {
+              if (dep[u]) {
+                const uint32_t r = rec[from[u]];
+                rec[NT * u + tid] = (uint16_t)r;
+                from[u] = (int32_t)r;
+                v[u] = r & 255u;
+                dep[u] = r < 0x8000u;
+              }
+            }
+            const int32_t x = x0 + NT * u + tid;
+            if (x < total) ring[(op + x) & RM] = (uint8_t)v[u];
+          }
+          if (x0 + 2 * NT >= total && tid < G::kStageWords)
+            reinterpret_cast<uint32_t *>(stage + (buf ^ 1) * G::kStage)[tid] = ahead;
+          lds_barrier();
+        }
+        op += total;
+        if (op >= flush_at) flush(op);
+        if (stop >= 0) {
+          ip = base + stop;
+          break;
+        }
+        base = nbase;
+        entry = e;
+        buf ^= 1;
       }
     }
-    if (op >= flush_at) {
+    if (!general) continue;  // cut where the round's output was full
+    // ---- general path: one sequence.  Every wavefront keeps the 256 input
+    // bytes from gb in a register and parses them alike.
+    int32_t gb = 0;
+    uint32_t gw = 0;
+    auto look = [&](int32_t pos) {
+      gb = pos & ~3;
+      gw = ld_word(gb, lane);
+    };
+    auto rbyte = [&](int32_t pos) -> uint32_t {  // gb <= pos < gb + 256
+      const int32_t q = pos - gb;
+      return (rdlane(gw, q >> 2) >> ((q & 3) << 3)) & 0xffu;
+    };
+    // Adds the length continuation bytes from ip on (255s, then one below 255)
+    // to v, 64 input bytes a step (a ballot finds the last one); false when the
+    // stream ends first or the length exceeds the block.
+    auto read_len = [&](int32_t &v) -> bool {
+      for (;;) {
+        if (ip + 64 > gb + 256) look(ip);
+        const int32_t q = ip - gb + lane;
+        const uint32_t b = ((uint32_t)bperm(q >> 2, (int32_t)gw) >> ((q & 3) << 3)) & 255u;
+        const uint64_t stop = __ballot(ip + lane < iend && b != 255u);
+        if (stop) {
+          const int32_t t = (int32_t)__builtin_ctzll(stop);
+          v += 255 * t + (int32_t)rdlane(b, t);
+          ip += t + 1;
+          return true;
+        }
+        if (iend - ip < 64) return false;
+        v += 255 * 64;
+        ip += 64;
+        if (v > oend) return false;
+      }
+    };
+    // Writes n output bytes at op without the ring in between: what is pending
+    // goes out first, then whole 16-byte groups are stored to the slot, the
+    // next groups' bytes asked for before the last ones are stored; the last
+    // RING bytes also go to the ring.  byte_of and group_of give byte i and
+    // bytes i .. i + 15 of the n.
+    auto bulk = [&](int32_t n, auto byte_of, auto group_of) {
       flush(op);
-      continue;  // the fast loop again
-    }
-    refill(ip);
+      if (tid < op - flushed) dst[flushed + tid] = ring[(flushed + tid) & RM];
+      lds_barrier();  // the ring is written below
+      const int32_t keep = op + n - RING;                   // the ring holds positions from here
+      const int32_t head = min((16 - (op & 15)) & 15, n);  // bytes up to the first whole group
+      const int32_t ng = (n - head) >> 4;                   // whole groups after the head
+      const int32_t bend = head + (ng << 4);
+      uint8_t hb = 0, tb = 0;
+      if (tid < head) hb = byte_of(tid);
+      if (tid < n - bend) tb = byte_of(bend + tid);
+      auto group_store = [&](int32_t g, u32x4 w) {
+        const int32_t d = op + head + 16 * g;  // a multiple of 16
+        if (wide) {
+          *iamx::gptr<u32x4>((uint64_t)(dst + d)) = w;
+        } else {
+          dstw[d >> 2] = w.x;
+          dstw[(d >> 2) + 1] = w.y;
+          dstw[(d >> 2) + 2] = w.z;
+          dstw[(d >> 2) + 3] = w.w;
+        }
+        if (d >= keep) {
+          *reinterpret_cast<u32x4 *>(ring + (d & RM)) = w;
+        } else if (d + 16 > keep) {  // the group the ring starts in
+          for (int t = 0; t < 16; t++)
+            if (d + t >= keep) ring[(d + t) & RM] = (uint8_t)(w[t >> 2] >> (8 * (t & 3)));
+        }
+      };
+      u32x4 wa, wb;
+      if (tid < ng) wa = group_of(head + 16 * tid);
+      for (int32_t g = tid; g < ng; g += 2 * NT) {
+        if (g + NT < ng) wb = group_of(head + 16 * (g + NT));
+        group_store(g, wa);
+        if (g + 2 * NT < ng) wa = group_of(head + 16 * (g + 2 * NT));
+        if (g + NT < ng) group_store(g + NT, wb);
+      }
+      auto put_byte = [&](int32_t i, uint8_t v) {
+        dst[op + i] = v;
+        if (op + i >= keep) ring[(op + i) & RM] = v;
+      };
+      if (tid < head) put_byte(tid, hb);
+      if (tid < n - bend) put_byte(bend + tid, tb);
+      op += n;
+      flushed = __builtin_amdgcn_readfirstlane(op & ~15);
+      flush_at = flushed + FLUSH_AT;
+      if (NW > 1) drain();
+      lds_barrier();
+    };
     if (ip >= iend) { bad = 1; break; }
+    look(ip);
     const uint32_t token = rbyte(ip);
     ++ip;
     int32_t lit = (int32_t)(token >> 4);
     if (lit == 15 && !read_len(lit)) { bad = 2; break; }
     if (lit > iend - ip || lit > oend - op) { bad = 3; break; }
+    lds_barrier();  // no wavefront still reads the LDS of the last round
     if (lit > 0) {
-      if (lit <= 64) {
-        // literals from the register window
-        refill(ip);
-        const int32_t q = ip - wb + lane;  // < 320
-        const int sl = (q >> 2) & 63;
-        const uint32_t a0 = (uint32_t)__shfl((int)w0, sl, 64), a1 = (uint32_t)__shfl((int)w1, sl, 64);
-        const uint32_t v = ((q < 256 ? a0 : a1) >> ((q & 3) << 3)) & 0xffu;
-        ring[(op + lane) & RM] = (uint8_t)v;
-        __builtin_amdgcn_wave_barrier();
+      if (lit <= NT) {
+        if (ip - gb + lit <= 256) {
+          const int32_t q = ip - gb + tid;
+          const uint32_t b = (uint32_t)bperm(q >> 2, (int32_t)gw) >> ((q & 3) << 3);
+          if (tid < lit) ring[(op + tid) & RM] = (uint8_t)b;
+        } else if (tid < lit) {
+          ring[(op + tid) & RM] = sb[ip + tid];
+        }
+        lds_barrier();
         ip += lit;
         op += lit;
         if (op >= flush_at) flush(op);
       } else {
-        // long run: what is pending goes out first, then the run is copied
-        // global -> global, 16 bytes a lane, the source realigned to the
-        // destination's dwords with alignbyte; every run byte is also written
-        // to the ring in position order, so the ring ends holding the run's
-        // last RING bytes.  The window for the next header is requested now.
-        flush(op);
-        if (lane < op - flushed) dst[flushed + lane] = ring[(flushed + lane) & RM];
-        const int32_t nip = ip + lit;
-        if (nip - wb >= 256) jump(nip);
-        const int32_t head = min((4 - (op & 3)) & 3, lit);  // bytes up to the first destination dword
-        const int32_t ng = (lit - head) >> 4;                // whole 16-byte groups after the head
-        const int32_t bend = head + (ng << 4);
-        if (lane < head) {
-          const uint8_t v = sb[ip + lane];
-          dst[op + lane] = v;
-          ring[(op + lane) & RM] = v;
-        }
-        const int32_t d0 = op + head;  // multiple of 4
-        const int32_t sw0 = (ip + head) >> 2;
-        const uint32_t sh = (uint32_t)((ip + head) & 3);  // the same for every group
-        // one group: words k..k+3 hold run bytes, word k+4 only when sh > 0
-        auto group_load = [&](int32_t g, uint32_t *w) {
-          const int32_t k = sw0 + 4 * g;
-          w[0] = sw[k];
-          w[1] = sw[k + 1];
-          w[2] = sw[k + 2];
-          w[3] = sw[k + 3];
-          w[4] = sw[min(k + 4, lastw)];
-        };
-        auto group_store = [&](int32_t g, const uint32_t *w) {
-          const int32_t d = d0 + 16 * g;
-          uint32_t o[4];
-#pragma unroll
-          for (int t = 0; t < 4; t++) o[t] = __builtin_amdgcn_alignbyte(w[t + 1], w[t], sh);
-#pragma unroll
-          for (int t = 0; t < 4; t++) dstw[(d >> 2) + t] = o[t];
-#pragma unroll
-          for (int t = 0; t < 4; t++) ring32w[((d + 4 * t) & RM) >> 2] = o[t];
-        };
-        int32_t g0 = 0;
-        for (; g0 + 64 * kRunUnroll <= ng; g0 += 64 * kRunUnroll) {  // every lane has all groups
-          uint32_t w[kRunUnroll][5];
-#pragma unroll
-          for (int u = 0; u < kRunUnroll; u++) group_load(g0 + 64 * u + lane, w[u]);
-#pragma unroll
-          for (int u = 0; u < kRunUnroll; u++) group_store(g0 + 64 * u + lane, w[u]);
-        }
-        for (; g0 < ng; g0 += 64) {
-          if (g0 + lane < ng) {
-            uint32_t w[5];
-            group_load(g0 + lane, w);
-            group_store(g0 + lane, w);
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane < lit - bend) {  // fewer than 16 tail bytes, after the groups (ring order)
-          const uint8_t v = sb[ip + bend + lane];
-          dst[op + bend + lane] = v;
-          ring[(op + bend + lane) & RM] = v;
-        }
-        __builtin_amdgcn_wave_barrier();
-        ip = nip;
-        op += lit;
-        flushed = __builtin_amdgcn_readfirstlane(op & ~3);
-        flush_at = flushed + FLUSH_AT;
+        look(ip + lit);  // for what follows the run
+        const IAMX_GLOBAL uint8_t *from = sb + ip;
+        bulk(
+            lit, [&](int32_t i) -> uint8_t { return from[i]; },
+            [&](int32_t i) -> u32x4 { return *(const IAMX_GLOBAL u32x4_any *)(from + i); });
+        ip += lit;
       }
     }
     if (ip == iend) break;  // last sequence: literals only
-    refill(ip);
     if (iend - ip < 2) { bad = 4; break; }
+    if (ip + 2 > gb + 256) look(ip);
     const int32_t off = (int32_t)(rbyte(ip) | (rbyte(ip + 1) << 8));
     ip += 2;
     int32_t ml = (int32_t)(token & 15u);
     if (ml == 15 && !read_len(ml)) { bad = 5; break; }
     ml += 4;
     if (off == 0 || off > op || ml > oend - op) { bad = 6; break; }
-    // back distance of this lane's source: off * ceil((lane + 1) / off) for off < 64
-    int32_t back = off;
-    if (off < 64) {
-      const int32_t num = lane + off;
-      int32_t qq = (int32_t)((float)num * __builtin_amdgcn_rcpf((float)off));
-      const int32_t r = num - qq * off;
-      qq += (r >= off) - (r < 0);
-      back = off * qq;
+    if (ml >= 512 && off <= 16 && (off & (off - 1)) == 0) {
+      // the match repeats 1, 2, 4, 8 or 16 bytes: every whole 16-byte group of
+      // the output is the same one
+      const int32_t m0 = op - off;  // byte i of the output is byte m0 + (i - op) mod off
+      const uint32_t b = ring[(m0 + ((lane - op) & (off - 1))) & RM];  // of an i that is lane mod 16
+      u32x4 w;
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        w[t] = rdlane(b, 4 * t) | (rdlane(b, 4 * t + 1) << 8) | (rdlane(b, 4 * t + 2) << 16) | (rdlane(b, 4 * t + 3) << 24);
+      const int32_t op0 = op;
+      bulk(
+          ml,
+          [&](int32_t i) -> uint8_t {
+            const int32_t j = (op0 + i) & 15;
+            const uint32_t lo = j & 4 ? w.y : w.x, hi = j & 4 ? w.w : w.z;
+            return (uint8_t)((j & 8 ? hi : lo) >> (8 * (j & 3)));
+          },
+          [&](int32_t) -> u32x4 { return w; });
+      continue;
     }
-    if (off <= NEAR) {
-      auto step = [&](int32_t k) {
-        const uint8_t v = ring[(op + k + lane - back) & RM];
-        __builtin_amdgcn_wave_barrier();
-        ring[(op + k + lane) & RM] = v;
-        __builtin_amdgcn_wave_barrier();
-        const int32_t cur = op + min(ml, k + 64);
-        if (cur >= flush_at) flush(cur);
-      };
-      // The match is periodic with period off, so position p may also copy
-      // from p - backU, the first multiple of off at least 256 back (at most
-      // 511 or off, both within the ring).  Once 256 bytes of that history
-      // exist, four 64-byte steps read nothing the same four steps write and
-      // go out together.
-      constexpr int32_t U = 4;
-      const int32_t backU = off >= 64 * U ? off : off * ((64 * U + off - 1) / off);
-      int32_t k = 0;
-      for (; k < ml && k < backU - off; k += 64) step(k);
-      for (; k + 64 * U <= ml; k += 64 * U) {
+    // kStep bytes a step: byte i of a step is byte (i mod off) of the `off`
+    // bytes before the step
+    {
+      constexpr int U = G::kStep / NT;
+      int32_t at[U];  // source of this thread's bytes, from the step's first byte less off
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int32_t i = NT * u + tid;
+        // i < 4096: (i + 1/2) / off is at least 1/8192 of a turn from a whole number
+        const int32_t turn = off > i ? 0 : (int32_t)(((float)i + 0.5f) / (float)off);
+        at[u] = i - turn * off;
+      }
+      for (int32_t k = 0; k < ml; k += G::kStep) {
         uint8_t v[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = ring[(op + k + 64 * u + lane - backU) & RM];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int u = 0; u < U; u++) ring[(op + k + 64 * u + lane) & RM] = v[u];
-        __builtin_amdgcn_wave_barrier();
-        if (op + k + 64 * U >= flush_at) flush(op + k + 64 * U);
-      }
-      for (; k < ml; k += 64) step(k);
-    } else {
-      for (int32_t k = 0; k < ml; k += 64) {
-        // positions at or after `lo` are still in the ring; older ones were
-        // flushed and are read back from global memory
-        const int32_t lo = op + k + 64 - RING;
-        const int32_t gmax = min(op + k + 64 - back, lo);  // end of the global positions this step reads
-        if (gmax > fenced) {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-          fenced = flushed;
+        for (int u = 0; u < U; u++) {
+          const int32_t s = op + k - off + at[u];
+          v[u] = 0;
+          if (k + NT * u + tid < ml) v[u] = off > NEAR ? dst[s] : ring[s & RM];
         }
-        const int32_t i = k + lane;
-        const int32_t s = op + i - back;
-        uint8_t v = 0;
-        if (i < ml) v = s >= lo ? ring[s & RM] : dst[s];
-        __builtin_amdgcn_wave_barrier();
-        ring[(op + i) & RM] = v;
-        __builtin_amdgcn_wave_barrier();
-        const int32_t cur = op + min(ml, k + 64);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (k + NT * u + tid < ml) ring[(op + k + NT * u + tid) & RM] = v[u];
+        lds_barrier();
+        const int32_t cur = op + min(ml, k + G::kStep);
         if (cur >= flush_at) flush(cur);
       }
+      op += ml;
     }
-    op += ml;
   }
   if (!bad && op != oend) bad = 7;
-  if (!bad) flush((oend + 3) & ~3);  // the slot is padded to 16 bytes
-  if (bad && lane == 0) atomicOr(status, 1 << bad);
+  if (!bad) {  // the slot is padded to 4 bytes at least
+    flush(oend);
+    const int32_t p = flushed + 4 * tid;
+    if (p < oend) dstw[p >> 2] = *reinterpret_cast<const uint32_t *>(ring + (p & RM));
+  }
+  if (bad && tid == 0) atomicOr(status, 1 << bad);
 }
 
 // One BloscLZ stream by one wavefront (the stream format is restated in the
@@ -534,11 +851,13 @@ __device__ __forceinline__ void blosclz_stream(const iamx_lz4_job_t job, uint8_t
   if (bad && lane == 0) atomicOr(status, IAMX_STATUS_BLOSCLZ);
 }
 
-template <int RING>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RING <= 4096 ? 8 : 1, 8))) void k_lz4_streams(
+constexpr int kBloscRing = 4096;
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 1 ? 7 : 8, 8))) void k_lz4_streams(
     const iamx_lz4_job_t *__restrict__ jobs, int njobs, uint8_t *__restrict__ scratch, int64_t cap, int *status,
     int zstd_on) {
-  __shared__ __align__(16) uint8_t ring[RING];
+  __shared__ __align__(16) uint8_t lds[Lz4Geom<NW>::kLds];
   const int j = blockIdx.x;
   if (j >= njobs) return;
   const iamx_lz4_job_t job = jobs[j];
@@ -548,7 +867,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RING <= 4096
     return;
   }
   if (job.codec == IAMX_CODEC_BLOSCLZ) {
-    blosclz_stream<RING>(job, scratch, status, ring);
+    if (threadIdx.x < 64) blosclz_stream<kBloscRing>(job, scratch, status, lds);
     return;
   }
   if (job.codec == IAMX_CODEC_ZSTD) {  // decoded by a pass of its own
@@ -559,7 +878,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RING <= 4096
     if (threadIdx.x == 0) atomicOr(status, IAMX_STATUS_CODEC);
     return;
   }
-  lz4_stream<RING>(job, scratch, status, ring);
+  if (job.csize <= 0) {  // nothing to read: ends before its first token
+    if (threadIdx.x == 0) atomicOr(status, 1 << 1);
+    return;
+  }
+  lz4_stream<NW>(job, scratch, status, lds);
 }
 
 struct Planes {
@@ -579,8 +902,6 @@ template <typename T>
 __device__ __forceinline__ void put_elem(uint8_t *dst, int64_t idx, uint64_t v) {
   reinterpret_cast<T *>(dst)[idx] = (T)v;
 }
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // 4x4 byte transpose: r[g] = bytes g of (a, b, c, d)
 __device__ __forceinline__ void bytes4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t r[4]) {
@@ -894,33 +1215,27 @@ __global__ __launch_bounds__(256) void k_transpose(int64_t rows, int64_t cols, c
 
 namespace iamx {
 
-// History ring of the LZ4 kernel in KiB (4, 8 or 16): a bigger ring serves
-// more matches from LDS, a smaller one fits more wavefronts per CU.
-static int lz4_ring_kib() {
-  static const int kib = [] {
-    const char *e = getenv("IAMX_LZ4_RING_KIB");
-    const int v = e ? atoi(e) : 4;
-    return (v == 8 || v == 16) ? v : 4;
-  }();
-  return kib;
-}
-
+// Wavefronts per stream, by how many streams a CU gets.  A stream's time is set
+// by its own chain of rounds, so few streams are spread over many wavefronts
+// each; many streams hide each other's waits, and one wavefront decodes a
+// sequence with the fewest instructions.  The lines are where the launch still
+// holds every stream at once (2 x 8 and 8 x 4 wavefronts per CU).  Measured in
+// us with 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250 KB:
+// 4 streams 235 / 289 / 537, 512 streams 330 / 395 / 690, 1024 streams
+// 650 / 484 / 775, 2048 streams 1220 / 741 / 857, 4096 streams
+// - / 1318 / 1050, 6400 streams - / 1884 / 1424; exponent planes of float32
+// (64 KB): 1024 streams 805 / 696 / 1156, 6400 streams - / 3019 / 1950.
 int launch_lz4(const char *name, const iamx_lz4_job_t *d_lz4, int n_lz4, void *d_scratch, int64_t cap) {
   const int z = zstd_enabled() ? 1 : 0;
-  switch (lz4_ring_kib()) {
-    case 8:
-      IAMX_LAUNCH(name, k_lz4_streams<8192>, dim3(n_lz4), dim3(64), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
-                  status_word(), z);
-      break;
-    case 16:
-      IAMX_LAUNCH(name, k_lz4_streams<16384>, dim3(n_lz4), dim3(64), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
-                  status_word(), z);
-      break;
-    default:
-      IAMX_LAUNCH(name, k_lz4_streams<4096>, dim3(n_lz4), dim3(64), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
-                  status_word(), z);
-      break;
-  }
+  if (n_lz4 <= 2 * g_num_cus)
+    IAMX_LAUNCH(name, k_lz4_streams<8>, dim3(n_lz4), dim3(512), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
+                status_word(), z);
+  else if (n_lz4 <= 8 * g_num_cus)
+    IAMX_LAUNCH(name, k_lz4_streams<4>, dim3(n_lz4), dim3(256), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
+                status_word(), z);
+  else
+    IAMX_LAUNCH(name, k_lz4_streams<1>, dim3(n_lz4), dim3(64), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
+                status_word(), z);
   if (z) return launch_zstd("zstd_streams", d_lz4, n_lz4, d_scratch, cap);
   return IAMX_OK;
 }

@@ -336,6 +336,56 @@ def test_crafted_lz4_streams(ctx, orc, plan, n):
     assert got == want
 
 
+# Lengths on both sides of what a decoding round holds (59 literals, a match of
+# 273 bytes, 63 input bytes a sequence), matches that fill a round's output,
+# and offsets on both sides of the output ring of every stream-to-wavefront
+# mapping (4 KiB, 16 KiB and 32 KiB rings) and of one output step.
+ROUND_PLANS = {
+    "round_limits": ([(0, 2), (14, 16), (57, 61)], [(1, 70), (250, 300)], [(4, 5), (18, 20), (271, 276)]),
+    "full_rounds": ([(0, 1)], [(1, 20), (300, 600)], [(200, 273)]),
+    "ring_edges": ([(0, 5)], [(4020, 4100), (3580, 3590), (15350, 15370), (16380, 16390), (30710, 30730), (32760, 32775)],
+                   [(4, 80)]),
+    "step_edges": ([(0, 3)], [(60, 70), (500, 530), (1000, 1040)], [(4, 40), (510, 515)]),
+    "repeats": ([(0, 20)], [(1, 2), (4, 4), (8, 8), (16, 17)], [(505, 520), (4090, 4100), (17000, 17010)]),
+    **{k: LZ4_PLANS[k] for k in ("mixed", "long-matches", "far-long", "edges")},
+}
+
+
+# the decoder gives a stream 8, 4 or 1 wavefronts by the number of streams of the launch
+@pytest.mark.parametrize("copies", [3, 700, 2100])
+@pytest.mark.parametrize("plan", sorted(ROUND_PLANS))
+def test_crafted_lz4_rounds(ctx, orc, plan, copies):
+    print(f"case: crafted lz4 rounds {plan} x {copies}", flush=True)
+    lits, offs, mls = ROUND_PLANS[plan]
+    c = ia.Context(clevel=5, filters=0)
+    chunks, want = [], []
+    for i, n in enumerate([41_001, 36_864, 50_003]):
+        rng = np.random.default_rng(zlib.crc32(plan.encode()) + n)
+        stream, raw = _craft_lz4(rng, n, lambda r: (_choice(r, lits), _choice(r, offs), _choice(r, mls)))
+        assert orc.lz4_decode(stream, n) == raw
+        chunks.append(_one_stream_chunk(c, stream, n))
+        want.append(raw)
+    got = ia.decode_chunks_flat(c, [chunks[i % 3] for i in range(copies)], sum(len(want[i % 3]) for i in range(copies)))
+    at = 0
+    for i in range(copies):
+        assert got[at:at + len(want[i % 3])] == want[i % 3], i
+        at += len(want[i % 3])
+
+
+@pytest.mark.parametrize("copies", [3, 700, 2100])
+def test_corrupt_stream_among_many(ctx, orc, copies):
+    rng = np.random.default_rng(copies)
+    c = ia.Context(clevel=5, filters=0)
+    stream, raw = _craft_lz4(rng, 3000, lambda r: (int(r.integers(0, 8)), int(r.integers(1, 600)), int(r.integers(4, 40))))
+    good = _one_stream_chunk(c, stream, 3000)
+    short = _one_stream_chunk(c, stream[:-7], 3000)  # ends early
+    chunks = [good] * copies
+    chunks[copies // 2] = short
+    with pytest.raises(ia.IArrayError):
+        ia.decode_chunks_flat(c, chunks, 3000 * copies)
+    assert ia.decode_chunks_flat(c, [good] * copies, 3000 * copies) == raw * copies
+
+
 # ---- BloscLZ streams and chunks of mixed codecs ------------------------------------------------
 def _cblosc_compress(b, compressor, raw, clevel, shuf, ts, bs):
     b.blosc_set_compressor(compressor)
