@@ -74,6 +74,11 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// A sequence that rounds decode has at most one literal and one match length
+// byte: 269 literals and a match of 273 bytes, in kSeqIn input bytes.
+constexpr int kSeqIn = 1 + 1 + 269 + 2 + 1;
+constexpr int kSeqOut = 269 + 273;
+
 // Sizes of a stream decoder of NW wavefronts (NW > 1: one window of 64 input
 // positions per wavefront and round).
 template <int NW>
@@ -82,7 +87,7 @@ struct Lz4Geom {
   static constexpr int kRing = 4096 * NW;         // output history, bytes
   static constexpr int kOut = 256 * NW;           // most output bytes of a round
   static constexpr int kStep = kOut;              // output bytes of a step of the general path
-  static constexpr int kStageWords = 16 * NW + 24;  // input of a round: 64 NW positions and what the last ones reach
+  static constexpr int kStageWords = 16 * NW + 72;  // input of a round: 64 NW positions and what the last ones reach
   static constexpr int kStage = 4 * kStageWords;
   static constexpr int kSeqs = 22 * NW;           // a sequence takes at least 3 input bytes
   // LDS: ring, two stages, sequence table, first-output-byte bits, source
@@ -91,13 +96,15 @@ struct Lz4Geom {
   static constexpr int kBitsAt = kTabAt + 8 * kSeqs;
   static constexpr int kRecAt = kBitsAt + kOut / 8;
   static constexpr int kExitAt = kRecAt + 4 * kThreads;
-  static constexpr int kTotAt = kExitAt + kThreads;
+  static constexpr int kTotAt = kExitAt + 2 * kThreads;
   static constexpr int kCutAt = kTotAt + ((4 * NW + 7) & ~7);
   static constexpr int kLds = kCutAt + 8;
-  static_assert(kOut >= 59 + 273, "a round holds any one sequence");
+  static_assert(kOut >= kSeqOut, "a round holds any one sequence");
+  static_assert(kStage >= 3 + 64 * NW + kSeqIn + 8, "and the stage its input");
 };
 
-// One wavefront: three windows of 63 positions a round, at most 64 sequences.
+// One wavefront: up to three windows of 63 positions a round, at most 64
+// sequences.
 template <>
 struct Lz4Geom<1> {
   static constexpr int kThreads = 64;
@@ -110,6 +117,7 @@ struct Lz4Geom<1> {
   static constexpr int kBitsAt = kTabAt + 8 * kSeqs;
   static constexpr int kListAt = kBitsAt + kOut / 8;
   static constexpr int kLds = kListAt + 2 * kSeqs;
+  static_assert(kOut >= kSeqOut, "a round holds any one sequence");
 };
 
 // One LZ4 stream by one workgroup of NW wavefronts.  The state (input and
@@ -119,8 +127,8 @@ struct Lz4Geom<1> {
 // Rounds.  A round takes the 64 NW input positions from `base`, whatever the
 // sequences in them, so its input is staged in LDS one round ahead.
 //   headers  thread t decodes the sequence that would start at position base
-//            + t.  Sequences of at most 63 input bytes, 59 literals and 273
-//            match bytes inside the stream are decoded by rounds (`ok`).
+//            + t.  Sequences of at most 269 literals and 273 match bytes (one
+//            length byte each) inside the stream are decoded by rounds (`ok`).
 //   reach    each wavefront follows the sequences of its 64-position window
 //            from all 64 starts at once, by pointer doubling (at most 21
 //            hops): the set of starts passed, and where the chain leaves the
@@ -232,10 +240,9 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         put_stage(have - 256, c);
       }
       for (;;) {
-        // a round reads at most 384 bytes from ip (three windows entered 125
-        // apart, and what the last one's sequences reach); one window's worth
-        // less than it loads ahead is usual
-        while (have < ip + 384) {
+        // no window of a round starts more than 320 bytes from ip, and its last
+        // sequence starts within 62
+        while (have < ip + 320 + 62 + kSeqIn + 8) {
           put_stage(have, ld_word(have, lane));
           have += 256;
         }
@@ -251,7 +258,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           const uint32_t h = lds_u32(stage + ((at + lane) & SM));
           const uint32_t hl = (h >> 4) & 15u, lb = (h >> 8) & 255u;
           const int32_t adv = 3 + (int32_t)hl + (hl == 15 ? (int32_t)lb + 1 : 0) + ((h & 15u) == 15 ? 1 : 0);
-          const bool ok = ((adv <= 63) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
+          const bool ok = (!((hl == 15) & (lb == 255)) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
           const int32_t to = ok ? min(lane + adv, WIN) : lane;
           const int32_t to2 = bperm(to, to);
           uint64_t starts = 0;
@@ -269,7 +276,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           n += __builtin_popcountll(starts);
           const int32_t last = 63 - __builtin_clzll(starts);
           at += last + (int32_t)rdlane((uint32_t)adv, last);
-          if (stopped || n >= G::kSeqs) break;
+          if (stopped || n >= G::kSeqs || at - ip > 320) break;
         }
         if (n == 0) {
           general = true;
@@ -383,7 +390,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       }
     } else {
       volatile uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
-      uint8_t *exits = lds + G::kExitAt;
+      uint16_t *exits = reinterpret_cast<uint16_t *>(lds + G::kExitAt);
       uint32_t *tot = reinterpret_cast<uint32_t *>(lds + G::kTotAt);
       unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
       int32_t base = ip, entry = 0, buf = 0;
@@ -409,10 +416,10 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
         const int32_t adv = 3 + lit + (int32_t)(lext + ext);
         // (bitwise: one vector compare chain, no branches)
-        const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) & (adv <= 63) &
+        const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
                          (adv <= iend - base - tid)) != 0;
         const uint64_t okm = __ballot(ok);
-        // reach: 64 and more is a position of the next window; a start that is
+        // reach: 64 and more is a position of a later window; a start that is
         // not ok leads to itself
         int32_t to = ok ? lane + adv : lane;
         uint32_t rlo = lane < 32 ? 1u << lane : 0u, rhi = lane < 32 ? 0u : 1u << (lane - 32);
@@ -425,20 +432,21 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           rhi |= in ? fhi : 0u;
           to = in ? f : to;
         }
-        exits[tid] = (uint8_t)to;
+        exits[tid] = (uint16_t)to;
         lds_barrier();
         // chain
-        uint32_t ex[(NW + 3) / 4];
+        uint32_t ex[NW / 2];  // lane l of ex[v]: the exits of starts 2 l and 2 l + 1 of windows 2 v and 2 v + 1
 #pragma unroll
-        for (int v = 0; v < (NW + 3) / 4; v++) ex[v] = reinterpret_cast<const uint32_t *>(exits)[(64 * v + lane) & (16 * NW - 1)];
+        for (int v = 0; v < NW / 2; v++) ex[v] = reinterpret_cast<const uint32_t *>(exits)[64 * v + lane];
         int32_t e = entry, mine_at = 64, stop = -1;
 #pragma unroll
         for (int v = 0; v < NW; v++) {
-          if (stop < 0) {
-            if (v == wave) mine_at = e;
-            const int32_t x = (int32_t)((rdlane(ex[v / 4], 16 * (v & 3) + (e >> 2)) >> (8 * (e & 3))) & 255u);
+          if ((e >> 6) == v) {
+            if (v == wave) mine_at = e & 63;
+            const uint32_t two = rdlane(ex[v / 2], (e >> 1) & 63);
+            const int32_t x = (int32_t)(e & 1 ? two >> 16 : two & 0xffffu);
             if (x < 64) stop = 64 * v + x;
-            e = x - 64;
+            e = x < 64 ? -1 : 64 * v + x;
           }
         }
         if (stop == entry) {  // the first sequence is not one for a round
@@ -551,8 +559,12 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           ip = base + stop;
           break;
         }
+        if (e >= 128 * NW) {  // past all of the next round
+          ip = base + e;
+          break;
+        }
         base = nbase;
-        entry = e;
+        entry = e - 64 * NW;
         buf ^= 1;
       }
     }

@@ -336,12 +336,13 @@ def test_crafted_lz4_streams(ctx, orc, plan, n):
     assert got == want
 
 
-# Lengths on both sides of what a decoding round holds (59 literals, a match of
-# 273 bytes, 63 input bytes a sequence), matches that fill a round's output,
+# Lengths on both sides of what a decoding round holds (269 literals, a match of
+# 273 bytes) and of a window (63 input bytes), matches that fill a round's output,
 # and offsets on both sides of the output ring of every stream-to-wavefront
 # mapping (4 KiB, 16 KiB and 32 KiB rings) and of one output step.
 ROUND_PLANS = {
     "round_limits": ([(0, 2), (14, 16), (57, 61)], [(1, 70), (250, 300)], [(4, 5), (18, 20), (271, 276)]),
+    "row_literals": ([(90, 130), (267, 272)], [(1, 3), (60, 200)], [(4, 40)]),
     "full_rounds": ([(0, 1)], [(1, 20), (300, 600)], [(200, 273)]),
     "ring_edges": ([(0, 5)], [(4020, 4100), (3580, 3590), (15350, 15370), (16380, 16390), (30710, 30730), (32760, 32775)],
                    [(4, 80)]),
