@@ -4,16 +4,20 @@
 // workgroup per compressed A block turns the block's streams straight into
 // row sums of A_blk x_seg without writing A anywhere.
 //
-// Bit-shuffled single-stream blocks (the common case) take the quad path:
-// a thread takes 32 consecutive elements ("quad" u = elements 32u..32u+31):
-// one dword from each of the 8*typesize bit planes (byte 4u..4u+3 of every
-// plane), byte-permutes them into 8-byte columns, runs one 8x8 bit-matrix
-// transpose per (group, element byte) and byte-permutes the results into
-// elements.  A quad spans at most two rows of the block (rows have >= 32
-// elements), so it leaves two partial sums in LDS; then one thread per row
-// adds its quads' partial sums in quad order.  Any other block layout takes
-// the group path: 8 elements per thread, bytes gathered one by one.
-// Rows are processed in windows so the partials fit in LDS.  Row sums land in
+// Bit-shuffled single-stream blocks take the quad path: a thread takes 32
+// consecutive elements ("quad" u = elements 32u..32u+31): one dword from each
+// of the 8*typesize bit planes (byte 4u..4u+3 of every plane), byte-permutes
+// them into 8-byte columns, runs one 8x8 bit-matrix transpose per (group,
+// element byte) and byte-permutes the results into elements.  A quad spans at
+// most two rows of the block (rows have >= 32 elements), so it leaves two
+// partial sums in LDS; then one thread per row adds its quads' partial sums in
+// quad order.  Byte-shuffled blocks take the plane path, the same with 16
+// elements a thread: 16 bytes from each of the typesize planes and 4x4 byte
+// transposes.  Any other block layout takes the group path: 8 elements per
+// thread, bytes gathered one by one.
+// Rows are processed in windows so the partials fit in LDS; where a matrix has
+// too few blocks for the GPU, several workgroups share a block's rows (a row's
+// sum is the same whichever workgroup forms it).  Row sums land in
 // partial[block column][row]; a second launch adds the block columns in
 // order, so y is bit-identical run to run.
 #include "iamx_internal.h"
@@ -93,6 +97,10 @@ struct Word<double> {
   }
 };
 
+// 4 and 16 bytes at any address
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
 struct Src {
   const IAMX_GLOBAL uint8_t *ptr[IAMX_MAX_STREAMS];
   uint8_t fill[IAMX_MAX_STREAMS];
@@ -103,17 +111,16 @@ struct Src {
 // unshuffled and form one more (short) quad.
 template <typename T>
 __device__ void quad_path(const IAMX_GLOBAL uint8_t *base, int32_t n, int32_t n8, int32_t rowlen, int32_t cols,
-                          int32_t vrows, int32_t vcols, const T *xs, T *p0, T *p1, T *prow, int64_t row0,
-                          int64_t M) {
+                          int32_t rfirst, int32_t rlast, int32_t vcols, const T *xs, T *p0, T *p1, T *prow,
+                          int64_t row0, int64_t M) {
   constexpr int TS = sizeof(T);
   constexpr int NP = 8 * TS;
   const int tid = threadIdx.x;
   const int32_t nq = n8 / 32;  // quads drawn whole from the planes
   const int32_t nqe = (n + 31) / 32;
-  const bool aligned = ((rowlen & 3) == 0) && ((((uint64_t)base) & 3) == 0);
   const int32_t rows_per_win = (int32_t)(((int64_t)(kGroups - 2) * 32) / cols);
-  for (int32_t ra = 0; ra < vrows; ra += rows_per_win) {
-    const int32_t rb = min(vrows, ra + rows_per_win);
+  for (int32_t ra = rfirst; ra < rlast; ra += rows_per_win) {
+    const int32_t rb = min(rlast, ra + rows_per_win);
     const int32_t u0 = (ra * cols) / 32, u1 = min(nqe - 1, (rb * cols - 1) / 32);  // quads [u0, u1]
     for (int32_t u = u0 + tid; u <= u1; u += 256) {
       const int32_t e0 = 32 * u;
@@ -123,16 +130,8 @@ __device__ void quad_path(const IAMX_GLOBAL uint8_t *base, int32_t n, int32_t n8
       T s0 = 0, s1 = 0;
       if (u < nq) {
         uint32_t d[NP];
-        if (aligned) {
 #pragma unroll
-          for (int p = 0; p < NP; p++) d[p] = *(const IAMX_GLOBAL uint32_t *)(base + (int64_t)p * rowlen + 4 * u);
-        } else {
-#pragma unroll
-          for (int p = 0; p < NP; p++) {
-            const IAMX_GLOBAL uint8_t *q = base + (int64_t)p * rowlen + 4 * u;
-            d[p] = (uint32_t)q[0] | ((uint32_t)q[1] << 8) | ((uint32_t)q[2] << 16) | ((uint32_t)q[3] << 24);
-          }
-        }
+        for (int p = 0; p < NP; p++) d[p] = *(const IAMX_GLOBAL u32_any *)(base + (int64_t)p * rowlen + 4 * u);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           // Y[j] = bit transpose of byte g of planes 8j..8j+7: byte i is byte j of element 8g+i
@@ -227,6 +226,76 @@ __device__ void quad_path(const IAMX_GLOBAL uint8_t *base, int32_t n, int32_t n8
   }
 }
 
+// Row sums of one byte-shuffled block, 16 elements a thread.  Plane j holds
+// byte j of every element: n bytes at plane[j], or `fill[j]` throughout where
+// plane[j] is null.  Bound by reading the planes; gathering the bytes one by
+// one took 663 us on a 7001x5003 float64 matrix of 125x125 blocks.
+template <typename T>
+__device__ void plane_path(const IAMX_GLOBAL uint8_t *const *plane, const uint8_t *fill, int32_t n, int32_t cols,
+                           int32_t rfirst, int32_t rlast, int32_t vcols, const T *xs, T *p0, T *p1, T *prow,
+                           int64_t row0, int64_t M) {
+  constexpr int TS = sizeof(T);
+  const int tid = threadIdx.x;
+  const int32_t rows_per_win = (int32_t)(((int64_t)(kGroups - 2) * 16) / cols);
+  for (int32_t ra = rfirst; ra < rlast; ra += rows_per_win) {
+    const int32_t rb = min(rlast, ra + rows_per_win);
+    const int32_t u0 = (ra * cols) / 16, u1 = (rb * cols - 1) / 16;  // groups [u0, u1]
+    for (int32_t u = u0 + tid; u <= u1; u += 256) {
+      const int32_t e0 = 16 * u;
+      const int32_t r0 = e0 / cols;
+      const int32_t c0 = e0 - r0 * cols;
+      const int32_t k0 = cols - c0;  // elements of the group in row r0
+      uint32_t d[TS][4];
+#pragma unroll
+      for (int j = 0; j < TS; j++) {
+        const IAMX_GLOBAL uint8_t *p = plane[j];
+        if (!p) {
+#pragma unroll
+          for (int t = 0; t < 4; t++) d[j][t] = 0x01010101u * fill[j];
+        } else if (e0 + 16 <= n) {
+          const u32x4_any v = *(const IAMX_GLOBAL u32x4_any *)(p + e0);
+#pragma unroll
+          for (int t = 0; t < 4; t++) d[j][t] = v[t];
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            uint32_t v = 0;
+            for (int i = 0; i < 4; i++)
+              if (e0 + 4 * t + i < n) v |= (uint32_t)p[e0 + 4 * t + i] << (8 * i);
+            d[j][t] = v;
+          }
+        }
+      }
+      T s0 = 0, s1 = 0;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        uint32_t lo[4], hi[4] = {0, 0, 0, 0};
+        tr4(d[0][t], d[1][t], d[2][t], d[3][t], lo);
+        if (TS == 8) tr4(d[4 % TS][t], d[5 % TS][t], d[6 % TS][t], d[7 % TS][t], hi);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int32_t k = 4 * t + i;
+          const bool first = k < k0;
+          const int32_t c = first ? c0 + k : c0 + k - cols;
+          const T prod = c < vcols ? Word<T>::of(lo[i], hi[i]) * xs[xpad(c)] : (T)0;
+          if (first) s0 += prod;
+          else s1 += prod;
+        }
+      }
+      p0[u - u0] = s0;
+      p1[u - u0] = s1;
+    }
+    __syncthreads();
+    for (int32_t r = ra + tid; r < rb; r += 256) {
+      const int32_t ua = (r * cols) / 16, ub = (r * cols + cols - 1) / 16;
+      T acc = 0;
+      for (int32_t u = ua; u <= ub; u++) acc += ((16 * u) / cols == r) ? p0[u - u0] : p1[u - u0];
+      if (row0 + r < M) prow[row0 + r] = acc;
+    }
+    __syncthreads();
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__restrict__ jobs,
                                                     const int32_t *__restrict__ blk_rc, int njobs,
@@ -237,6 +306,8 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
   __shared__ Src S;
   __shared__ T xs[kMaxCols + kMaxCols / 32];
   __shared__ T p0[kGroups], p1[kGroups];
+  __shared__ const IAMX_GLOBAL uint8_t *plane[sizeof(T)];
+  __shared__ uint8_t pfill[sizeof(T)];
   __shared__ int job_ok;
   const int b = blockIdx.x;
   if (b >= njobs) return;
@@ -280,12 +351,26 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
   const bool bits = filter == IAMX_FILTER_BITSHUFFLE || filter == IAMX_FILTER_BITSHUFFLE_V2;
   const int32_t n8 = filter == IAMX_FILTER_BITSHUFFLE ? n - n % 8 : n;
   const int32_t rowlen = n8 / 8;
+  // this workgroup's share of the block's rows
+  const int32_t rfirst = (int32_t)((int64_t)vrows * blockIdx.y / gridDim.y);
+  const int32_t rlast = (int32_t)((int64_t)vrows * (blockIdx.y + 1) / gridDim.y);
+  if (rfirst >= rlast) return;
   if (bits && J.nstreams == 1 && S.ptr[0] != nullptr && cols >= 32 && n8 >= 32 && ts == (int)sizeof(T)) {
-    quad_path<T>(S.ptr[0], n, n8, rowlen, cols, vrows, vcols, xs, p0, p1, partial + (int64_t)bcol * M, row0, M);
+    quad_path<T>(S.ptr[0], n, n8, rowlen, cols, rfirst, rlast, vcols, xs, p0, p1, partial + (int64_t)bcol * M, row0, M);
     return;
   }
   const bool one_stream = J.nstreams == 1;
   const bool split_planes = filter == IAMX_FILTER_SHUFFLE && ts > 1;
+  if (split_planes && ts == (int)sizeof(T) && cols >= 16 && (one_stream || (J.nstreams == ts && neblock >= n))) {
+    if (tid < ts) {
+      const IAMX_GLOBAL uint8_t *p = S.ptr[one_stream ? 0 : tid];
+      plane[tid] = p && one_stream ? p + (int64_t)tid * n : p;
+      pfill[tid] = S.fill[one_stream ? 0 : tid];
+    }
+    __syncthreads();
+    plane_path<T>(plane, pfill, n, cols, rfirst, rlast, vcols, xs, p0, p1, partial + (int64_t)bcol * M, row0, M);
+    return;
+  }
 
   // byte q of the block's concatenated streams
   auto byte_at = [&](int32_t q) -> uint32_t {
@@ -305,7 +390,7 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
   if (rows_per_win <= 0) {
     // tiny blocks (fewer than 8 columns): one wavefront per row, plain gather
     const int lane = tid & 63, wave = tid >> 6;
-    for (int32_t r = wave; r < vrows; r += 4) {
+    for (int32_t r = rfirst + wave; r < rlast; r += 4) {
       T acc = 0;
       for (int32_t c = lane; c < vcols; c += 64) {
         const int32_t e = r * cols + c;
@@ -326,8 +411,8 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
     return;
   }
 
-  for (int32_t ra = 0; ra < vrows; ra += rows_per_win) {
-    const int32_t rb = min(vrows, ra + rows_per_win);
+  for (int32_t ra = rfirst; ra < rlast; ra += rows_per_win) {
+    const int32_t rb = min(rlast, ra + rows_per_win);
     const int32_t g0 = (ra * cols) / 8, g1 = (rb * cols - 1) / 8;  // groups [g0, g1]
     // phase 1: per-group partial sums for rows in [ra, rb)
     for (int32_t g = g0 + tid; g <= g1; g += 256) {
@@ -427,13 +512,17 @@ int gemv_fused_launch(int dtype, const iamx_lz4_job_t *d_lz4, int n_lz4, const i
   }
   const dim3 rgrid((unsigned)((M + 255) / 256));
   int *st = iamx::status_word();
+  // enough workgroups for 4 a CU (what the LDS holds), up to 16 to a block: the
+  // four 250x250 blocks of a 500x500 matrix took 36 us with one each
+  const int share = n_blocks >= 4 * iamx::g_num_cus ? 1 : (4 * iamx::g_num_cus + n_blocks - 1) / n_blocks;
+  const dim3 bgrid((unsigned)n_blocks, (unsigned)(share < 16 ? share : 16));
   if (dtype == 0) {
-    IAMX_LAUNCH("gemv_fused_f64", k_gemv_fused<double>, dim3(n_blocks), dim3(256), 0, d_blocks, d_blk_rc, n_blocks,
+    IAMX_LAUNCH("gemv_fused_f64", k_gemv_fused<double>, bgrid, dim3(256), 0, d_blocks, d_blk_rc, n_blocks,
                 (const double *)x, (const uint8_t *)d_scratch, (double *)d_partial, M, K, nbc, cap, st, d_xzero);
     IAMX_LAUNCH("gemv_reduce_f64", k_reduce_cols<double>, rgrid, dim3(256), 0, (const double *)d_partial, nbc, M,
                 (double *)y);
   } else if (dtype == 1) {
-    IAMX_LAUNCH("gemv_fused_f32", k_gemv_fused<float>, dim3(n_blocks), dim3(256), 0, d_blocks, d_blk_rc, n_blocks,
+    IAMX_LAUNCH("gemv_fused_f32", k_gemv_fused<float>, bgrid, dim3(256), 0, d_blocks, d_blk_rc, n_blocks,
                 (const float *)x, (const uint8_t *)d_scratch, (float *)d_partial, M, K, nbc, cap, st, d_xzero);
     IAMX_LAUNCH("gemv_reduce_f32", k_reduce_cols<float>, rgrid, dim3(256), 0, (const float *)d_partial, nbc, M,
                 (float *)y);
