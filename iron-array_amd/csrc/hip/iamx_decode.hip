@@ -8,11 +8,9 @@
 //                   are picked out by following them from every start, and
 //                   output bytes are produced one a lane, whatever sequences
 //                   they belong to.
-//   k_unfilter      one workgroup per block: gathers each element's bytes from
-//                   its byte planes (byte shuffle) or bit planes (bitshuffle,
-//                   8x8 bit-matrix transposes), and writes the element into its
-//                   tile of the dense destination, skipping the padding outside
-//                   the valid extent.
+//   k_unfilter      (iamx_unfilter.hip) gathers each element's bytes from its
+//                   byte or bit planes and writes it into its tile of the dense
+//                   destination.
 // Stream sources are either the compressed chunk arena (raw streams, read in
 // place), the LZ4 scratch, or a constant byte (zero / run streams, special
 // chunks).
@@ -21,28 +19,17 @@
 
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));  // at any address
-
-// Delta-swap transpose of an 8x8 bit matrix held in a uint64 (row r = byte r,
-// column c = bit c): bit 8r+c moves to bit 8c+r (Hacker's Delight, 7-3).
-__device__ __forceinline__ uint64_t transpose8(uint64_t x) {
-  uint64_t t;
-  t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
-  x = x ^ t ^ (t << 7);
-  t = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
-  x = x ^ t ^ (t << 14);
-  t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
-  x = x ^ t ^ (t << 28);
-  return x;
-}
+using iamx::tr4;
+using iamx::transpose8;
+using iamx::u32_any;
+using iamx::u32x4;
+using iamx::u32x4_any;
 
 __device__ __forceinline__ uint32_t rdlane(uint32_t v, int32_t l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
 }
 
 __device__ __forceinline__ uint32_t lds_u32(const uint8_t *p) {  // any alignment
-  typedef uint32_t u32_any __attribute__((aligned(1)));
   return *reinterpret_cast<const u32_any *>(p);
 }
 
@@ -897,203 +884,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 1
   lz4_stream<NW>(job, scratch, status, lds);
 }
 
-struct Planes {
-  const IAMX_GLOBAL uint8_t *ptr[IAMX_MAX_STREAMS];
-  uint8_t fill[IAMX_MAX_STREAMS];
-  uint8_t is_const[IAMX_MAX_STREAMS];
-};
-
-// Byte q of the block's concatenated streams.
-__device__ __forceinline__ uint8_t block_byte(const Planes &P, int32_t neblock, int32_t q) {
-  const int s = q / neblock;
-  const int32_t o = q - s * neblock;
-  return P.is_const[s] ? P.fill[s] : P.ptr[s][o];
-}
-
-template <typename T>
-__device__ __forceinline__ void put_elem(uint8_t *dst, int64_t idx, uint64_t v) {
-  reinterpret_cast<T *>(dst)[idx] = (T)v;
-}
-
-// 4x4 byte transpose: r[g] = bytes g of (a, b, c, d)
-__device__ __forceinline__ void bytes4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t r[4]) {
-  const uint32_t t0 = __builtin_amdgcn_perm(b, a, 0x05010400u);  // a0 b0 a1 b1
-  const uint32_t t1 = __builtin_amdgcn_perm(b, a, 0x07030602u);  // a2 b2 a3 b3
-  const uint32_t t2 = __builtin_amdgcn_perm(d, c, 0x05010400u);  // c0 d0 c1 d1
-  const uint32_t t3 = __builtin_amdgcn_perm(d, c, 0x07030602u);  // c2 d2 c3 d3
-  r[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-  r[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-  r[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  r[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
-
-// The 4 bytes at p as a little-endian dword, p of any alignment: the aligned
-// dword(s) holding them, funnel-shifted.  The second dword is read only when
-// p is unaligned, and then it holds p[3], so no read leaves the page of the
-// last byte asked for.
-__device__ __forceinline__ uint32_t load_u32_any(const IAMX_GLOBAL uint8_t *p) {
-  const uint64_t a = (uint64_t)p;
-  const IAMX_GLOBAL uint32_t *w = iamx::gptr<const uint32_t>(a & ~3ull);
-  const uint32_t sh = (uint32_t)(a & 3);
-  if (sh == 0) return w[0];
-  return __builtin_amdgcn_alignbyte(w[1], w[0], sh);
-}
-
-__device__ __forceinline__ void store_elem(uint8_t *dst, int ts, int64_t idx, uint64_t v) {
-  switch (ts) {
-    case 8: put_elem<uint64_t>(dst, idx, v); break;
-    case 4: put_elem<uint32_t>(dst, idx, v); break;
-    case 2: put_elem<uint16_t>(dst, idx, v); break;
-    default: put_elem<uint8_t>(dst, idx, v); break;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_unfilter(const iamx_block_job_t *__restrict__ jobs, int njobs,
-                                                  const uint8_t *__restrict__ scratch, uint8_t *__restrict__ dst) {
-  __shared__ iamx_block_job_t J;
-  __shared__ Planes P;
-  const int bj = blockIdx.x;
-  if (bj >= njobs) return;
-  if (threadIdx.x == 0) {
-    J = jobs[bj];
-    for (int s = 0; s < IAMX_MAX_STREAMS; s++) {
-      P.is_const[s] = (s >= J.nstreams) || J.kind[s] == IAMX_SRC_CONST;
-      P.fill[s] = s < J.nstreams ? J.fill[s] : 0;
-      P.ptr[s] = J.kind[s] == IAMX_SRC_ADDR      ? iamx::gptr<const uint8_t>(J.src[s])
-                 : J.kind[s] == IAMX_SRC_SCRATCH ? iamx::gptr<const uint8_t>((uint64_t)(scratch + J.src[s]))
-                                                 : nullptr;
-    }
-  }
-  __syncthreads();
-  const int ts = J.typesize;
-  const int32_t n = J.bsize / ts;  // elements in the block
-  const int32_t cols = J.cols;
-  const int64_t ld = J.dst_ld;
-  const int64_t base = J.dst_off;
-  // a transposed destination takes tile element (r, c) at base + c * ld + r
-  const bool tr = (J.filter & IAMX_JOB_TRANSPOSE) != 0;
-  const int64_t sr = tr ? 1 : ld, sc = tr ? ld : 1;
-  const int filter = J.filter & ~IAMX_JOB_TRANSPOSE;
-  if (filter == IAMX_FILTER_BITSHUFFLE || filter == IAMX_FILTER_BITSHUFFLE_V2) {
-    const int32_t n8 = filter == IAMX_FILTER_BITSHUFFLE ? n - n % 8 : n;
-    const int32_t rowlen = n8 / 8;
-    const int32_t ngroups = rowlen + (n - n8);  // 8-element groups, then tail elements one by one
-    for (int32_t g = threadIdx.x; g < ngroups; g += blockDim.x) {
-      uint64_t elems[8];
-      int cnt;
-      int32_t e0;
-      if (g < rowlen) {
-        for (int i = 0; i < 8; i++) elems[i] = 0;
-        for (int j = 0; j < ts; j++) {
-          uint64_t x = 0;
-          for (int k = 0; k < 8; k++) {
-            const int32_t q = (8 * j + k) * rowlen + g;
-            const uint8_t b = J.nstreams == 1 ? (P.is_const[0] ? P.fill[0] : P.ptr[0][q]) : block_byte(P, J.neblock, q);
-            x |= (uint64_t)b << (8 * k);
-          }
-          const uint64_t y = transpose8(x);
-          for (int i = 0; i < 8; i++) elems[i] |= ((y >> (8 * i)) & 0xffull) << (8 * j);
-        }
-        cnt = 8;
-        e0 = 8 * g;
-      } else {
-        const int32_t e = n8 + (g - rowlen);
-        uint64_t v = 0;
-        for (int j = 0; j < ts; j++) v |= (uint64_t)block_byte(P, J.neblock, e * ts + j) << (8 * j);
-        elems[0] = v;
-        cnt = 1;
-        e0 = e;
-      }
-      int32_t r = e0 / cols, c = e0 - r * cols;
-      for (int i = 0; i < cnt; i++) {
-        if (r < J.vrows && c < J.vcols) store_elem(dst, ts, base + (int64_t)r * sr + (int64_t)c * sc, elems[i]);
-        if (++c == cols) { c = 0; ++r; }
-      }
-    }
-    return;
-  }
-  // byte shuffle (planes) or no filter
-  const bool shuffled = filter == IAMX_FILTER_SHUFFLE && ts > 1;
-  const IAMX_GLOBAL uint8_t *plane[8];
-  uint8_t pconst[8], pfill[8];
-  if (shuffled) {
-    for (int j = 0; j < ts; j++) {
-      if (J.nstreams == ts) {
-        plane[j] = P.ptr[j]; pconst[j] = P.is_const[j]; pfill[j] = P.fill[j];
-      } else {  // one stream holds all planes back to back
-        plane[j] = P.ptr[0] ? P.ptr[0] + (int64_t)j * n : nullptr; pconst[j] = P.is_const[0]; pfill[j] = P.fill[0];
-      }
-    }
-  }
-  if (shuffled && (ts == 4 || ts == 8) && (J.nstreams == ts || J.nstreams == 1)) {
-    // Four consecutive elements per thread: one dword from each plane (a last
-    // group of fewer than 4 elements reads its bytes one by one, so nothing
-    // past the planes is read) and a 4x4 byte transpose per 4 planes.  The
-    // four are stored together when they share a row of an untransposed
-    // destination, one by one otherwise.
-    for (int32_t q = threadIdx.x; 4 * q < n; q += blockDim.x) {
-      const int32_t e0 = 4 * q;
-      const int32_t ne = min(4, n - e0);
-      uint32_t w[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        if (j >= ts) continue;
-        if (pconst[j]) {
-          w[j] = 0x01010101u * pfill[j];
-        } else if (ne == 4) {
-          w[j] = load_u32_any(plane[j] + e0);
-        } else {
-          uint32_t v = 0;
-          for (int i = 0; i < ne; i++) v |= (uint32_t)plane[j][e0 + i] << (8 * i);
-          w[j] = v;
-        }
-      }
-      uint32_t lo[4], hi[4] = {0, 0, 0, 0};
-      bytes4x4(w[0], w[1], w[2], w[3], lo);
-      if (ts == 8) bytes4x4(w[4], w[5], w[6], w[7], hi);
-      int32_t r = e0 / cols, c = e0 - r * cols;
-      if (!tr && ne == 4 && r < J.vrows && c + 4 <= J.vcols) {
-        const int64_t idx = base + (int64_t)r * ld + c;
-        if (((uint64_t)(dst + idx * ts) & 15) == 0) {
-          if (ts == 4) {
-            *iamx::gptr<u32x4>((uint64_t)(dst + idx * 4)) = u32x4{lo[0], lo[1], lo[2], lo[3]};
-          } else {
-            IAMX_GLOBAL u32x4 *o = iamx::gptr<u32x4>((uint64_t)(dst + idx * 8));
-            o[0] = u32x4{lo[0], hi[0], lo[1], hi[1]};
-            o[1] = u32x4{lo[2], hi[2], lo[3], hi[3]};
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; i++) store_elem(dst, ts, idx + i, ((uint64_t)hi[i] << 32) | lo[i]);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          if (i < ne && r < J.vrows && c < J.vcols)
-            store_elem(dst, ts, base + (int64_t)r * sr + (int64_t)c * sc, ((uint64_t)hi[i] << 32) | lo[i]);
-          if (++c == cols) {
-            c = 0;
-            ++r;
-          }
-        }
-      }
-    }
-    return;
-  }
-  for (int32_t r = threadIdx.x / 64; r < J.vrows; r += blockDim.x / 64) {
-    for (int32_t c = threadIdx.x % 64; c < J.vcols; c += 64) {
-      const int32_t e = r * cols + c;
-      uint64_t v = 0;
-      if (shuffled) {
-        for (int j = 0; j < ts; j++) v |= (uint64_t)(pconst[j] ? pfill[j] : plane[j][e]) << (8 * j);
-      } else {
-        for (int j = 0; j < ts; j++) v |= (uint64_t)block_byte(P, J.neblock, e * ts + j) << (8 * j);
-      }
-      store_elem(dst, ts, base + (int64_t)r * sr + (int64_t)c * sc, v);
-    }
-  }
-}
-
 __device__ __forceinline__ uint64_t load_elem(const uint8_t *src, int ts, int64_t idx) {
   switch (ts) {
     case 8: return reinterpret_cast<const uint64_t *>(src)[idx];
@@ -1181,8 +971,8 @@ __global__ __launch_bounds__(256) void k_pack(iamx_tiling_t t, const uint8_t *__
         }
       }
       uint32_t w[8];
-      bytes4x4(lo[0], lo[1], lo[2], lo[3], w);
-      if (ts == 8) bytes4x4(hi[0], hi[1], hi[2], hi[3], w + 4);
+      tr4(lo[0], lo[1], lo[2], lo[3], w);
+      if (ts == 8) tr4(hi[0], hi[1], hi[2], hi[3], w + 4);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         if (j >= ts) continue;
@@ -1265,9 +1055,8 @@ IAMX_API int iamx_decode(const iamx_lz4_job_t *d_lz4, int n_lz4, const iamx_bloc
     rc = iamx::launch_lz4("lz4_streams", d_lz4, n_lz4, d_scratch);
   if (rc) return rc;
   if (n_blocks > 0)
-    IAMX_LAUNCH("unfilter", k_unfilter, dim3(n_blocks), dim3(256), 0, d_blocks, n_blocks,
-                (const uint8_t *)d_scratch, (uint8_t *)d_dst);
-  return IAMX_OK;
+    rc = iamx::launch_unfilter(d_blocks, n_blocks, d_scratch, d_dst);
+  return rc;
 }
 
 IAMX_API int iamx_pack_blocks_range(const iamx_tiling_t *t, const void *d_src, int64_t src_ld, void *d_out,

@@ -24,6 +24,12 @@
 
 namespace {
 
+using iamx::tr4;
+using iamx::transpose8;
+using iamx::transpose8_32;
+using iamx::u32_any;
+using iamx::u32x4_any;
+
 template <typename T>
 __device__ __forceinline__ T bits_to(uint64_t v);
 template <>
@@ -35,52 +41,12 @@ __device__ __forceinline__ double bits_to<double>(uint64_t v) {
   return __longlong_as_double((long long)v);
 }
 
-__device__ __forceinline__ uint64_t transpose8(uint64_t x) {
-  uint64_t t;
-  t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
-  x = x ^ t ^ (t << 7);
-  t = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
-  x = x ^ t ^ (t << 14);
-  t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
-  x = x ^ t ^ (t << 28);
-  return x;
-}
-
 constexpr int kMaxCols = 1024;
 constexpr int kGroups = 2048;  // per-window groups (or quads) whose partial sums live in LDS
 
 // x is staged in LDS with one pad word per 32 columns: the lanes of a wave
 // read columns 32 apart, which then fall in different banks.
 __device__ __forceinline__ int xpad(int c) { return c + (c >> 5); }
-
-// 4x4 byte transpose: r[g] = bytes g of (a, b, c, d)
-__device__ __forceinline__ void tr4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t r[4]) {
-  const uint32_t t0 = __builtin_amdgcn_perm(b, a, 0x05010400u);  // a0 b0 a1 b1
-  const uint32_t t1 = __builtin_amdgcn_perm(b, a, 0x07030602u);  // a2 b2 a3 b3
-  const uint32_t t2 = __builtin_amdgcn_perm(d, c, 0x05010400u);  // c0 d0 c1 d1
-  const uint32_t t3 = __builtin_amdgcn_perm(d, c, 0x07030602u);  // c2 d2 c3 d3
-  r[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-  r[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-  r[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-  r[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
-
-// 8x8 bit transpose of (hi:lo) as two 32-bit halves (the delta swaps of
-// transpose8 below, the first two of which stay inside each half)
-__device__ __forceinline__ void transpose8_32(uint32_t &lo, uint32_t &hi) {
-  uint32_t t;
-  t = (lo ^ (lo >> 7)) & 0x00AA00AAu;
-  lo ^= t ^ (t << 7);
-  t = (hi ^ (hi >> 7)) & 0x00AA00AAu;
-  hi ^= t ^ (t << 7);
-  t = (lo ^ (lo >> 14)) & 0x0000CCCCu;
-  lo ^= t ^ (t << 14);
-  t = (hi ^ (hi >> 14)) & 0x0000CCCCu;
-  hi ^= t ^ (t << 14);
-  t = (lo ^ __builtin_amdgcn_alignbit(hi, lo, 28)) & 0xF0F0F0F0u;
-  lo ^= t ^ (t << 28);
-  hi ^= t >> 4;
-}
 
 template <typename T>
 struct Word;
@@ -96,10 +62,6 @@ struct Word<double> {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
   }
 };
-
-// 4 and 16 bytes at any address
-typedef uint32_t u32_any __attribute__((aligned(1)));
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 
 struct Src {
   const IAMX_GLOBAL uint8_t *ptr[IAMX_MAX_STREAMS];

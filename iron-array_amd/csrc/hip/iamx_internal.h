@@ -56,6 +56,10 @@ void blt_shutdown();
 int tune_run(int form, int64_t M, int64_t N, int64_t K, const int *cands, int ncand, int (*run)(int, void *),
              void *ctx, int *rc);
 
+// The un-filter pass of a decode (iamx_unfilter.hip): every block's streams
+// into its tile of the dense destination.
+int launch_unfilter(const iamx_block_job_t *d_blocks, int n_blocks, const void *d_scratch, void *d_dst);
+
 // Zstd streams: their decode pass (jobs of other codecs are skipped) and
 // whether it runs (switched on once a zstd stream has been planned).
 int launch_zstd(const char *name, const iamx_lz4_job_t *d_jobs, int njobs, void *d_scratch, int64_t cap);
@@ -79,6 +83,53 @@ struct ProfScope {
 template <typename T>
 __device__ __forceinline__ IAMX_GLOBAL T *gptr(uint64_t a) {
   return (IAMX_GLOBAL T *)a;
+}
+
+// 4 and 16 bytes, and the same at any address
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// Delta-swap transpose of an 8x8 bit matrix held in a uint64 (row r = byte r,
+// column c = bit c): bit 8r+c moves to bit 8c+r (Hacker's Delight, 7-3).
+__device__ __forceinline__ uint64_t transpose8(uint64_t x) {
+  uint64_t t;
+  t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
+  x = x ^ t ^ (t << 7);
+  t = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
+  x = x ^ t ^ (t << 14);
+  t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
+  x = x ^ t ^ (t << 28);
+  return x;
+}
+
+// 8x8 bit transpose of (hi:lo) as two 32-bit halves (the delta swaps of
+// transpose8 above, the first two of which stay inside each half)
+__device__ __forceinline__ void transpose8_32(uint32_t &lo, uint32_t &hi) {
+  uint32_t t;
+  t = (lo ^ (lo >> 7)) & 0x00AA00AAu;
+  lo ^= t ^ (t << 7);
+  t = (hi ^ (hi >> 7)) & 0x00AA00AAu;
+  hi ^= t ^ (t << 7);
+  t = (lo ^ (lo >> 14)) & 0x0000CCCCu;
+  lo ^= t ^ (t << 14);
+  t = (hi ^ (hi >> 14)) & 0x0000CCCCu;
+  hi ^= t ^ (t << 14);
+  t = (lo ^ __builtin_amdgcn_alignbit(hi, lo, 28)) & 0xF0F0F0F0u;
+  lo ^= t ^ (t << 28);
+  hi ^= t >> 4;
+}
+
+// 4x4 byte transpose: r[g] = bytes g of (a, b, c, d)
+__device__ __forceinline__ void tr4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t r[4]) {
+  const uint32_t t0 = __builtin_amdgcn_perm(b, a, 0x05010400u);  // a0 b0 a1 b1
+  const uint32_t t1 = __builtin_amdgcn_perm(b, a, 0x07030602u);  // a2 b2 a3 b3
+  const uint32_t t2 = __builtin_amdgcn_perm(d, c, 0x05010400u);  // c0 d0 c1 d1
+  const uint32_t t3 = __builtin_amdgcn_perm(d, c, 0x07030602u);  // c2 d2 c3 d3
+  r[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+  r[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+  r[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+  r[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
 }
 
 }  // namespace iamx

@@ -1,0 +1,425 @@
+// iamx_unfilter.hip -- the second launch of a block decode: un-shuffle or
+// bit-un-shuffle of every block's streams into its tile of a dense row-major
+// destination (or of its transposed image).
+//
+// A block's streams are the decoded LZ4 scratch, the compressed chunk arena
+// (raw streams, read in place) or a constant byte.  Three ways through a block:
+//   planes   byte-shuffled 4- and 8-byte elements, untransposed: 4 elements a
+//            thread, one dword from each byte plane and 4x4 byte transposes,
+//            stored together; four such groups in flight per thread.
+//   staged   bit-shuffled elements, and byte-shuffled ones with a transposed
+//            destination: some rows of the block at a time (16 KB) are put
+//            together in LDS, 32 (bits) or 4 (bytes) elements
+//            a thread, and written out along the destination's rows.
+//   general  any other layout, element by element.
+// All three are bound by memory, the first two by having enough loads in
+// flight: a block is shared by up to 16 workgroups when blocks are few.
+#include "iamx_internal.h"
+
+namespace {
+
+using iamx::tr4;
+using iamx::transpose8;
+using iamx::transpose8_32;
+using iamx::u32_any;
+using iamx::u32x4_any;
+
+constexpr int kThreads = 128;
+// Bytes of a staged piece (9 workgroups then fit a CU's LDS), with an element
+// of padding after every 32: a thread's 32 elements start in another bank than
+// its neighbour's.
+constexpr int kPieceBytes = 16128;
+__device__ __forceinline__ int32_t pad(int32_t k) { return k + (k >> 5); }
+constexpr int kBufBytes = kPieceBytes + kPieceBytes / 32 + 8;
+
+struct Planes {
+  const IAMX_GLOBAL uint8_t *ptr[IAMX_MAX_STREAMS];
+  uint8_t fill[IAMX_MAX_STREAMS];
+  uint8_t is_const[IAMX_MAX_STREAMS];
+};
+
+// Byte q of the block's concatenated streams.
+__device__ __forceinline__ uint8_t block_byte(const Planes &P, int32_t neblock, int32_t q) {
+  const int s = q / neblock;
+  const int32_t o = q - s * neblock;
+  return P.is_const[s] ? P.fill[s] : P.ptr[s][o];
+}
+
+template <typename T>
+__device__ __forceinline__ void put_elem(uint8_t *dst, int64_t idx, uint64_t v) {
+  reinterpret_cast<T *>(dst)[idx] = (T)v;
+}
+
+__device__ __forceinline__ void store_elem(uint8_t *dst, int ts, int64_t idx, uint64_t v) {
+  switch (ts) {
+    case 8: put_elem<uint64_t>(dst, idx, v); break;
+    case 4: put_elem<uint32_t>(dst, idx, v); break;
+    case 2: put_elem<uint16_t>(dst, idx, v); break;
+    default: put_elem<uint8_t>(dst, idx, v); break;
+  }
+}
+
+template <int TS>
+struct Elem;
+template <>
+struct Elem<4> {
+  typedef uint32_t T;
+  static __device__ __forceinline__ T of(uint32_t lo, uint32_t) { return lo; }
+};
+template <>
+struct Elem<8> {
+  typedef uint64_t T;
+  static __device__ __forceinline__ T of(uint32_t lo, uint32_t hi) { return ((uint64_t)hi << 32) | lo; }
+};
+
+// Division of x < 2^31 by a fixed d >= 1: m = floor(2^32 / d) + 1 gives the
+// quotient or one more.
+struct Div {
+  uint32_t d, m;
+  __device__ __forceinline__ explicit Div(int32_t v) : d((uint32_t)v), m((uint32_t)(0xffffffffu / (uint32_t)v) + 1u) {}
+  __device__ __forceinline__ int32_t operator()(int32_t x) const {
+    if (d == 1) return x;
+    const uint32_t q = __umulhi((uint32_t)x, m);
+    return (int32_t)(q * d > (uint32_t)x ? q - 1 : q);
+  }
+};
+
+// Four elements from e0 (ne of them) of a byte-shuffled block.
+template <int TS>
+__device__ __forceinline__ void load_planes(const IAMX_GLOBAL uint8_t *const *plane, const uint8_t *fill, int32_t e0,
+                                            int32_t n, uint32_t *w) {
+#pragma unroll
+  for (int j = 0; j < TS; j++) {
+    const IAMX_GLOBAL uint8_t *p = plane[j];
+    if (!p) {
+      w[j] = 0x01010101u * fill[j];
+    } else if (e0 + 4 <= n) {
+      w[j] = *(const IAMX_GLOBAL u32_any *)(p + e0);
+    } else {
+      uint32_t v = 0;
+      for (int i = 0; e0 + i < n; i++) v |= (uint32_t)p[e0 + i] << (8 * i);
+      w[j] = v;
+    }
+  }
+}
+
+template <int TS>
+__device__ __forceinline__ void join_planes(const uint32_t *w, typename Elem<TS>::T *v) {
+  uint32_t lo[4], hi[4] = {0, 0, 0, 0};
+  tr4(w[0], w[1], w[2], w[3], lo);
+  if (TS == 8) tr4(w[4 % TS], w[5 % TS], w[6 % TS], w[7 % TS], hi);
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = Elem<TS>::of(lo[i], hi[i]);
+}
+
+// planes: the block's rows [0, vrows), this workgroup's share.  A 256x256
+// float32 block is 16384 groups; with one group in flight the pass moved 2.4
+// TB/s on an 8192x8192 matrix (214 us), with four 4.9 TB/s (104 us).
+template <int TS>
+__device__ __forceinline__ void unfilter_planes(const IAMX_GLOBAL uint8_t *const *plane, const uint8_t *fill, int32_t n,
+                                const iamx_block_job_t &J, uint8_t *__restrict__ dst) {
+  typedef typename Elem<TS>::T T;
+  constexpr int U = 4;
+  const int32_t cols = J.cols, vrows = J.vrows, vcols = J.vcols;
+  const int64_t ld = J.dst_ld;
+  T *out = reinterpret_cast<T *>(dst) + J.dst_off;
+  const Div by_cols(cols);
+  const int32_t ng = (int32_t)(((int64_t)vrows * cols + 3) >> 2);
+  const int32_t step = kThreads * gridDim.y;
+  for (int32_t q0 = blockIdx.y * kThreads + threadIdx.x; q0 < ng; q0 += U * step) {
+    uint32_t w[U][TS];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (q0 + u * step < ng) load_planes<TS>(plane, fill, 4 * (q0 + u * step), n, w[u]);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (q0 + u * step >= ng) continue;
+      const int32_t e0 = 4 * (q0 + u * step);
+      T v[4];
+      join_planes<TS>(w[u], v);
+      int32_t r = by_cols(e0), c = e0 - r * cols;
+      if (c + 4 <= vcols) {  // one row (r < vrows)
+        T *o = out + (int64_t)r * ld + c;
+        if (TS == 4) {
+          *(IAMX_GLOBAL u32x4_any *)iamx::gptr<uint8_t>((uint64_t)o) =
+              u32x4_any{(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+        } else {
+          IAMX_GLOBAL u32x4_any *g = (IAMX_GLOBAL u32x4_any *)iamx::gptr<uint8_t>((uint64_t)o);
+          g[0] = u32x4_any{(uint32_t)v[0], (uint32_t)((uint64_t)v[0] >> 32), (uint32_t)v[1],
+                           (uint32_t)((uint64_t)v[1] >> 32)};
+          g[1] = u32x4_any{(uint32_t)v[2], (uint32_t)((uint64_t)v[2] >> 32), (uint32_t)v[3],
+                           (uint32_t)((uint64_t)v[3] >> 32)};
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (r < vrows && c < vcols) out[(int64_t)r * ld + c] = v[i];
+          if (++c == cols) {
+            c = 0;
+            ++r;
+          }
+        }
+      }
+    }
+  }
+}
+
+// Elements [32 u, 32 u + 32) of a bit-shuffled block, all of them below n8, the
+// ones in [ea, eb) into buf, 4 bytes of them at a time (32 planes: twice the
+// registers for 64 planes together spilled).  Plane p starts at base + p * rowlen.
+template <int TS>
+__device__ __forceinline__ void stage_bits(const IAMX_GLOBAL uint8_t *base, int32_t rowlen, int32_t u, int32_t ea,
+                                           int32_t eb, typename Elem<TS>::T *buf) {
+  const int32_t e0 = 32 * u;
+  uint32_t *out = reinterpret_cast<uint32_t *>(buf);
+#pragma unroll 1
+  for (int half = 0; half < TS / 4; half++) {
+    uint32_t d[32];
+#pragma unroll
+    for (int p = 0; p < 32; p++) d[p] = *(const IAMX_GLOBAL u32_any *)(base + (int64_t)(32 * half + p) * rowlen + 4 * u);
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      // Y[j] = bit transpose of byte g of planes 8j..8j+7: byte i is byte j of element 8g+i
+      uint32_t ylo[4], yhi[4];
+      const uint32_t sel = (uint32_t)g | ((uint32_t)(g + 4) << 8);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint32_t a0 = __builtin_amdgcn_perm(d[8 * j + 1], d[8 * j + 0], sel);
+        const uint32_t a1 = __builtin_amdgcn_perm(d[8 * j + 3], d[8 * j + 2], sel);
+        const uint32_t a2 = __builtin_amdgcn_perm(d[8 * j + 5], d[8 * j + 4], sel);
+        const uint32_t a3 = __builtin_amdgcn_perm(d[8 * j + 7], d[8 * j + 6], sel);
+        uint32_t lo = __builtin_amdgcn_perm(a1, a0, 0x05040100u);
+        uint32_t hi = __builtin_amdgcn_perm(a3, a2, 0x05040100u);
+        transpose8_32(lo, hi);
+        ylo[j] = lo;
+        yhi[j] = hi;
+      }
+      uint32_t v[8];
+      tr4(ylo[0], ylo[1], ylo[2], ylo[3], v);
+      tr4(yhi[0], yhi[1], yhi[2], yhi[3], v + 4);
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int32_t e = e0 + 8 * g + i;
+        if (e >= ea && e < eb) out[pad(e - ea) * (TS / 4) + half] = v[i];
+      }
+    }
+  }
+}
+
+// One element of a bit-shuffled block of n elements; elements [n8, n) follow
+// the planes unshuffled.
+template <int TS>
+__device__ __forceinline__ typename Elem<TS>::T one_of_bits(const IAMX_GLOBAL uint8_t *base, int32_t n8, int32_t e) {
+  uint64_t v = 0;
+  if (e < n8) {
+#pragma unroll 8
+    for (int p = 0; p < 8 * TS; p++) v |= (uint64_t)((base[(int64_t)p * (n8 / 8) + (e >> 3)] >> (e & 7)) & 1u) << p;
+  } else {
+    const IAMX_GLOBAL uint8_t *q = base + (int64_t)e * TS;
+#pragma unroll
+    for (int b = 0; b < TS; b++) v |= (uint64_t)q[b] << (8 * b);
+  }
+  return (typename Elem<TS>::T)v;
+}
+
+// staged: `bits` is the stream of a bit-shuffled block, null for a byte-shuffled
+// one.  The general path's byte gathers and scattered 8-byte stores took 199 us
+// on a 3001x4507 bit-shuffled float64 matrix (70 here) and 340 on the transposed
+// image of a 4001x6007 byte-shuffled one (104 here).
+template <int TS>
+__device__ __forceinline__ void unfilter_staged(const IAMX_GLOBAL uint8_t *bits, const IAMX_GLOBAL uint8_t *const *plane,
+                                const uint8_t *fill, int32_t n, int32_t n8, const iamx_block_job_t &J, bool tr,
+                                typename Elem<TS>::T *buf, uint8_t *__restrict__ dst) {
+  typedef typename Elem<TS>::T T;
+  constexpr int32_t kPiece = kPieceBytes / TS;
+  const int tid = threadIdx.x;
+  const int32_t cols = J.cols, vrows = J.vrows, vcols = J.vcols;
+  const int64_t ld = J.dst_ld;
+  T *out = reinterpret_cast<T *>(dst) + J.dst_off;
+  // pieces of whole rows, or of one row's kPiece columns
+  const bool whole = cols <= kPiece;
+  const int32_t prows = whole ? kPiece / cols : 1;
+  const int32_t segs = whole ? 1 : (vcols + kPiece - 1) / kPiece;
+  const int32_t npieces = whole ? (vrows + prows - 1) / prows : vrows * segs;
+  for (int32_t k = blockIdx.y; k < npieces; k += gridDim.y) {
+    int32_t r0, c0, nr, nc;  // rows and columns of the piece (whole rows keep their padding columns in LDS)
+    if (whole) {
+      r0 = k * prows;
+      nr = min(prows, vrows - r0);
+      c0 = 0;
+      nc = cols;
+    } else {
+      r0 = k / segs;
+      nr = 1;
+      c0 = (k - r0 * segs) * kPiece;
+      nc = min(kPiece, vcols - c0);
+    }
+    const int32_t ea = r0 * cols + c0, eb = ea + (nr - 1) * cols + nc;
+    if (bits) {
+      const int32_t eq = min(eb, n8 & ~31);  // whole groups of 32 end here
+      for (int32_t u = ea / 32 + tid; 32 * u < eq; u += kThreads) stage_bits<TS>(bits, n8 / 8, u, ea, eb, buf);
+      for (int32_t e = max(ea, n8 & ~31) + tid; e < eb; e += kThreads) buf[pad(e - ea)] = one_of_bits<TS>(bits, n8, e);
+    } else {
+      constexpr int U = 4;
+      for (int32_t e0 = ea + 4 * tid; e0 < eb; e0 += 4 * U * kThreads) {
+        uint32_t w[U][TS];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (e0 + 4 * u * kThreads < eb) load_planes<TS>(plane, fill, e0 + 4 * u * kThreads, n, w[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          T v[4];
+          join_planes<TS>(w[u], v);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int32_t e = e0 + 4 * u * kThreads + i;
+            if (e < eb) buf[pad(e - ea)] = v[i];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    const int32_t wc = min(nc, vcols - c0);  // columns written
+    if (tr) {
+      const Div by_rows(nr);
+      for (int32_t i = tid; i < nr * wc; i += kThreads) {
+        const int32_t c = by_rows(i), r = i - c * nr;
+        out[(int64_t)(c0 + c) * ld + r0 + r] = buf[pad(r * nc + c)];
+      }
+    } else {
+      const Div by_wc(wc);
+      for (int32_t i = tid; i < nr * wc; i += kThreads) {
+        const int32_t r = by_wc(i), c = i - r * wc;
+        out[(int64_t)(r0 + r) * ld + c0 + c] = buf[pad(r * nc + c)];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_unfilter(
+    const iamx_block_job_t *__restrict__ jobs, int njobs, const uint8_t *__restrict__ scratch,
+    uint8_t *__restrict__ dst) {
+  __shared__ iamx_block_job_t J;
+  __shared__ Planes P;
+  __shared__ const IAMX_GLOBAL uint8_t *plane[8];
+  __shared__ uint8_t pfill[8];
+  __shared__ uint64_t buf[kBufBytes / 8];
+  const int bj = blockIdx.x;
+  if (bj >= njobs) return;
+  if (threadIdx.x == 0) {
+    J = jobs[bj];
+    for (int s = 0; s < IAMX_MAX_STREAMS; s++) {
+      P.is_const[s] = (s >= J.nstreams) || J.kind[s] == IAMX_SRC_CONST;
+      P.fill[s] = s < J.nstreams ? J.fill[s] : 0;
+      P.ptr[s] = J.kind[s] == IAMX_SRC_ADDR      ? iamx::gptr<const uint8_t>(J.src[s])
+                 : J.kind[s] == IAMX_SRC_SCRATCH ? iamx::gptr<const uint8_t>((uint64_t)(scratch + J.src[s]))
+                                                 : nullptr;
+      if (P.is_const[s]) P.ptr[s] = nullptr;
+    }
+  }
+  __syncthreads();
+  const int ts = J.typesize;
+  const int32_t n = J.bsize / ts;  // elements in the block
+  const int32_t cols = J.cols;
+  const int64_t ld = J.dst_ld;
+  const int64_t base = J.dst_off;
+  // a transposed destination takes tile element (r, c) at base + c * ld + r
+  const bool tr = (J.filter & IAMX_JOB_TRANSPOSE) != 0;
+  const int filter = J.filter & ~IAMX_JOB_TRANSPOSE;
+  const bool bits = filter == IAMX_FILTER_BITSHUFFLE || filter == IAMX_FILTER_BITSHUFFLE_V2;
+  const bool shuffled = filter == IAMX_FILTER_SHUFFLE && ts > 1;
+  const int32_t n8 = filter == IAMX_FILTER_BITSHUFFLE ? n - n % 8 : n;
+  if (cols < 1 || J.vrows < 1 || J.vcols < 1) return;
+  const bool fits = (int64_t)J.vrows * cols <= n && J.vcols <= cols;
+  if (fits && (ts == 4 || ts == 8) &&
+      ((shuffled && (J.nstreams == ts || J.nstreams == 1)) || (bits && J.nstreams == 1 && P.ptr[0]))) {
+    if (shuffled) {
+      if (threadIdx.x < ts) {
+        const int j = threadIdx.x;
+        // one stream holds all planes back to back
+        const IAMX_GLOBAL uint8_t *p = P.ptr[J.nstreams == ts ? j : 0];
+        plane[j] = p && J.nstreams != ts ? p + (int64_t)j * n : p;
+        pfill[j] = P.fill[J.nstreams == ts ? j : 0];
+      }
+      __syncthreads();
+    }
+    const IAMX_GLOBAL uint8_t *stream = bits ? P.ptr[0] : nullptr;
+    if (shuffled && !tr) {
+      if (ts == 4) unfilter_planes<4>(plane, pfill, n, J, dst);
+      else unfilter_planes<8>(plane, pfill, n, J, dst);
+    } else if (ts == 4) {
+      unfilter_staged<4>(stream, plane, pfill, n, n8, J, tr, reinterpret_cast<uint32_t *>(buf), dst);
+    } else {
+      unfilter_staged<8>(stream, plane, pfill, n, n8, J, tr, buf, dst);
+    }
+    return;
+  }
+  // general
+  const int64_t sr = tr ? 1 : ld, sc = tr ? ld : 1;
+  if (bits) {
+    const int32_t rowlen = n8 / 8;
+    const int32_t ngroups = rowlen + (n - n8);  // 8-element groups, then tail elements one by one
+    for (int32_t g = blockIdx.y * kThreads + threadIdx.x; g < ngroups; g += kThreads * gridDim.y) {
+      uint64_t elems[8];
+      int cnt;
+      int32_t e0;
+      if (g < rowlen) {
+        for (int i = 0; i < 8; i++) elems[i] = 0;
+        for (int j = 0; j < ts; j++) {
+          uint64_t x = 0;
+          for (int k = 0; k < 8; k++) {
+            const int32_t q = (8 * j + k) * rowlen + g;
+            const uint8_t b = J.nstreams == 1 ? (P.is_const[0] ? P.fill[0] : P.ptr[0][q]) : block_byte(P, J.neblock, q);
+            x |= (uint64_t)b << (8 * k);
+          }
+          const uint64_t y = transpose8(x);
+          for (int i = 0; i < 8; i++) elems[i] |= ((y >> (8 * i)) & 0xffull) << (8 * j);
+        }
+        cnt = 8;
+        e0 = 8 * g;
+      } else {
+        const int32_t e = n8 + (g - rowlen);
+        uint64_t v = 0;
+        for (int j = 0; j < ts; j++) v |= (uint64_t)block_byte(P, J.neblock, e * ts + j) << (8 * j);
+        elems[0] = v;
+        cnt = 1;
+        e0 = e;
+      }
+      int32_t r = e0 / cols, c = e0 - r * cols;
+      for (int i = 0; i < cnt; i++) {
+        if (r < J.vrows && c < J.vcols) store_elem(dst, ts, base + (int64_t)r * sr + (int64_t)c * sc, elems[i]);
+        if (++c == cols) { c = 0; ++r; }
+      }
+    }
+    return;
+  }
+  // byte shuffle (planes) or no filter
+  auto plane_byte = [&](int j, int32_t e) -> uint64_t {
+    if (J.nstreams == ts) return P.is_const[j] ? P.fill[j] : P.ptr[j][e];
+    return P.is_const[0] ? P.fill[0] : P.ptr[0][(int64_t)j * n + e];
+  };
+  for (int32_t r = blockIdx.y * (kThreads / 64) + threadIdx.x / 64; r < J.vrows; r += kThreads / 64 * gridDim.y) {
+    for (int32_t c = threadIdx.x % 64; c < J.vcols; c += 64) {
+      const int32_t e = r * cols + c;
+      uint64_t v = 0;
+      if (shuffled) {
+        for (int j = 0; j < ts; j++) v |= plane_byte(j, e) << (8 * j);
+      } else {
+        for (int j = 0; j < ts; j++) v |= (uint64_t)block_byte(P, J.neblock, e * ts + j) << (8 * j);
+      }
+      store_elem(dst, ts, base + (int64_t)r * sr + (int64_t)c * sc, v);
+    }
+  }
+}
+
+}  // namespace
+
+int iamx::launch_unfilter(const iamx_block_job_t *d_blocks, int n_blocks, const void *d_scratch, void *d_dst) {
+  // enough workgroups for 16 a CU, up to 16 to a block
+  const int want = 16 * g_num_cus;
+  const int share = n_blocks >= want ? 1 : (want + n_blocks - 1) / n_blocks;
+  IAMX_LAUNCH("unfilter", k_unfilter, dim3((unsigned)n_blocks, (unsigned)(share < 16 ? share : 16)), dim3(kThreads), 0,
+              d_blocks, n_blocks, (const uint8_t *)d_scratch, (uint8_t *)d_dst);
+  return IAMX_OK;
+}
