@@ -7,8 +7,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <map>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "iamx_internal.h"
@@ -161,6 +163,34 @@ struct Workspace {
 };
 static Workspace g_ws[IAMX_WORKSPACES];
 
+// ---- device blocks -------------------------------------------------------------------
+// Freed blocks of at most kKeepBlock bytes are kept for the next iamx_malloc
+// of about their size, kKeepBytes of them at most: a result's arena and job
+// tables come and go with every product, and each hipMalloc + hipFree pair cost
+// 20-300 us.  A block is kept only after the device has finished everything
+// queued before its free (what hipFree waits for too), so its next owner may
+// use it on any stream.  All are given back at shutdown, and when an allocation
+// fails.
+constexpr size_t kKeepBytes = (size_t)256 << 20, kKeepBlock = (size_t)64 << 20;
+static std::mutex g_blocks_mu;
+static std::unordered_map<void *, size_t> g_live_blocks;  // sizes of the blocks handed out
+static std::multimap<size_t, void *> g_kept_blocks;
+static size_t g_kept_bytes = 0;
+
+// sizes in steps of an eighth of a power of two, at least 4 KiB
+static size_t block_size(size_t bytes) {
+  size_t step = 512;
+  while (step * 16 <= bytes) step *= 2;
+  const size_t r = (bytes + step - 1) / step * step;
+  return r < 4096 ? 4096 : r;
+}
+
+static void release_kept() {
+  for (auto &b : g_kept_blocks) (void)hipFree(b.second);
+  g_kept_blocks.clear();
+  g_kept_bytes = 0;
+}
+
 }  // namespace iamx
 
 using namespace iamx;
@@ -184,16 +214,44 @@ IAMX_API int iamx_device_info(char *name, int namelen, int *cus, char *arch, int
 
 IAMX_API void *iamx_malloc(size_t bytes) {
   if (ensure_init()) return nullptr;
+  const size_t want = bytes <= kKeepBlock ? block_size(bytes) : bytes;
+  std::lock_guard<std::mutex> lk(g_blocks_mu);
   void *p = nullptr;
-  if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) {
+  const auto kept = g_kept_blocks.lower_bound(want);
+  if (want <= kKeepBlock && kept != g_kept_blocks.end() && kept->first <= want + want / 4) {
+    p = kept->second;
+    g_live_blocks[p] = kept->first;
+    g_kept_bytes -= kept->first;
+    g_kept_blocks.erase(kept);
+    return p;
+  }
+  hipError_t e = hipMalloc(&p, want);
+  if (e != hipSuccess && g_kept_bytes) {
+    release_kept();
+    e = hipMalloc(&p, want);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
     set_error(IAMX_ENOMEM, "hipMalloc(%zu) failed", bytes);
     return nullptr;
   }
+  g_live_blocks[p] = want;
   return p;
 }
 
 IAMX_API void iamx_free(void *p) {
-  if (p && g_init_state == 1) (void)hipFree(p);
+  if (!p || g_init_state != 1) return;
+  std::lock_guard<std::mutex> lk(g_blocks_mu);
+  const auto live = g_live_blocks.find(p);
+  const size_t bytes = live == g_live_blocks.end() ? 0 : live->second;
+  if (live != g_live_blocks.end()) g_live_blocks.erase(live);
+  if (bytes && bytes <= kKeepBlock && g_kept_bytes + bytes <= kKeepBytes && !capturing() &&
+      hipDeviceSynchronize() == hipSuccess) {
+    g_kept_blocks.emplace(bytes, p);
+    g_kept_bytes += bytes;
+    return;
+  }
+  (void)hipFree(p);
 }
 
 IAMX_API int iamx_h2d(void *dst, const void *src, size_t bytes) {
@@ -486,6 +544,10 @@ IAMX_API void iamx_shutdown(void) {
   if (g_init_state != 1) return;
   sync_streams();
   blt_shutdown();
+  {
+    std::lock_guard<std::mutex> lk(g_blocks_mu);
+    release_kept();
+  }
   for (auto &w : g_ws) {
     if (w.ptr) (void)hipFree(w.ptr);
     w = Workspace{};

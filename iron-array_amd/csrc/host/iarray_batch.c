@@ -145,7 +145,8 @@ static void append_jobs(const iarray_container_t *o, int64_t dense_off, int64_t 
 static ina_rc_t upload(void **d, const void *h, size_t bytes) {
   *d = iamx_malloc(bytes ? bytes : 16);
   if (!*d) return iax_dev_error(IAMX_ENOMEM, "batch plan");
-  int e = iamx_h2d(*d, h, bytes);
+  const iax_piece_t piece = {h, 0, bytes};
+  int e = iax_upload(*d, &piece, 1, 1);
   return e ? iax_dev_error(e, "batch plan upload") : INA_SUCCESS;
 }
 

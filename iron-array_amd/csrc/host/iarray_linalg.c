@@ -41,8 +41,7 @@ static struct {
 } g_pair;
 
 static void free_pair(void) {
-  iamx_free(g_pair.d_lz4);
-  iamx_free(g_pair.d_blocks);
+  iamx_free(g_pair.d_lz4); /* the blocks follow in the same device block */
   memset(&g_pair, 0, sizeof(g_pair));
 }
 
@@ -74,13 +73,19 @@ static ina_rc_t build_pair(iarray_container_t *a, iarray_container_t *b) {
   }
   iax_sort_lz4_jobs(lz4, nl);
   ina_rc_t rc = INA_SUCCESS;
-  g_pair.d_lz4 = (iamx_lz4_job_t *)iamx_malloc(sizeof(iamx_lz4_job_t) * (size_t)(nl ? nl : 1));
-  g_pair.d_blocks = (iamx_block_job_t *)iamx_malloc(sizeof(iamx_block_job_t) * (size_t)(nb ? nb : 1));
-  if (!g_pair.d_lz4 || !g_pair.d_blocks) rc = iax_dev_error(IAMX_ENOMEM, "pair plan");
-  int e = 0;
-  if (INA_SUCCEED(rc) && nl) e = iamx_h2d(g_pair.d_lz4, lz4, sizeof(iamx_lz4_job_t) * (size_t)nl);
-  if (INA_SUCCEED(rc) && !e && nb) e = iamx_h2d(g_pair.d_blocks, blk, sizeof(iamx_block_job_t) * (size_t)nb);
-  if (e) rc = iax_dev_error(e, "pair plan upload");
+  /* both tables in one device block */
+  const size_t o_blk = (sizeof(iamx_lz4_job_t) * (size_t)nl + 255) & ~(size_t)255;
+  const iax_piece_t pieces[2] = {{lz4, 0, sizeof(iamx_lz4_job_t) * (size_t)nl},
+                                 {blk, o_blk, sizeof(iamx_block_job_t) * (size_t)nb}};
+  uint8_t *d = (uint8_t *)iamx_malloc(o_blk + sizeof(iamx_block_job_t) * (size_t)(nb ? nb : 1));
+  g_pair.d_lz4 = (iamx_lz4_job_t *)d;
+  if (!d) {
+    rc = iax_dev_error(IAMX_ENOMEM, "pair plan");
+  } else {
+    g_pair.d_blocks = (iamx_block_job_t *)(d + o_blk);
+    const int e = iax_upload(d, pieces, 2, 1);
+    if (e) rc = iax_dev_error(e, "pair plan upload");
+  }
   free(lz4);
   free(blk);
   if (INA_FAILED(rc)) {

@@ -76,7 +76,7 @@ struct iarray_container_s {
   uint8_t **chunks;
   int32_t *csizes;
   /* device mirror */
-  uint8_t *d_arena;
+  uint8_t *d_arena; /* the chunks, then the plan's tables */
   int64_t *arena_off;
   int device_valid;
   uint64_t generation; /* bumped whenever the device arena is (re)built */
@@ -167,8 +167,15 @@ typedef int (*iax_rows_fn)(void *ctx, int64_t row0, int64_t nrows);
 /* ---- containers (iarray_container.c) ---------------------------------------------------- */
 ina_rc_t iax_container_new(iarray_context_t *ctx, iarray_dtshape_t *dtshape, iarray_storage_t *storage,
                            iarray_container_t **c);
-ina_rc_t iax_ensure_device(iarray_container_t *c);
+/* Builds and uploads the container's device mirror and decode plan on first use. */
 ina_rc_t iax_ensure_plan(iarray_container_t *c);
+/* Host pieces, in rising order of `off`, to d_dst + off; complete on return.
+ * Returns an iamx error code. */
+typedef struct {
+  const void *src;
+  size_t off, len;
+} iax_piece_t;
+int iax_upload(void *d_dst, const iax_piece_t *pieces, int64_t n, int nthreads);
 /* Decode the whole (base) container into a dense row-major device buffer of
  * shape (shape0, shape1) with leading dimension shape1. */
 ina_rc_t iax_decode_dense(iarray_container_t *c, void *d_dst, int scratch_slot);

@@ -1,0 +1,41 @@
+"""Containers to the device and arrays back, at the sizes where the transfers
+change: one pinned stage or several (16 MiB pieces, 512 KiB copies), small
+results in one copy, large ones piece by piece; and device blocks handed from
+freed containers to new ones.
+"""
+import numpy as np
+import pytest
+
+import pyiarray as ia
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [1, 255, 256, 257, 1023, 1024, 2047, 2048, 2049, 4100, 8192, 8193, 12300])
+def test_roundtrip_sizes(rows):
+    """Random bytes stored raw: `rows` rows of 2 KiB in chunks of 512 KiB."""
+    rng = np.random.default_rng(rows)
+    a = rng.integers(-2 ** 62, 2 ** 62, (rows, 256))
+    ctx = ia.Context(clevel=1, filters=0)
+    c = ia.Container.from_numpy(ctx, a, (min(rows, 256), 256), (min(rows, 64), 256))
+    assert np.array_equal(c.to_numpy(), a)
+
+
+def test_blocks_reused_by_other_containers():
+    """Containers freed and made in turn, each decoded while others live: a
+    reused device block never shows another container's data."""
+    rng = np.random.default_rng(5)
+    ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
+    live = []
+    for i in range(60):
+        n = int(rng.choice([40, 41, 100, 333, 700]))
+        a = rng.integers(-50, 50, (n, n)).astype(np.float64)
+        c = ia.Container.from_numpy(ctx, a, (n, n), (min(n, 64), min(n, 64)))
+        live.append((a, c))
+        if len(live) > 4:
+            live.pop(int(rng.integers(0, len(live))))
+        for a, c in live:
+            assert np.array_equal(c.to_numpy(), a)
+        a, c = live[int(rng.integers(0, len(live)))]
+        p = ia.matmul(c, c, a.shape, (min(a.shape[0], 64),) * 2)
+        assert np.array_equal(p.to_numpy(), a @ a)
