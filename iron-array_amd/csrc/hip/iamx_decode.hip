@@ -78,13 +78,12 @@ struct Lz4Geom {
   static constexpr int kStage = 4 * kStageWords;
   static constexpr int kSeqs = 22 * NW;           // a sequence takes at least 3 input bytes
   // LDS: ring, two stages, sequence table, first-output-byte bits, source
-  // records of an output step, window exits, window totals, the cut
+  // records of an output step, window exits, the cut
   static constexpr int kTabAt = kRing + 2 * kStage;
   static constexpr int kBitsAt = kTabAt + 8 * kSeqs;
   static constexpr int kRecAt = kBitsAt + kOut / 8;
   static constexpr int kExitAt = kRecAt + 4 * kThreads;
-  static constexpr int kTotAt = kExitAt + 2 * kThreads;
-  static constexpr int kCutAt = kTotAt + ((4 * NW + 7) & ~7);
+  static constexpr int kCutAt = kExitAt + 4 * kThreads;
   static constexpr int kLds = kCutAt + 8;
   static_assert(kOut >= kSeqOut, "a round holds any one sequence");
   static_assert(kStage >= 3 + 64 * NW + kSeqIn + 8, "and the stage its input");
@@ -118,14 +117,16 @@ struct Lz4Geom<1> {
 //            length byte each) inside the stream are decoded by rounds (`ok`).
 //   reach    each wavefront follows the sequences of its 64-position window
 //            from all 64 starts at once, by pointer doubling (at most 21
-//            hops): the set of starts passed, and where the chain leaves the
-//            window or stops at a sequence that is not ok.  None of this needs
-//            to know where the window is entered.
+//            hops): where the chain leaves the window or stops at a sequence
+//            that is not ok, and how many sequences and output bytes it
+//            passes.  None of this needs to know where the window is entered.
 //   chain    the windows' exits are then followed from the round's entry, one
-//            lookup per window, and each wavefront picks its set of starts.
-//   scan     prefix sums of the sequences' output lengths, over the lanes and
-//            over the windows, give every sequence's first output byte; the
-//            round is cut before the first one that does not fit.
+//            lookup per window, which gives each wavefront its first start, the
+//            sequences and the output bytes before it.
+//   walk     from there each wavefront collects its starts, eight hops a step.
+//   scan     a prefix sum of their output lengths over the lanes gives every
+//            sequence's first output byte; the round is cut before the first
+//            one that does not fit.
 //   table    the starts store their fields in LDS in sequence order and set
 //            the bit of their first output byte.
 //   output   one byte a thread, two at a time, whatever sequences they belong
@@ -377,8 +378,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       }
     } else {
       volatile uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
-      uint16_t *exits = reinterpret_cast<uint16_t *>(lds + G::kExitAt);
-      uint32_t *tot = reinterpret_cast<uint32_t *>(lds + G::kTotAt);
+      uint32_t *exits = reinterpret_cast<uint32_t *>(lds + G::kExitAt);
       unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
       int32_t base = ip, entry = 0, buf = 0;
       if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage)[tid] = ld_word(base, tid);
@@ -406,52 +406,72 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
                          (adv <= iend - base - tid)) != 0;
         const uint64_t okm = __ballot(ok);
-        // reach: 64 and more is a position of a later window; a start that is
-        // not ok leads to itself
-        int32_t to = ok ? lane + adv : lane;
-        uint32_t rlo = lane < 32 ? 1u << lane : 0u, rhi = lane < 32 ? 0u : 1u << (lane - 32);
-#pragma unroll
-        for (int t = 0; t < 5; t++) {
-          const int32_t f = bperm(to, to);
-          const uint32_t flo = (uint32_t)bperm(to, (int32_t)rlo), fhi = (uint32_t)bperm(to, (int32_t)rhi);
-          const bool in = to < 64;
-          rlo |= in ? flo : 0u;
-          rhi |= in ? fhi : 0u;
-          to = in ? f : to;
+        // reach: bits 0..8 the lane the chain from here has got to (64 and more
+        // is a position of a later window; a start that is not ok leads to
+        // itself), bits 10..23 the output bytes and bits 24..28 the sequences on
+        // the way (at most 21 of 542 bytes)
+        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 24) : (uint32_t)lane;
+        auto hop = [&]() {
+          const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
+          if ((way & 1023u) < 64) way = f + (way & ~1023u);
+        };
+        uint64_t pass = 1ull << lane;  // the starts of the next eight hops
+        auto join = [&]() {
+          const uint32_t lo = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)pass);
+          const uint32_t hi = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)(pass >> 32));
+          if ((way & 1023u) < 64) pass |= ((uint64_t)hi << 32) | lo;
+        };
+        {
+          const uint32_t to = way & 1023u;
+          if (to < 64) pass |= 1ull << to;
         }
-        exits[tid] = (uint16_t)to;
+        hop();
+        join();
+        hop();
+        join();
+        hop();
+        const uint32_t way8 = way & 1023u;
+        hop();
+        hop();
+        exits[tid] = way + 64 * wave;  // positions from base
         lds_barrier();
-        // chain
-        uint32_t ex[NW / 2];  // lane l of ex[v]: the exits of starts 2 l and 2 l + 1 of windows 2 v and 2 v + 1
+        // chain: a stop stays in its window, where no later step takes it up
+        uint32_t ex[NW];
 #pragma unroll
-        for (int v = 0; v < NW / 2; v++) ex[v] = reinterpret_cast<const uint32_t *>(exits)[64 * v + lane];
-        int32_t e = entry, mine_at = 64, stop = -1;
+        for (int v = 0; v < NW; v++) ex[v] = exits[64 * v + lane];
+        int32_t e = entry, mine_at = -1, obase = 0, kbase = 0, total = 0, nseq = 0;
 #pragma unroll
         for (int v = 0; v < NW; v++) {
-          if ((e >> 6) == v) {
-            if (v == wave) mine_at = e & 63;
-            const uint32_t two = rdlane(ex[v / 2], (e >> 1) & 63);
-            const int32_t x = (int32_t)(e & 1 ? two >> 16 : two & 0xffffu);
-            if (x < 64) stop = 64 * v + x;
-            e = x < 64 ? -1 : 64 * v + x;
-          }
+          const bool here = (e >> 6) == v;
+          const uint32_t x = here ? rdlane(ex[v], e & 63) : (uint32_t)e;
+          mine_at = v == wave && here ? e & 63 : mine_at;
+          obase = v == wave ? total : obase;
+          kbase = v == wave ? nseq : kbase;
+          total += (int32_t)(x >> 10 & 0x3fffu);
+          nseq += (int32_t)(x >> 24);
+          e = (int32_t)(x & 1023u);
         }
+        int32_t stop = e < 64 * NW ? e : -1;
         if (stop == entry) {  // the first sequence is not one for a round
           ip = base + entry;
           general = true;
           break;
         }
-        const uint64_t starts =
-            mine_at < 64 ? (((uint64_t)rdlane(rhi, mine_at) << 32) | rdlane(rlo, mine_at)) & okm : 0ull;
+        // walk
+        uint64_t starts = 0;
+        if (mine_at >= 0) {
+          int32_t l = mine_at, n;
+          for (;;) {
+            starts |= ((uint64_t)rdlane((uint32_t)(pass >> 32), l) << 32) | rdlane((uint32_t)pass, l);
+            n = (int32_t)rdlane(way8, l);
+            if (n >= 64 || n == l) break;
+            l = n;
+          }
+          starts &= okm;
+        }
         // scan
         const bool mine = ((starts >> lane) & 1ull) != 0;
-        int32_t oinc = wave_inclusive_sum(mine ? len : 0);
-        if (lane == 0) tot[wave] = rdlane((uint32_t)oinc, 63) | ((uint32_t)__builtin_popcountll(starts) << 20);
-        lds_barrier();
-        const int32_t tsum = wave_inclusive_sum(lane < NW ? (int32_t)tot[lane & (NW - 1)] : 0);
-        const uint32_t prev = wave ? rdlane((uint32_t)tsum, wave - 1) : 0u;  // of the windows before
-        int32_t total = (int32_t)(rdlane((uint32_t)tsum, NW - 1) & 0xfffffu);
-        oinc += (int32_t)(prev & 0xfffffu);
+        const int32_t oinc = obase + wave_inclusive_sum(mine ? len : 0);
         const int32_t os = oinc - len;  // this sequence's first output byte, from op
         if (mine) {
           const bool hard = (oinc > oend - op) | (hoff > op + os + lit);
@@ -459,12 +479,15 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             atomicMin(cut, ((unsigned long long)tid << 32) | ((uint32_t)os << 1) | (hard ? 1u : 0u));
           } else {
             // table: byte x of the output is a literal below `os + lit`
-            tab[bits_below(starts, (int32_t)(prev >> 20))] =
+            tab[bits_below(starts, kbase)] =
                 (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
             atomicOr(obits + (os >> 5), 1u << (os & 31));
           }
         }
         lds_barrier();
+        // output: lane q of a wavefront holds the bits of bytes 64 q .. 64 q + 63
+        // and the number of sequences that start before them
+        const uint64_t ob = reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)];
         const uint64_t c = *cut;
         const uint32_t clo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)c),
                        chi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(c >> 32));
@@ -481,9 +504,6 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         } else {
           general = stop >= 0;
         }
-        // output: lane q of a wavefront holds the bits of bytes 64 q .. 64 q + 63
-        // and the number of sequences that start before them
-        const uint64_t ob = lane < G::kOut / 64 ? reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)] : 0ull;
         const int32_t own = __builtin_popcountll(ob);
         const int32_t before = wave_inclusive_sum(own) - own;
         for (int32_t x0 = 0; x0 < total; x0 += 2 * NT) {
