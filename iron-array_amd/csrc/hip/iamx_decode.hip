@@ -140,8 +140,8 @@ struct Lz4Geom<1> {
 // What bounds it is the chain from round to round (about 6000 cycles for 4
 // windows: header reads, 5 hops of pointer doubling, the exits, the scans, the
 // table, the sources), so its time falls with the windows a round takes: a
-// 250 KB bitshuffled float32 stream takes 537 us with one wavefront, 289 with
-// 4, 235 with 8; one sequence after the other, with 64 lanes copying each,
+// 250 KB bitshuffled float32 stream takes 537 us with one wavefront, 251 with
+// 4, 185 with 8; one sequence after the other, with 64 lanes copying each,
 // took 783.  Of a launch of 6400 such streams, 0.35 ms are their literal runs
 // crossing HBM at 4.8 TB/s.
 //
@@ -406,23 +406,23 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
                          (adv <= iend - base - tid)) != 0;
         const uint64_t okm = __ballot(ok);
-        // reach: bits 0..8 the lane the chain from here has got to (64 and more
+        // reach: bits 0..10 the lane the chain from here has got to (64 and more
         // is a position of a later window; a start that is not ok leads to
-        // itself), bits 10..23 the output bytes and bits 24..28 the sequences on
+        // itself), bits 11..24 the output bytes and bits 25..29 the sequences on
         // the way (at most 21 of 542 bytes)
-        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 24) : (uint32_t)lane;
+        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 11) | (1u << 25) : (uint32_t)lane;
         auto hop = [&]() {
           const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
-          if ((way & 1023u) < 64) way = f + (way & ~1023u);
+          if ((way & 2047u) < 64) way = f + (way & ~2047u);
         };
         uint64_t pass = 1ull << lane;  // the starts of the next eight hops
         auto join = [&]() {
           const uint32_t lo = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)pass);
           const uint32_t hi = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)(pass >> 32));
-          if ((way & 1023u) < 64) pass |= ((uint64_t)hi << 32) | lo;
+          if ((way & 2047u) < 64) pass |= ((uint64_t)hi << 32) | lo;
         };
         {
-          const uint32_t to = way & 1023u;
+          const uint32_t to = way & 2047u;
           if (to < 64) pass |= 1ull << to;
         }
         hop();
@@ -430,7 +430,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         hop();
         join();
         hop();
-        const uint32_t way8 = way & 1023u;
+        const uint32_t way8 = way & 2047u;
         hop();
         hop();
         exits[tid] = way + 64 * wave;  // positions from base
@@ -447,9 +447,9 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           mine_at = v == wave && here ? e & 63 : mine_at;
           obase = v == wave ? total : obase;
           kbase = v == wave ? nseq : kbase;
-          total += (int32_t)(x >> 10 & 0x3fffu);
-          nseq += (int32_t)(x >> 24);
-          e = (int32_t)(x & 1023u);
+          total += (int32_t)(x >> 11 & 0x3fffu);
+          nseq += (int32_t)(x >> 25);
+          e = (int32_t)(x & 2047u);
         }
         int32_t stop = e < 64 * NW ? e : -1;
         if (stop == entry) {  // the first sequence is not one for a round
@@ -1040,16 +1040,16 @@ namespace iamx {
 // Wavefronts per stream, by how many streams a CU gets.  A stream's time is set
 // by its own chain of rounds, so few streams are spread over many wavefronts
 // each; many streams hide each other's waits, and one wavefront decodes a
-// sequence with the fewest instructions.  The lines are where the launch still
-// holds every stream at once (2 x 8 and 8 x 4 wavefronts per CU).  Measured in
-// us with 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250 KB:
-// 4 streams 235 / 289 / 537, 512 streams 330 / 395 / 690, 1024 streams
-// 650 / 484 / 775, 2048 streams 1220 / 741 / 857, 4096 streams
-// - / 1318 / 1050, 6400 streams - / 1884 / 1424; exponent planes of float32
-// (64 KB): 1024 streams 805 / 696 / 1156, 6400 streams - / 3019 / 1950.
+// sequence with the fewest instructions.  The lines are where a CU still holds
+// all of its streams at once (4 x 8 and 8 x 4 wavefronts).  Measured in us with
+// 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250 KB: 4 streams
+// 185 / 251 / 537, 1024 streams 416 / 437 / 775, 2048 streams 800 / 664 / 857,
+// 4096 streams - / 1318 / 1006, 6400 streams - / 1884 / 1358; exponent planes of
+// float32 (64 KB): 4 streams 325 / 474 / 1005, 1024 streams 644 / 693 / 1156,
+// 6400 streams - / 3019 / 1966.
 int launch_lz4(const char *name, const iamx_lz4_job_t *d_lz4, int n_lz4, void *d_scratch, int64_t cap) {
   const int z = zstd_enabled() ? 1 : 0;
-  if (n_lz4 <= 2 * g_num_cus)
+  if (n_lz4 <= 4 * g_num_cus)
     IAMX_LAUNCH(name, k_lz4_streams<8>, dim3(n_lz4), dim3(512), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
                 status_word(), z);
   else if (n_lz4 <= 8 * g_num_cus)

@@ -353,7 +353,7 @@ ROUND_PLANS = {
 
 
 # the decoder gives a stream 8, 4 or 1 wavefronts by the number of streams of the launch
-@pytest.mark.parametrize("copies", [3, 700, 2100])
+@pytest.mark.parametrize("copies", [3, 1100, 2100])
 @pytest.mark.parametrize("plan", sorted(ROUND_PLANS))
 def test_crafted_lz4_rounds(ctx, orc, plan, copies):
     print(f"case: crafted lz4 rounds {plan} x {copies}", flush=True)
@@ -373,7 +373,7 @@ def test_crafted_lz4_rounds(ctx, orc, plan, copies):
         at += len(want[i % 3])
 
 
-@pytest.mark.parametrize("copies", [3, 700, 2100])
+@pytest.mark.parametrize("copies", [3, 1100, 2100])
 def test_corrupt_stream_among_many(ctx, orc, copies):
     rng = np.random.default_rng(copies)
     c = ia.Context(clevel=5, filters=0)
