@@ -242,8 +242,10 @@ __global__ __launch_bounds__(256) void k_ozaki_level(const int32_t *__restrict__
 
 // ---- Ozaki CRT prep and combine ------------------------------------------------------------
 constexpr int kMaxMods = 15;   // W_l < M < 2^118 fits 6 limbs of 20 bits; p, q <= 52
-constexpr int kLimbs = 7;      // S = sum r_l W_l < 2^130 needs 7
+constexpr int kLimbs = 6;      // of W_l; their sums of up to 15 products stay below 2^32
 constexpr uint32_t kLimbMask = (1u << 20) - 1;
+
+typedef double double2_any __attribute__((ext_vector_type(2), aligned(8)));
 
 struct CrtMods {
   int32_t n;
@@ -253,10 +255,16 @@ struct CrtMods {
 
 // n residue planes, each rows_p x cols_p int8: the integer rint(X 2^(scale -
 // e[r])) reduced to the symmetric range of m_l ([-128, 127] for 256,
-// [-(m-1)/2, (m-1)/2] for odd m).  trans as in k_slice_i8 (B's planes are
-// stored transposed); e[r] is the exponent of plane row r (ilogb(max) + 2, or
-// 0 for an all-zero line).  The scaled integer has at most 52 bits, so
-// a - m rint(a/m) is exact (the quotient may be off by one; one correction).
+// [-(m-1)/2, (m-1)/2] for odd m, or one past either end).  trans as in
+// k_slice_i8 (B's planes are stored transposed); e[r] is the exponent of plane
+// row r (ilogb(max) + 2, or 0 for an all-zero line).  The scaled integer has at
+// most 52 bits, so a - m rint(a/m) is exact, and as the quotient is off by at
+// most one next to a half its magnitude is at most 128: only +128 needs
+// bringing back into an int8 (any residue of the class gives the exact product
+// modulo m, and 131071 products of 128^2 stay below 2^31).  6000x6000 operands
+// with 13 moduli read 0.29 GB and write 0.47 in 167 (A) and 260 us (B, through
+// the LDS tile); both ends brought back in FP64 took 229 and 281.  A tile kept
+// column by column in LDS measured the same (264).
 __global__ __launch_bounds__(256) void k_residues_i8(const double *__restrict__ X, int64_t xr, int64_t xc,
                                                      int64_t ldx, int trans, const int32_t *__restrict__ e, int scale,
                                                      const CrtMods mods, int8_t *__restrict__ planes, int64_t rows_p,
@@ -281,21 +289,28 @@ __global__ __launch_bounds__(256) void k_residues_i8(const double *__restrict__ 
     if (r >= rows_p || c >= cols_p) continue;
     const int er = r < (trans ? xc : xr) ? e[r] : 0;
     double a[4];
+    if (!trans && r < xr && c + 4 <= xc) {  // inside: two 16-byte loads
+      const double2_any *x = reinterpret_cast<const double2_any *>(X + r * ldx + c);
+      const double2_any x0 = x[0], x1 = x[1];
+      a[0] = x0.x;
+      a[1] = x0.y;
+      a[2] = x1.x;
+      a[3] = x1.y;
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const double v = trans ? t[4 * tx + k][i] : ((r < xr && c + k < xc) ? X[r * ldx + c + k] : 0.0);
-      a[k] = rint(ldexp(v, scale - er));
+      for (int k = 0; k < 4; k++)
+        a[k] = trans ? t[4 * tx + k][i] : ((r < xr && c + k < xc) ? X[r * ldx + c + k] : 0.0);
     }
+#pragma unroll
+    for (int k = 0; k < 4; k++) a[k] = rint(ldexp(a[k], scale - er));
     for (int l = 0; l < mods.n; l++) {
       const double m = (double)mods.m[l];
-      const double hi = (double)((mods.m[l] - 1) / 2), lo = -(double)(mods.m[l] / 2);
       uint32_t word = 0;
 #pragma unroll
       for (int k = 0; k < 4; k++) {
-        double res = fma(-m, rint(a[k] * mods.inv[l]), a[k]);
-        res -= res > hi ? m : 0.0;
-        res += res < lo ? m : 0.0;
-        word |= (uint32_t)(uint8_t)(int8_t)(int)res << (8 * k);
+        int32_t res = (int32_t)fma(-m, rint(a[k] * mods.inv[l]), a[k]);
+        res -= res > 127 ? mods.m[l] : 0;
+        word |= (uint32_t)(uint8_t)res << (8 * k);
       }
       *reinterpret_cast<uint32_t *>(planes + (int64_t)l * plane + r * cols_p + c) = word;
     }
@@ -305,35 +320,34 @@ __global__ __launch_bounds__(256) void k_residues_i8(const double *__restrict__ 
 struct CrtCombine {
   int32_t n;
   int32_t m[kMaxMods];               // the moduli
-  double minv[kMaxMods];             // 1 / m_l, rounded
-  uint32_t w[kMaxMods][kLimbs - 1];  // W_l in 20-bit limbs, least significant first
-  uint32_t mlimb[kLimbs];            // M
-  uint32_t half[kLimbs];             // ceil(M / 2)
+  int32_t c16[kMaxMods];             // 2^16 mod m_l, in [-m/2, m/2]
+  float minv[kMaxMods];              // 1 / m_l, rounded
+  uint32_t w[kMaxMods][kLimbs];      // W_l in 20-bit limbs, least significant first
+  uint32_t mword[4];                 // M in 32-bit words, least significant first
   double inv_m;                      // 1 / M, rounded
   int32_t p1, q1;                    // p + 1, q + 1
 };
 
-// r >= s over kLimbs limbs (most significant last)
-__device__ __forceinline__ bool limbs_ge(const uint32_t *r, const uint32_t *s) {
-#pragma unroll
-  for (int k = kLimbs - 1; k >= 0; k--)
-    if (r[k] != s[k]) return r[k] > s[k];
-  return true;
-}
+// C[i][j] = 2^(e_i + f_j - p - q - 2) * C', C' the representative nearest zero
+// of sum_l r_l W_l (mod M), r_l the residue of plane l.  Everything up to the
+// conversion to FP64 is exact integer arithmetic: |C'| is below M/2 by at least
+// a factor of 1 - 2^-31, so the nearest integer to the FP64 quotient
+// sum / M (relative error below 2^-49, at most 15 * 256) is the right one and
+// C' = sum - q M fits 118 bits.
+//
+// Four columns a thread, so that a load is 16 bytes of one plane (4 of the byte
+// planes).  Bound by reading the residues: 6000x6000 with 13 INT32 planes is
+// 1.87 GB read and 0.29 written.  With one column a thread, FP64 quotients and
+// 64-bit limb arithmetic with a correction each way it took 803 us; now 430.
 
-// C[i][j] = 2^(e_i + f_j - p - q - 2) * C', C' the representative in
-// [-M/2, M/2) of sum_l r_l W_l (mod M), r_l the residue byte of plane l.
-// Everything up to the conversion to FP64 is exact integer arithmetic.
-// r_l: a residue byte in [0, m_l), or an exact INT32 product sum reduced
-// here: the quotient from the FP64 product with 1/m (exact v, so off by at
-// most one) and one correction each way
-__device__ __forceinline__ uint32_t residue(uint8_t v, int32_t, double) { return v; }
-__device__ __forceinline__ uint32_t residue(int32_t v, int32_t m, double minv) {
-  // (wrapping unsigned arithmetic: the true difference lies in [-m, 2m))
-  int32_t r = (int32_t)((uint32_t)v - (uint32_t)(int32_t)floor((double)v * minv) * (uint32_t)m);
-  r += r < 0 ? m : 0;
-  r -= r >= m ? m : 0;
-  return (uint32_t)r;
+// r_l: a residue byte in [0, m_l), or an exact INT32 product sum reduced here:
+// with v = 65536 h + l, h c16 + l is congruent and below 2^23, exact in FP32;
+// the nearest quotient leaves at most about m/2 either side of zero
+__device__ __forceinline__ uint32_t residue(uint8_t v, int32_t, int32_t, float) { return v; }
+__device__ __forceinline__ uint32_t residue(int32_t v, int32_t m, int32_t c16, float minv) {
+  const int32_t s = __mul24(v >> 16, c16) + (v & 0xffff);
+  const int32_t r = s - __mul24((int32_t)rintf((float)s * minv), m);
+  return (uint32_t)(r + ((r >> 31) & m));
 }
 
 template <typename RT>
@@ -341,63 +355,55 @@ __global__ __launch_bounds__(256) void k_crt_combine(const RT *__restrict__ R, i
                                                      int64_t rows, int64_t cols, const int32_t *__restrict__ ea,
                                                      const int32_t *__restrict__ fb, const CrtCombine P,
                                                      double *__restrict__ C, int64_t ldc) {
-  const int64_t i = blockIdx.y, j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  typedef RT RT4 __attribute__((ext_vector_type(4)));
+  // planes have whole groups of four columns (ldr a multiple of 256)
+  const int64_t i = blockIdx.y, j = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
   if (i >= rows || j >= cols) return;
-  uint32_t acc[kLimbs] = {0, 0, 0, 0, 0, 0, 0};
+  uint32_t acc[4][kLimbs] = {};
   const RT *rp = R + i * ldr + j;
+#pragma unroll 4
   for (int l = 0; l < P.n; l++) {
-    const uint32_t r = residue(rp[(int64_t)l * plane], P.m[l], P.minv[l]);
+    const RT4 v = *reinterpret_cast<const RT4 *>(rp + (int64_t)l * plane);
 #pragma unroll
-    for (int k = 0; k < kLimbs - 1; k++) acc[k] += __umul24(r, P.w[l][k]);  // < 15 * 255 * 2^20 < 2^32
-  }
+    for (int c = 0; c < 4; c++) {
+      const uint32_t r = residue((RT)v[c], P.m[l], P.c16[l], P.minv[l]);
 #pragma unroll
-  for (int k = 0; k < kLimbs - 1; k++) {
-    acc[k + 1] += acc[k] >> 20;
-    acc[k] &= kLimbMask;
-  }
-  // q = floor(S / M) from the top limbs (may be one off), then S - q M exactly
-  const double sd = ldexp((double)acc[6], 120) + ldexp((double)acc[5], 100) + ldexp((double)acc[4], 80) +
-                    ldexp((double)acc[3], 60);
-  const int64_t q = (int64_t)floor(sd * P.inv_m);
-  int64_t carry = 0;
-#pragma unroll
-  for (int k = 0; k < kLimbs; k++) {
-    const int64_t t = (int64_t)acc[k] - q * (int64_t)P.mlimb[k] + carry;
-    acc[k] = (uint32_t)(t & kLimbMask);
-    carry = t >> 20;  // arithmetic shift: floor division
-  }
-  if (carry < 0) {  // q one too large: add M back
-    carry = 0;
-#pragma unroll
-    for (int k = 0; k < kLimbs; k++) {
-      const int64_t t = (int64_t)acc[k] + P.mlimb[k] + carry;
-      acc[k] = (uint32_t)(t & kLimbMask);
-      carry = t >> 20;
-    }
-  } else if (limbs_ge(acc, P.mlimb)) {  // q one too small
-    int64_t b = 0;
-#pragma unroll
-    for (int k = 0; k < kLimbs; k++) {
-      const int64_t t = (int64_t)acc[k] - P.mlimb[k] + b;
-      acc[k] = (uint32_t)(t & kLimbMask);
-      b = t >> 20;
+      for (int k = 0; k < kLimbs; k++) acc[c][k] += __umul24(r, P.w[l][k]);  // < 15 * 255 * 2^20 < 2^32
     }
   }
-  // representative in [-M/2, M/2)
-  const bool neg = limbs_ge(acc, P.half);
-  if (neg) {
-    int64_t b = 0;
+  double out[4];
 #pragma unroll
-    for (int k = 0; k < kLimbs; k++) {
-      const int64_t t = (int64_t)P.mlimb[k] - acc[k] + b;
-      acc[k] = (uint32_t)(t & kLimbMask);
-      b = t >> 20;
+  for (int c = 0; c < 4; c++) {
+    const uint32_t *x = acc[c];
+    double sd = (double)x[kLimbs - 1];
+#pragma unroll
+    for (int k = kLimbs - 2; k >= 0; k--) sd = fma(sd, 1048576.0, (double)x[k]);
+    const uint32_t q = (uint32_t)rint(sd * P.inv_m);  // at most 15 * 256
+    // the sum and q M modulo 2^128
+    const uint64_t t0 = (uint64_t)x[0] + ((uint64_t)x[1] << 20), t1 = (uint64_t)x[2] << 40, t2 = (uint64_t)x[3] << 60;
+    const uint64_t s0 = t0 + t1, lo = s0 + t2;
+    const uint64_t hi = (uint64_t)(x[2] >> 24) + (x[3] >> 4) + ((uint64_t)x[4] << 16) + ((uint64_t)x[5] << 36) +
+                        (s0 < t1 ? 1 : 0) + (lo < t2 ? 1 : 0);
+    const uint64_t p0 = (uint64_t)q * P.mword[0], p1 = (uint64_t)q * P.mword[1] + (p0 >> 32),
+                   p2 = (uint64_t)q * P.mword[2] + (p1 >> 32), p3 = (uint64_t)q * P.mword[3] + (p2 >> 32);
+    const uint64_t qlo = (p1 << 32) | (uint32_t)p0, qhi = (p3 << 32) | (uint32_t)p2;
+    uint64_t dlo = lo - qlo, dhi = hi - qhi - (lo < qlo ? 1 : 0);
+    const bool neg = (int64_t)dhi < 0;
+    if (neg) {
+      dlo = 0 - dlo;
+      dhi = ~dhi + (dlo == 0 ? 1 : 0);
     }
+    const double v = fma((double)dhi, 18446744073709551616.0, (double)dlo);
+    out[c] = ldexp(neg ? -v : v, ea[i] + (j + c < cols ? fb[j + c] : 0) - P.p1 - P.q1);
   }
-  double v = (double)acc[kLimbs - 1];
-#pragma unroll
-  for (int k = kLimbs - 2; k >= 0; k--) v = fma(v, 1048576.0, (double)acc[k]);
-  C[i * ldc + j] = ldexp(neg ? -v : v, ea[i] + fb[j] - P.p1 - P.q1);
+  double *o = C + i * ldc + j;
+  if (j + 4 <= cols) {
+    double2_any *d = reinterpret_cast<double2_any *>(o);
+    d[0] = double2_any{out[0], out[1]};
+    d[1] = double2_any{out[2], out[3]};
+  } else {
+    for (int c = 0; j + c < cols; c++) o[c] = out[c];
+  }
 }
 
 // ---- the segmented GEMM -----------------------------------------------------------------
@@ -1011,14 +1017,15 @@ static CrtCombine crt_combine_consts(int n, int p, int q) {
     const unsigned r = (unsigned)(Ml % m);
     unsigned inv = 1;
     while ((r * inv) % m != 1) inv++;  // m <= 256: a direct search
-    to_limbs((Ml * inv) % M, c.w[l], kLimbs - 1);
+    to_limbs((Ml * inv) % M, c.w[l], kLimbs);
   }
-  to_limbs(M, c.mlimb, kLimbs);
-  to_limbs(M / 2, c.half, kLimbs);
+  for (int k = 0; k < 4; k++) c.mword[k] = (uint32_t)(M >> (32 * k));
   c.inv_m = 1.0 / (double)M;
   for (int l = 0; l < n; l++) {
-    c.m[l] = kMods[l];
-    c.minv[l] = 1.0 / (double)kMods[l];
+    const int m = kMods[l], r = 65536 % m;
+    c.m[l] = m;
+    c.c16[l] = r > m / 2 ? r - m : r;
+    c.minv[l] = 1.0f / (float)m;
   }
   c.p1 = p + 1;
   c.q1 = q + 1;
@@ -1166,7 +1173,7 @@ static int mixed_rows(const PrepB &pb, int form, int64_t M, const void *A, int64
     P.ldc = Np;
     P.tiles_n = (int)(Np / BN);
     const CrtCombine comb = crt_combine_consts(n, pb.p, pb.q);
-    const dim3 cgrid((unsigned)((N + 255) / 256), (unsigned)M);
+    const dim3 cgrid((unsigned)((N + 1023) / 1024), (unsigned)M);
     // both candidates give the exact residues, so the same bits
     tuned(2, M, N, K * n, {256, kLib},
           [&](int tile) -> int {

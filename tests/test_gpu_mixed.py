@@ -210,6 +210,23 @@ def test_ozaki_crt_exact_on_integers_and_signs(orc):
     assert np.array_equal(c, want)
 
 
+@pytest.mark.parametrize("moduli", [9, 13, 15])
+@pytest.mark.parametrize("N", [1, 3, 4, 5, 257, 1023, 1026])
+def test_ozaki_crt_column_edges(N, moduli, monkeypatch):
+    """The combine takes four columns a thread and 1024 a workgroup: exact
+    integer products around both, from INT32 sums and from residue bytes."""
+    ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
+    rng = np.random.default_rng(N)
+    a = rng.integers(-500, 501, (37, 131)).astype(np.float64)
+    b = rng.integers(-500, 501, (131, N)).astype(np.float64)
+    ca = ia.Container.from_numpy(ctx, a, (37, 131), (19, 33))
+    cb = ia.Container.from_numpy(ctx, b, (131, N), (33, min(N, 50)))
+    for tile in ("lib", "256"):
+        monkeypatch.setenv("IAMX_TILE", tile)
+        c = ia.matmul(ca, cb, (37, N), (19, min(N, 50)), precision=ia.OZAKI_CRT, slices=moduli).to_numpy()
+        assert np.array_equal(c, a @ b), tile
+
+
 def test_ozaki_exact_on_small_integers(orc):
     """Integers below 2^7 are one slice: every form must be exact."""
     ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
