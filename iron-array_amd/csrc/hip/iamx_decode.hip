@@ -29,8 +29,21 @@ __device__ __forceinline__ uint32_t rdlane(uint32_t v, int32_t l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
 }
 
-__device__ __forceinline__ uint32_t lds_u32(const uint8_t *p) {  // any alignment
-  return *reinterpret_cast<const u32_any *>(p);
+// lane l of v
+__device__ __forceinline__ void set_lane(uint32_t &v, int l, uint32_t x) {
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "n"(l));
+}
+
+// bit i of m
+__device__ __forceinline__ void bit_on(uint64_t &m, int32_t i) { asm("s_bitset1_b64 %0, %1" : "+s"(m) : "s"(i)); }
+__device__ __forceinline__ void bit_off(uint64_t &m, int32_t i) { asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(i)); }
+
+__device__ __forceinline__ uint64_t ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+
+// 4 bytes at any offset, by two aligned reads
+__device__ __forceinline__ uint32_t lds_u32(const uint8_t *lds, int32_t at) {
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(lds + (at & ~3));
+  return __builtin_amdgcn_alignbyte(w[1], w[0], (uint32_t)at);
 }
 
 __device__ __forceinline__ int32_t bperm(int32_t l, int32_t v) {  // v of lane l & 63
@@ -137,12 +150,23 @@ struct Lz4Geom<1> {
 //            source written in the same step is a lower byte: the threads
 //            leave their byte, or the number of their source byte, in LDS and
 //            follow the numbers until they find a byte.
-// What bounds it is the chain from round to round (about 6000 cycles for 4
-// windows: header reads, 5 hops of pointer doubling, the exits, the scans, the
-// table, the sources), so its time falls with the windows a round takes: a
-// 250 KB bitshuffled float32 stream takes 537 us with one wavefront, 251 with
-// 4, 185 with 8; one sequence after the other, with 64 lanes copying each,
-// took 783.  Of a launch of 6400 such streams, 0.35 ms are their literal runs
+// What bounds it where streams are few is the chain from round to round (about
+// 5200 cycles for 8 windows: header reads, 5 hops of pointer doubling, the
+// exits, the scans, the table, the sources), so its time falls with the windows
+// a round takes: a 250 KB bitshuffled float32 stream takes 443 us with one
+// wavefront, 205 with 4, 136 with 8; one sequence after the other, with 64
+// lanes copying each, took 783.  With four streams a CU it is vector issue (78%
+// of the cycles).  So a round's cost is its instructions and its waits:
+//  - LDS words at any byte offset are two aligned reads and a byte align; one
+//    misaligned read a lane took 522 us where this takes 424 (1024 exponent
+//    planes of 64 KB of float32).
+//  - The records are read and written as LDS; through a volatile pointer they
+//    were flat accesses that waited for every global load and store in flight
+//    (561 against 531 us), as a byte from the slot did where its path met the
+//    others', and a flush before the staged input had arrived.
+//  - The chain has no branch and selects nothing: what a window's wavefront
+//    needs is left in the lane of its number (645 to 561 us).
+// Of a launch of 6400 bitshuffled streams, 0.35 ms are their literal runs
 // crossing HBM at 4.8 TB/s.
 //
 // What a round cannot hold (long literal runs, matches of more than 273
@@ -228,9 +252,9 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         put_stage(have - 256, c);
       }
       for (;;) {
-        // no window of a round starts more than 320 bytes from ip, and its last
+        // no window of a round starts 189 bytes from ip or more, and its last
         // sequence starts within 62
-        while (have < ip + 320 + 62 + kSeqIn + 8) {
+        while (have < ip + 3 * WIN + 62 + kSeqIn + 8) {
           put_stage(have, ld_word(have, lane));
           have += 256;
         }
@@ -241,9 +265,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         // walk: the starts of up to three windows, listed by position
         int32_t n = 0, at = ip;  // sequences so far, the next one's position
         bool stopped = false;
-#pragma unroll 1
-        for (int w = 0; w < 3; w++) {
-          const uint32_t h = lds_u32(stage + ((at + lane) & SM));
+        do {
+          const uint32_t h = lds_u32(stage, (at + lane) & SM);
           const uint32_t hl = (h >> 4) & 15u, lb = (h >> 8) & 255u;
           const int32_t adv = 3 + (int32_t)hl + (hl == 15 ? (int32_t)lb + 1 : 0) + ((h & 15u) == 15 ? 1 : 0);
           const bool ok = (!((hl == 15) & (lb == 255)) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
@@ -253,19 +276,19 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           int32_t l = 0, t1;
           do {
             t1 = (int32_t)rdlane((uint32_t)to, l);
-            starts |= (1ull << l) | (1ull << t1);
+            bit_on(starts, l);
+            bit_on(starts, t1);
             l = (int32_t)rdlane((uint32_t)to2, l);
           } while (l != t1);
+          bit_off(starts, l);  // where it ends is no start: a stop, or past the window
           stopped = l < WIN;
-          starts &= __ballot(ok);
           if (starts == 0) break;
           const int32_t k = bits_below(starts, n);
-          if (((starts >> lane) & 1ull) && k < G::kSeqs) list[k] = (uint16_t)(at - ip + lane);
+          if ((starts >> lane) & 1ull) list[k] = (uint16_t)(at - ip + lane);
           n += __builtin_popcountll(starts);
           const int32_t last = 63 - __builtin_clzll(starts);
           at += last + (int32_t)rdlane((uint32_t)adv, last);
-          if (stopped || n >= G::kSeqs || at - ip > 320) break;
-        }
+        } while (!stopped && at - ip < 3 * WIN);  // a window leads past its 63 positions
         if (n == 0) {
           general = true;
           break;
@@ -273,12 +296,12 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         __builtin_amdgcn_wave_barrier();
         // lane k takes sequence k
         const int32_t pos = ip + (int32_t)list[lane];
-        const uint32_t h = lds_u32(stage + (pos & SM));
+        const uint32_t h = lds_u32(stage, pos & SM);
         const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
         const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
         const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
         const int32_t src = pos + 1 + (int32_t)lext;  // first literal
-        const uint32_t h2 = lds_u32(stage + ((src + lit) & SM));
+        const uint32_t h2 = lds_u32(stage, (src + lit) & SM);
         const int32_t hoff = (int32_t)(h2 & 0xffffu);
         const uint32_t he = (h2 >> 16) & 255u;
         const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
@@ -288,9 +311,9 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         const int32_t os = oinc - len;  // this sequence's first output byte, from op
         // the first sequence that does not fit, or ends in a second length byte
         const bool hard = (((ext != 0) & (he == 255)) | (hoff < 1) | (hoff > op + os + lit) | (oinc > oend - op)) != 0;
-        const uint64_t cutm = __ballot(mine & (hard | (oinc > G::kOut)));
-        const uint64_t hardm = __ballot(hard);
-        int32_t nseq = min(n, G::kSeqs);
+        const uint64_t cutm = ballot(mine & (hard | (oinc > G::kOut)));
+        const uint64_t hardm = ballot(hard);
+        int32_t nseq = n;
         if (cutm) {
           nseq = __builtin_ctzll(cutm);
           stopped = ((hardm >> nseq) & 1ull) != 0;
@@ -299,22 +322,20 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             general = true;
             break;
           }
-        } else if (n > G::kSeqs) {
-          stopped = false;
-          at = (int32_t)rdlane((uint32_t)(src + lit), 63) + 2 + (int32_t)rdlane(ext, 63);
         }
         const int32_t total = (int32_t)rdlane((uint32_t)oinc, nseq - 1);
         if (lane < nseq) {
           // byte x of the output is a literal below `os + lit`
           tab[lane] = (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
-          atomicOr(obits + (os >> 5), 1u << (os & 31));
+          const int32_t ob = (os - 1) & (G::kOut - 1);
+          atomicOr(obits + (ob >> 5), 1u << (ob & 31));
         }
         __builtin_amdgcn_wave_barrier();
         const uint64_t ob = lane < G::kOut / 64 ? reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)] : 0ull;
-        int32_t before = -1;  // sequences that start in earlier steps, less one
+        int32_t before = 0;  // sequences that start in earlier steps, or with this one, less one
         auto entry_of = [&](int32_t x0) -> uint64_t {
           const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), x0 >> 6) << 32) | rdlane((uint32_t)ob, x0 >> 6);
-          const int32_t k = bits_below(m >> 1, before + (int32_t)(m & 1));  // the last start at or before its byte
+          const int32_t k = bits_below(m, before);  // the last start at or before its byte
           before += __builtin_popcountll(m);
           return tab[k];
         };
@@ -330,29 +351,30 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           const bool odd = (im >= 0) & (x < total) & ((off > NEAR1) | (off <= max(im, lane)));
           const int32_t x1 = x0 + 64;
           uint32_t v;
-          if (__ballot(odd)) {
-            if (__ballot(odd & (im >= off))) {
+          if (ballot(odd)) {
+            if (odd & (im >= off)) {
               // (im + 1/2) / off is at least 1/546 away from a whole number
               const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
-              if (im >= off) off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
-              sp = op + x - off;
+              off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
             }
+            sp = op + x - off;
             v = lds[im < 0 ? lat : sp & RM];
             if (x1 < total) e = entry_of(x1);
-            const bool far = odd & (off > NEAR1);
-            // at most FLUSH_AT + 64 bytes are pending, so a far source was
+            // at most FLUSH_AT + kOut bytes are pending, so a far source was
             // flushed, by this wavefront's own stores
-            if (far) v = dst[sp];
+            if (odd & (off > NEAR1)) {
+              v = dst[sp];
+              asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
+            }
             const bool dep = odd & (off <= lane);
-            if (__ballot(dep)) {
+            if (ballot(dep)) {
               // bit 6: the lane has its own byte
               int32_t code = dep ? lane - off : lane | 64;
               do {
                 code = bperm(code, code);
-              } while (__ballot(code < 64));
+              } while (ballot(code < 64));
               v = (uint32_t)bperm(code, (int32_t)v);
             }
-            asm volatile("" : "+v"(v));  // a far byte has arrived
           } else {
             v = lds[im < 0 ? lat : sp & RM];
             if (x1 < total) e = entry_of(x1);
@@ -360,24 +382,24 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           __builtin_amdgcn_wave_barrier();
           ring[(op + x) & RM] = (uint8_t)v;
           __builtin_amdgcn_wave_barrier();
-          const int32_t cur = op + min(total, x1);
-          if (cur >= flush_at) flush(cur);
           if (x1 >= total) break;
           x0 = x1;
         }
         op += total;
         ip = at;
-        if (stopped) {
-          general = true;
-          break;
-        }
+        asm volatile("" : "+v"(ahead));  // arrived; what follows is stored without a wait
         if (more) {
           put_stage(have, ahead);
           have += 256;
         }
+        if (op >= flush_at) flush(op);
+        if (stopped) {
+          general = true;
+          break;
+        }
       }
     } else {
-      volatile uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
+      uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
       uint32_t *exits = reinterpret_cast<uint32_t *>(lds + G::kExitAt);
       unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
       int32_t base = ip, entry = 0, buf = 0;
@@ -390,13 +412,13 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         if (tid < G::kOut / 32) obits[tid] = 0;
         if (tid == 0) *cut = ~0ull;
         // headers
-        const uint8_t *st = stage + buf * G::kStage + (base & 3);
-        const uint32_t h = lds_u32(st + tid);
+        const int32_t st = RING + buf * G::kStage + (base & 3);
+        const uint32_t h = lds_u32(lds, st + tid);
         const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
         const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
         const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
         const int32_t src = tid + 1 + (int32_t)lext;  // first literal, from base
-        const uint32_t h2 = lds_u32(st + min(src + lit, G::kStage - 8));
+        const uint32_t h2 = lds_u32(lds, st + min(src + lit, G::kStage - 8));
         const int32_t hoff = (int32_t)(h2 & 0xffffu);
         const uint32_t he = (h2 >> 16) & 255u;
         const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
@@ -405,24 +427,24 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         // (bitwise: one vector compare chain, no branches)
         const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
                          (adv <= iend - base - tid)) != 0;
-        const uint64_t okm = __ballot(ok);
-        // reach: bits 0..10 the lane the chain from here has got to (64 and more
+        const uint64_t okm = ballot(ok);
+        // reach: bits 0..9 the lane the chain from here has got to (64 and more
         // is a position of a later window; a start that is not ok leads to
-        // itself), bits 11..24 the output bytes and bits 25..29 the sequences on
+        // itself), bits 10..26 the output bytes and bits 27..31 the sequences on
         // the way (at most 21 of 542 bytes)
-        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 11) | (1u << 25) : (uint32_t)lane;
+        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 27) : (uint32_t)lane;
         auto hop = [&]() {
           const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
-          if ((way & 2047u) < 64) way = f + (way & ~2047u);
+          if ((way & 1023u) < 64) way = f + (way & ~1023u);
         };
         uint64_t pass = 1ull << lane;  // the starts of the next eight hops
         auto join = [&]() {
           const uint32_t lo = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)pass);
           const uint32_t hi = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)(pass >> 32));
-          if ((way & 2047u) < 64) pass |= ((uint64_t)hi << 32) | lo;
+          if ((way & 1023u) < 64) pass |= ((uint64_t)hi << 32) | lo;
         };
         {
-          const uint32_t to = way & 2047u;
+          const uint32_t to = way & 1023u;
           if (to < 64) pass |= 1ull << to;
         }
         hop();
@@ -430,28 +452,35 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         hop();
         join();
         hop();
-        const uint32_t way8 = way & 2047u;
+        const uint32_t to8 = way & 1023u;
+        const uint32_t way8 = to8 == (uint32_t)lane ? 64u : to8;  // below 64: go on from there
         hop();
         hop();
         exits[tid] = way + 64 * wave;  // positions from base
         lds_barrier();
-        // chain: a stop stays in its window, where no later step takes it up
+        // chain: a stop stays in its window, where no later step takes it up.
+        // Lane v of `at` and `past` is where window v is entered, and the bytes
+        // (17 bits) and sequences before it.
         uint32_t ex[NW];
 #pragma unroll
         for (int v = 0; v < NW; v++) ex[v] = exits[64 * v + lane];
-        int32_t e = entry, mine_at = -1, obase = 0, kbase = 0, total = 0, nseq = 0;
+        uint32_t e = (uint32_t)entry, sum = 0;
+        uint32_t at = 0, past = 0;
 #pragma unroll
         for (int v = 0; v < NW; v++) {
-          const bool here = (e >> 6) == v;
-          const uint32_t x = here ? rdlane(ex[v], e & 63) : (uint32_t)e;
-          mine_at = v == wave && here ? e & 63 : mine_at;
-          obase = v == wave ? total : obase;
-          kbase = v == wave ? nseq : kbase;
-          total += (int32_t)(x >> 11 & 0x3fffu);
-          nseq += (int32_t)(x >> 25);
-          e = (int32_t)(x & 2047u);
+          const uint32_t x = rdlane(ex[v], (int32_t)(e & 63u));
+          set_lane(at, v, e);
+          set_lane(past, v, sum);
+          const uint32_t y = (e >> 6) == (uint32_t)v ? x : e;
+          sum += y >> 10;
+          e = y & 1023u;
         }
-        int32_t stop = e < 64 * NW ? e : -1;
+        asm("s_nop 1" : "+v"(at), "+v"(past));  // before lanes written in asm are read
+        const int32_t mine_at = (int32_t)rdlane(at, wave);
+        const uint32_t before_me = rdlane(past, wave);
+        const int32_t obase = (int32_t)(before_me & 0x1ffffu), kbase = (int32_t)(before_me >> 17);
+        int32_t total = (int32_t)(sum & 0x1ffffu);
+        int32_t stop = e < 64 * NW ? (int32_t)e : -1;
         if (stop == entry) {  // the first sequence is not one for a round
           ip = base + entry;
           general = true;
@@ -459,14 +488,12 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         }
         // walk
         uint64_t starts = 0;
-        if (mine_at >= 0) {
-          int32_t l = mine_at, n;
-          for (;;) {
+        if (mine_at >> 6 == wave) {
+          int32_t l = mine_at & 63;
+          do {
             starts |= ((uint64_t)rdlane((uint32_t)(pass >> 32), l) << 32) | rdlane((uint32_t)pass, l);
-            n = (int32_t)rdlane(way8, l);
-            if (n >= 64 || n == l) break;
-            l = n;
-          }
+            l = (int32_t)rdlane(way8, l);
+          } while (l < 64);
           starts &= okm;
         }
         // scan
@@ -481,7 +508,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             // table: byte x of the output is a literal below `os + lit`
             tab[bits_below(starts, kbase)] =
                 (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
-            atomicOr(obits + (os >> 5), 1u << (os & 31));
+            const int32_t ob = (os - 1) & (G::kOut - 1);
+            atomicOr(obits + (ob >> 5), 1u << (ob & 31));
           }
         }
         lds_barrier();
@@ -507,57 +535,61 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         const int32_t own = __builtin_popcountll(ob);
         const int32_t before = wave_inclusive_sum(own) - own;
         for (int32_t x0 = 0; x0 < total; x0 += 2 * NT) {
-          uint32_t v[2] = {0, 0};
-          int32_t from[2];
-          bool dep[2] = {false, false};
-#pragma unroll
-          for (int u = 0; u < 2; u++) {
-            const int32_t xw = x0 + NT * u + 64 * wave;
-            if (xw < total) {
-              const int32_t x = xw + lane;
-              const int32_t q = xw >> 6;
-              const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), q) << 32) | rdlane((uint32_t)ob, q);
-              // the last sequence that starts at or before this byte
-              const uint64_t en =
-                  tab[bits_below(m >> 1, (int32_t)rdlane((uint32_t)before, q) - 1 + (int32_t)(m & 1))];
-              const uint32_t elo = (uint32_t)en;
-              const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
-              int32_t off = (int32_t)(elo >> 16);
-              const bool live = (im >= 0) & (x < total);
-              const bool far = live & (off > NEAR);
-              if (__ballot(live & (im >= off))) {
-                // (im + 1/2) / off is at least 1/546 away from a whole number
-                const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
-                if (im >= off) off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
-              }
-              const int32_t sp = x - off;  // source byte of a match, from op
-              const int32_t lat = (int32_t)(st - lds) + x + (int32_t)(uint32_t)(en >> 32);
-              v[u] = lds[im < 0 ? lat : (op + sp) & RM];
-              if (__ballot(far)) {
-                if (far) v[u] = dst[op + sp];
-              }
-              dep[u] = live & (sp >= x0);
-              from[u] = sp - x0;
-              rec[NT * u + tid] = (uint16_t)(dep[u] ? (uint32_t)from[u] : 0x8000u | v[u]);
+          // bit 15 and the byte, or the number of the source byte
+          uint32_t w[2] = {0x8000u, 0x8000u};
+          auto entry_of = [&](int32_t xw) -> uint64_t {  // the last sequence that starts at or before the byte
+            const int32_t q = xw >> 6;
+            const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), q) << 32) | rdlane((uint32_t)ob, q);
+            return tab[bits_below(m, (int32_t)rdlane((uint32_t)before, q))];
+          };
+          auto source_of = [&](int32_t x, uint64_t en) -> uint32_t {
+            const uint32_t elo = (uint32_t)en;
+            const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
+            int32_t off = (int32_t)(elo >> 16);
+            const bool live = (im >= 0) & (x < total);
+            const bool far = live & (off > NEAR);
+            if (live & (im >= off)) {
+              // (im + 1/2) / off is at least 1/546 away from a whole number
+              const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
+              off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
             }
+            const int32_t sp = x - off;  // source byte of a match, from op
+            const int32_t lat = st + x + (int32_t)(uint32_t)(en >> 32);
+            const int32_t rat = (op + sp) & RM, lm = im >> 31;
+            uint32_t v = lds[(lat & lm) | (rat & ~lm)];
+            if (far) {
+              v = dst[op + sp];
+              asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
+            }
+            return live & (sp >= x0) ? (uint32_t)(sp - x0) : 0x8000u | v;
+          };
+          const int32_t xw = x0 + 64 * wave;
+          if (xw + NT < total) {
+            const uint64_t e0 = entry_of(xw), e1 = entry_of(xw + NT);
+            w[0] = source_of(xw + lane, e0);
+            w[1] = source_of(xw + NT + lane, e1);
+            rec[tid] = (uint16_t)w[0];
+            rec[NT + tid] = (uint16_t)w[1];
+          } else if (xw < total) {
+            w[0] = source_of(xw + lane, entry_of(xw));
+            rec[tid] = (uint16_t)w[0];
           }
           lds_barrier();
 #pragma unroll
           for (int u = 0; u < 2; u++) {
-            while (__ballot(dep[u])) {
-              if (dep[u]) {
-                const uint32_t r = rec[from[u]];
-                rec[NT * u + tid] = (uint16_t)r;
-                from[u] = (int32_t)r;
-                v[u] = r & 255u;
-                dep[u] = r < 0x8000u;
-              }
+            uint16_t *mine = rec + NT * u + tid;
+            while (ballot(w[u] < 0x8000u)) {
+              // (one that has its byte reads it again)
+              w[u] = __hip_atomic_load(w[u] < 0x8000u ? rec + w[u] : mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_store(mine, (uint16_t)w[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
             const int32_t x = x0 + NT * u + tid;
-            if (x < total) ring[(op + x) & RM] = (uint8_t)v[u];
+            if (x < total) ring[(op + x) & RM] = (uint8_t)w[u];
           }
-          if (x0 + 2 * NT >= total && tid < G::kStageWords)
-            reinterpret_cast<uint32_t *>(stage + (buf ^ 1) * G::kStage)[tid] = ahead;
+          if (x0 + 2 * NT >= total) {
+            asm volatile("" : "+v"(ahead));  // arrived, in every wavefront
+            if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage + (buf ^ 1) * G::kStage)[tid] = ahead;
+          }
           lds_barrier();
         }
         op += total;
@@ -567,11 +599,11 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           break;
         }
         if (e >= 128 * NW) {  // past all of the next round
-          ip = base + e;
+          ip = base + (int32_t)e;
           break;
         }
         base = nbase;
-        entry = e - 64 * NW;
+        entry = (int32_t)e - 64 * NW;
         buf ^= 1;
       }
     }
@@ -596,7 +628,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         if (ip + 64 > gb + 256) look(ip);
         const int32_t q = ip - gb + lane;
         const uint32_t b = ((uint32_t)bperm(q >> 2, (int32_t)gw) >> ((q & 3) << 3)) & 255u;
-        const uint64_t stop = __ballot(ip + lane < iend && b != 255u);
+        const uint64_t stop = ballot(ip + lane < iend && b != 255u);
         if (stop) {
           const int32_t t = (int32_t)__builtin_ctzll(stop);
           v += 255 * t + (int32_t)rdlane(b, t);
@@ -1043,10 +1075,13 @@ namespace iamx {
 // sequence with the fewest instructions.  The lines are where a CU still holds
 // all of its streams at once (4 x 8 and 8 x 4 wavefronts).  Measured in us with
 // 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250 KB: 4 streams
-// 185 / 251 / 537, 1024 streams 416 / 437 / 775, 2048 streams 800 / 664 / 857,
-// 4096 streams - / 1318 / 1006, 6400 streams - / 1884 / 1358; exponent planes of
-// float32 (64 KB): 4 streams 325 / 474 / 1005, 1024 streams 644 / 693 / 1156,
-// 6400 streams - / 3019 / 1966.
+// 136 / 205 / 443, 1024 streams 306 / 352 / 667, 2048 streams 545 / 536 / 732,
+// 3072 streams - / 762 / 803, 4096 streams - / 913 / 914, 6400 streams with one
+// 1266; exponent planes of float32 (64 KB): 4 streams 219 / 383 / 875, 1024
+// streams 429 / 528 / 1027, 2048 streams 791 / 765 / 1113, 3072 streams - /
+// 1125 / 1204, 4096 streams - / 1412 / 1303; byte planes of 16 KB of float64:
+// 2048 streams 185 / 175 / 239, 3072 streams - / 250 / 258; short ones (700
+// bytes): 3072 streams - / 151 / 121.
 int launch_lz4(const char *name, const iamx_lz4_job_t *d_lz4, int n_lz4, void *d_scratch, int64_t cap) {
   const int z = zstd_enabled() ? 1 : 0;
   if (n_lz4 <= 4 * g_num_cus)
