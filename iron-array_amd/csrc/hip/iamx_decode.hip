@@ -85,11 +85,11 @@ template <int NW>
 struct Lz4Geom {
   static constexpr int kThreads = 64 * NW;
   static constexpr int kRing = 4096 * NW;         // output history, bytes
-  static constexpr int kOut = 256 * NW;           // most output bytes of a round
-  static constexpr int kStep = kOut;              // output bytes of a step of the general path
+  static constexpr int kOut = 512 * NW;           // most output bytes of a round
+  static constexpr int kStep = 256 * NW;          // output bytes of a step of the general path
   static constexpr int kStageWords = 16 * NW + 72;  // input of a round: 64 NW positions and what the last ones reach
   static constexpr int kStage = 4 * kStageWords;
-  static constexpr int kSeqs = 22 * NW;           // a sequence takes at least 3 input bytes
+  static constexpr int kSeqs = (64 * NW + 2) / 3;   // a sequence takes at least 3 input bytes
   // LDS: ring, two stages, sequence table, first-output-byte bits, source
   // records of an output step, window exits, the cut
   static constexpr int kTabAt = kRing + 2 * kStage;
@@ -169,9 +169,16 @@ struct Lz4Geom<1> {
 // Of a launch of 6400 bitshuffled streams, 0.35 ms are their literal runs
 // crossing HBM at 4.8 TB/s.
 //
+// A round's output is cut at 8 bytes an input position (1024 bytes with one
+// wavefront); several wavefronts then take the rest of the same positions.  At 4
+// bytes a position, with the input staged anew, streams of sparse rows were cut
+// in every round: 1024 byte planes of 700 bytes for 15625 took 63 us, now 51.
+//
 // What a round cannot hold (long literal runs, matches of more than 273
 // bytes, the stream's end) is decoded one sequence at a time by the general
-// path, with all threads copying.
+// path, with all threads copying.  Where the next sequence is seen to be long as
+// well, several wavefronts stay there (a bitshuffled float32 stream 136 to 133
+// us, one of a matrix's last rows 102 to 94; nothing with one wavefront).
 //
 // Output bytes go to an LDS ring and reach the stream's scratch slot in
 // 16-byte stores whenever a quarter of the ring is pending.  An offset of more
@@ -230,381 +237,389 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
   };
 
   int bad = 0;
+  bool general = false;
   for (;;) {
     // ---- rounds
-    bool general = false;
-    if constexpr (NW == 1) {
-      constexpr int32_t SM = G::kStage - 1, WIN = 63, NEAR1 = RING - 64;
-      uint16_t *list = reinterpret_cast<uint16_t *>(lds + G::kListAt);
-      uint32_t *stage32 = reinterpret_cast<uint32_t *>(stage);
-      // 256 input bytes from pos, a multiple of 256, into the stage
-      auto put_stage = [&](int32_t pos, uint32_t w) {
-        const int32_t at = (pos & SM) >> 2;
-        stage32[at + lane] = w;
-        if (at == 0 && lane < 4) stage32[G::kStage / 4 + lane] = w;
-        __builtin_amdgcn_wave_barrier();
-      };
-      int32_t have = (ip & ~255) + 768;  // the stage holds the input from ip up to here
-      {
-        const uint32_t a = ld_word(have - 768, lane), b = ld_word(have - 512, lane), c = ld_word(have - 256, lane);
-        put_stage(have - 768, a);
-        put_stage(have - 512, b);
-        put_stage(have - 256, c);
-      }
-      for (;;) {
-        // no window of a round starts 189 bytes from ip or more, and its last
-        // sequence starts within 62
-        while (have < ip + 3 * WIN + 62 + kSeqIn + 8) {
-          put_stage(have, ld_word(have, lane));
-          have += 256;
+    if (!general) {
+      if constexpr (NW == 1) {
+        constexpr int32_t SM = G::kStage - 1, WIN = 63, NEAR1 = RING - 64;
+        uint16_t *list = reinterpret_cast<uint16_t *>(lds + G::kListAt);
+        uint32_t *stage32 = reinterpret_cast<uint32_t *>(stage);
+        // 256 input bytes from pos, a multiple of 256, into the stage
+        auto put_stage = [&](int32_t pos, uint32_t w) {
+          const int32_t at = (pos & SM) >> 2;
+          stage32[at + lane] = w;
+          if (at == 0 && lane < 4) stage32[G::kStage / 4 + lane] = w;
+          __builtin_amdgcn_wave_barrier();
+        };
+        int32_t have = (ip & ~255) + 768;  // the stage holds the input from ip up to here
+        {
+          const uint32_t a = ld_word(have - 768, lane), b = ld_word(have - 512, lane), c = ld_word(have - 256, lane);
+          put_stage(have - 768, a);
+          put_stage(have - 512, b);
+          put_stage(have - 256, c);
         }
-        const bool more = have - ip < 768;
-        uint32_t ahead = 0;
-        if (more) ahead = ld_word(have, lane);
-        if (lane < G::kOut / 32) obits[lane] = 0;
-        // walk: the starts of up to three windows, listed by position
-        int32_t n = 0, at = ip;  // sequences so far, the next one's position
-        bool stopped = false;
-        do {
-          const uint32_t h = lds_u32(stage, (at + lane) & SM);
-          const uint32_t hl = (h >> 4) & 15u, lb = (h >> 8) & 255u;
-          const int32_t adv = 3 + (int32_t)hl + (hl == 15 ? (int32_t)lb + 1 : 0) + ((h & 15u) == 15 ? 1 : 0);
-          const bool ok = (!((hl == 15) & (lb == 255)) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
-          const int32_t to = ok ? min(lane + adv, WIN) : lane;
-          const int32_t to2 = bperm(to, to);
-          uint64_t starts = 0;
-          int32_t l = 0, t1;
+        for (;;) {
+          // no window of a round starts 189 bytes from ip or more, and its last
+          // sequence starts within 62
+          while (have < ip + 3 * WIN + 62 + kSeqIn + 8) {
+            put_stage(have, ld_word(have, lane));
+            have += 256;
+          }
+          const bool more = have - ip < 768;
+          uint32_t ahead = 0;
+          if (more) ahead = ld_word(have, lane);
+          if (lane < G::kOut / 32) obits[lane] = 0;
+          // walk: the starts of up to three windows, listed by position
+          int32_t n = 0, at = ip;  // sequences so far, the next one's position
+          bool stopped = false;
           do {
-            t1 = (int32_t)rdlane((uint32_t)to, l);
-            bit_on(starts, l);
-            bit_on(starts, t1);
-            l = (int32_t)rdlane((uint32_t)to2, l);
-          } while (l != t1);
-          bit_off(starts, l);  // where it ends is no start: a stop, or past the window
-          stopped = l < WIN;
-          if (starts == 0) break;
-          const int32_t k = bits_below(starts, n);
-          if ((starts >> lane) & 1ull) list[k] = (uint16_t)(at - ip + lane);
-          n += __builtin_popcountll(starts);
-          const int32_t last = 63 - __builtin_clzll(starts);
-          at += last + (int32_t)rdlane((uint32_t)adv, last);
-        } while (!stopped && at - ip < 3 * WIN);  // a window leads past its 63 positions
-        if (n == 0) {
-          general = true;
-          break;
-        }
-        __builtin_amdgcn_wave_barrier();
-        // lane k takes sequence k
-        const int32_t pos = ip + (int32_t)list[lane];
-        const uint32_t h = lds_u32(stage, pos & SM);
-        const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
-        const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
-        const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
-        const int32_t src = pos + 1 + (int32_t)lext;  // first literal
-        const uint32_t h2 = lds_u32(stage, (src + lit) & SM);
-        const int32_t hoff = (int32_t)(h2 & 0xffffu);
-        const uint32_t he = (h2 >> 16) & 255u;
-        const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
-        const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
-        const bool mine = lane < n;
-        const int32_t oinc = wave_inclusive_sum(mine ? len : 0);
-        const int32_t os = oinc - len;  // this sequence's first output byte, from op
-        // the first sequence that does not fit, or ends in a second length byte
-        const bool hard = (((ext != 0) & (he == 255)) | (hoff < 1) | (hoff > op + os + lit) | (oinc > oend - op)) != 0;
-        const uint64_t cutm = ballot(mine & (hard | (oinc > G::kOut)));
-        const uint64_t hardm = ballot(hard);
-        int32_t nseq = n;
-        if (cutm) {
-          nseq = __builtin_ctzll(cutm);
-          stopped = ((hardm >> nseq) & 1ull) != 0;
-          at = (int32_t)rdlane((uint32_t)pos, nseq);
-          if (nseq == 0) {
+            const uint32_t h = lds_u32(stage, (at + lane) & SM);
+            const uint32_t hl = (h >> 4) & 15u, lb = (h >> 8) & 255u;
+            const int32_t adv = 3 + (int32_t)hl + (hl == 15 ? (int32_t)lb + 1 : 0) + ((h & 15u) == 15 ? 1 : 0);
+            const bool ok = (!((hl == 15) & (lb == 255)) & (adv <= iend - at - lane) & (lane < WIN)) != 0;
+            const int32_t to = ok ? min(lane + adv, WIN) : lane;
+            const int32_t to2 = bperm(to, to);
+            uint64_t starts = 0;
+            int32_t l = 0, t1;
+            do {
+              t1 = (int32_t)rdlane((uint32_t)to, l);
+              bit_on(starts, l);
+              bit_on(starts, t1);
+              l = (int32_t)rdlane((uint32_t)to2, l);
+            } while (l != t1);
+            bit_off(starts, l);  // where it ends is no start: a stop, or past the window
+            stopped = l < WIN;
+            if (starts == 0) break;
+            const int32_t k = bits_below(starts, n);
+            if ((starts >> lane) & 1ull) list[k] = (uint16_t)(at - ip + lane);
+            n += __builtin_popcountll(starts);
+            const int32_t last = 63 - __builtin_clzll(starts);
+            at += last + (int32_t)rdlane((uint32_t)adv, last);
+          } while (!stopped && at - ip < 3 * WIN);  // a window leads past its 63 positions
+          if (n == 0) {
             general = true;
             break;
           }
-        }
-        const int32_t total = (int32_t)rdlane((uint32_t)oinc, nseq - 1);
-        if (lane < nseq) {
-          // byte x of the output is a literal below `os + lit`
-          tab[lane] = (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
-          const int32_t ob = (os - 1) & (G::kOut - 1);
-          atomicOr(obits + (ob >> 5), 1u << (ob & 31));
-        }
-        __builtin_amdgcn_wave_barrier();
-        const uint64_t ob = lane < G::kOut / 64 ? reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)] : 0ull;
-        int32_t before = 0;  // sequences that start in earlier steps, or with this one, less one
-        auto entry_of = [&](int32_t x0) -> uint64_t {
-          const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), x0 >> 6) << 32) | rdlane((uint32_t)ob, x0 >> 6);
-          const int32_t k = bits_below(m, before);  // the last start at or before its byte
-          before += __builtin_popcountll(m);
-          return tab[k];
-        };
-        uint64_t e = entry_of(0);
-        for (int32_t x0 = 0;;) {
-          const int32_t x = x0 + lane;
-          const uint32_t elo = (uint32_t)e;
-          const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
-          int32_t off = (int32_t)(elo >> 16);
-          const int32_t lat = RING + ((x + (int32_t)(uint32_t)(e >> 32)) & SM);
-          int32_t sp = op + x - off;
-          // a source past the ring, inside the match itself or inside this step
-          const bool odd = (im >= 0) & (x < total) & ((off > NEAR1) | (off <= max(im, lane)));
-          const int32_t x1 = x0 + 64;
-          uint32_t v;
-          if (ballot(odd)) {
-            if (odd & (im >= off)) {
-              // (im + 1/2) / off is at least 1/546 away from a whole number
-              const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
-              off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
+          __builtin_amdgcn_wave_barrier();
+          // lane k takes sequence k
+          const int32_t pos = ip + (int32_t)list[lane];
+          const uint32_t h = lds_u32(stage, pos & SM);
+          const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
+          const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
+          const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
+          const int32_t src = pos + 1 + (int32_t)lext;  // first literal
+          const uint32_t h2 = lds_u32(stage, (src + lit) & SM);
+          const int32_t hoff = (int32_t)(h2 & 0xffffu);
+          const uint32_t he = (h2 >> 16) & 255u;
+          const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
+          const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
+          const bool mine = lane < n;
+          const int32_t oinc = wave_inclusive_sum(mine ? len : 0);
+          const int32_t os = oinc - len;  // this sequence's first output byte, from op
+          // the first sequence that does not fit, or ends in a second length byte
+          const bool hard =
+              (((ext != 0) & (he == 255)) | (hoff < 1) | (hoff > op + os + lit) | (oinc > oend - op)) != 0;
+          const uint64_t cutm = ballot(mine & (hard | (oinc > G::kOut)));
+          const uint64_t hardm = ballot(hard);
+          int32_t nseq = n;
+          if (cutm) {
+            nseq = __builtin_ctzll(cutm);
+            stopped = ((hardm >> nseq) & 1ull) != 0;
+            at = (int32_t)rdlane((uint32_t)pos, nseq);
+            if (nseq == 0) {
+              general = true;
+              break;
             }
-            sp = op + x - off;
-            v = lds[im < 0 ? lat : sp & RM];
-            if (x1 < total) e = entry_of(x1);
-            // at most FLUSH_AT + kOut bytes are pending, so a far source was
-            // flushed, by this wavefront's own stores
-            if (odd & (off > NEAR1)) {
-              v = dst[sp];
-              asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
-            }
-            const bool dep = odd & (off <= lane);
-            if (ballot(dep)) {
-              // bit 6: the lane has its own byte
-              int32_t code = dep ? lane - off : lane | 64;
-              do {
-                code = bperm(code, code);
-              } while (ballot(code < 64));
-              v = (uint32_t)bperm(code, (int32_t)v);
-            }
-          } else {
-            v = lds[im < 0 ? lat : sp & RM];
-            if (x1 < total) e = entry_of(x1);
           }
-          __builtin_amdgcn_wave_barrier();
-          ring[(op + x) & RM] = (uint8_t)v;
-          __builtin_amdgcn_wave_barrier();
-          if (x1 >= total) break;
-          x0 = x1;
-        }
-        op += total;
-        ip = at;
-        asm volatile("" : "+v"(ahead));  // arrived; what follows is stored without a wait
-        if (more) {
-          put_stage(have, ahead);
-          have += 256;
-        }
-        if (op >= flush_at) flush(op);
-        if (stopped) {
-          general = true;
-          break;
-        }
-      }
-    } else {
-      uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
-      uint32_t *exits = reinterpret_cast<uint32_t *>(lds + G::kExitAt);
-      unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
-      int32_t base = ip, entry = 0, buf = 0;
-      if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage)[tid] = ld_word(base, tid);
-      lds_barrier();
-      for (;;) {
-        const int32_t nbase = base + 64 * NW;
-        uint32_t ahead = 0;  // the next round's input, on its way until the end of this one
-        if (tid < G::kStageWords) ahead = ld_word(nbase, tid);
-        if (tid < G::kOut / 32) obits[tid] = 0;
-        if (tid == 0) *cut = ~0ull;
-        // headers
-        const int32_t st = RING + buf * G::kStage + (base & 3);
-        const uint32_t h = lds_u32(lds, st + tid);
-        const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
-        const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
-        const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
-        const int32_t src = tid + 1 + (int32_t)lext;  // first literal, from base
-        const uint32_t h2 = lds_u32(lds, st + min(src + lit, G::kStage - 8));
-        const int32_t hoff = (int32_t)(h2 & 0xffffu);
-        const uint32_t he = (h2 >> 16) & 255u;
-        const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
-        const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
-        const int32_t adv = 3 + lit + (int32_t)(lext + ext);
-        // (bitwise: one vector compare chain, no branches)
-        const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
-                         (adv <= iend - base - tid)) != 0;
-        const uint64_t okm = ballot(ok);
-        // reach: bits 0..9 the lane the chain from here has got to (64 and more
-        // is a position of a later window; a start that is not ok leads to
-        // itself), bits 10..26 the output bytes and bits 27..31 the sequences on
-        // the way (at most 21 of 542 bytes)
-        uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 27) : (uint32_t)lane;
-        auto hop = [&]() {
-          const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
-          if ((way & 1023u) < 64) way = f + (way & ~1023u);
-        };
-        uint64_t pass = 1ull << lane;  // the starts of the next eight hops
-        auto join = [&]() {
-          const uint32_t lo = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)pass);
-          const uint32_t hi = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)(pass >> 32));
-          if ((way & 1023u) < 64) pass |= ((uint64_t)hi << 32) | lo;
-        };
-        {
-          const uint32_t to = way & 1023u;
-          if (to < 64) pass |= 1ull << to;
-        }
-        hop();
-        join();
-        hop();
-        join();
-        hop();
-        const uint32_t to8 = way & 1023u;
-        const uint32_t way8 = to8 == (uint32_t)lane ? 64u : to8;  // below 64: go on from there
-        hop();
-        hop();
-        exits[tid] = way + 64 * wave;  // positions from base
-        lds_barrier();
-        // chain: a stop stays in its window, where no later step takes it up.
-        // Lane v of `at` and `past` is where window v is entered, and the bytes
-        // (17 bits) and sequences before it.
-        uint32_t ex[NW];
-#pragma unroll
-        for (int v = 0; v < NW; v++) ex[v] = exits[64 * v + lane];
-        uint32_t e = (uint32_t)entry, sum = 0;
-        uint32_t at = 0, past = 0;
-#pragma unroll
-        for (int v = 0; v < NW; v++) {
-          const uint32_t x = rdlane(ex[v], (int32_t)(e & 63u));
-          set_lane(at, v, e);
-          set_lane(past, v, sum);
-          const uint32_t y = (e >> 6) == (uint32_t)v ? x : e;
-          sum += y >> 10;
-          e = y & 1023u;
-        }
-        asm("s_nop 1" : "+v"(at), "+v"(past));  // before lanes written in asm are read
-        const int32_t mine_at = (int32_t)rdlane(at, wave);
-        const uint32_t before_me = rdlane(past, wave);
-        const int32_t obase = (int32_t)(before_me & 0x1ffffu), kbase = (int32_t)(before_me >> 17);
-        int32_t total = (int32_t)(sum & 0x1ffffu);
-        int32_t stop = e < 64 * NW ? (int32_t)e : -1;
-        if (stop == entry) {  // the first sequence is not one for a round
-          ip = base + entry;
-          general = true;
-          break;
-        }
-        // walk
-        uint64_t starts = 0;
-        if (mine_at >> 6 == wave) {
-          int32_t l = mine_at & 63;
-          do {
-            starts |= ((uint64_t)rdlane((uint32_t)(pass >> 32), l) << 32) | rdlane((uint32_t)pass, l);
-            l = (int32_t)rdlane(way8, l);
-          } while (l < 64);
-          starts &= okm;
-        }
-        // scan
-        const bool mine = ((starts >> lane) & 1ull) != 0;
-        const int32_t oinc = obase + wave_inclusive_sum(mine ? len : 0);
-        const int32_t os = oinc - len;  // this sequence's first output byte, from op
-        if (mine) {
-          const bool hard = (oinc > oend - op) | (hoff > op + os + lit);
-          if (hard | (oinc > G::kOut)) {
-            atomicMin(cut, ((unsigned long long)tid << 32) | ((uint32_t)os << 1) | (hard ? 1u : 0u));
-          } else {
-            // table: byte x of the output is a literal below `os + lit`
-            tab[bits_below(starts, kbase)] =
+          const int32_t total = (int32_t)rdlane((uint32_t)oinc, nseq - 1);
+          if (lane < nseq) {
+            // byte x of the output is a literal below `os + lit`
+            tab[lane] =
                 (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
             const int32_t ob = (os - 1) & (G::kOut - 1);
             atomicOr(obits + (ob >> 5), 1u << (ob & 31));
           }
-        }
-        lds_barrier();
-        // output: lane q of a wavefront holds the bits of bytes 64 q .. 64 q + 63
-        // and the number of sequences that start before them
-        const uint64_t ob = reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)];
-        const uint64_t c = *cut;
-        const uint32_t clo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)c),
-                       chi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(c >> 32));
-        const bool is_cut = chi != ~0u;
-        if (is_cut) {
-          total = (int32_t)(clo >> 1);
-          stop = (int32_t)chi;
-          general = (clo & 1u) != 0;
-          if (total == 0) {  // the first sequence itself (never for its length alone)
-            ip = base + stop;
+          __builtin_amdgcn_wave_barrier();
+          const uint64_t *words = reinterpret_cast<const uint64_t *>(obits);
+          const uint64_t ob = lane < G::kOut / 64 ? words[lane & (G::kOut / 64 - 1)] : 0ull;
+          int32_t before = 0;  // sequences that start in earlier steps, or with this one, less one
+          auto entry_of = [&](int32_t x0) -> uint64_t {
+            const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), x0 >> 6) << 32) | rdlane((uint32_t)ob, x0 >> 6);
+            const int32_t k = bits_below(m, before);  // the last start at or before its byte
+            before += __builtin_popcountll(m);
+            return tab[k];
+          };
+          uint64_t e = entry_of(0);
+          for (int32_t x0 = 0;;) {
+            const int32_t x = x0 + lane;
+            const uint32_t elo = (uint32_t)e;
+            const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
+            int32_t off = (int32_t)(elo >> 16);
+            const int32_t lat = RING + ((x + (int32_t)(uint32_t)(e >> 32)) & SM);
+            int32_t sp = op + x - off;
+            // a source past the ring, inside the match itself or inside this step
+            const bool odd = (im >= 0) & (x < total) & ((off > NEAR1) | (off <= max(im, lane)));
+            const int32_t x1 = x0 + 64;
+            uint32_t v;
+            if (ballot(odd)) {
+              if (odd & (im >= off)) {
+                // (im + 1/2) / off is at least 1/546 away from a whole number
+                const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
+                off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
+              }
+              sp = op + x - off;
+              v = lds[im < 0 ? lat : sp & RM];
+              if (x1 < total) e = entry_of(x1);
+              // at most FLUSH_AT + kOut bytes are pending, so a far source was
+              // flushed, by this wavefront's own stores
+              if (odd & (off > NEAR1)) {
+                v = dst[sp];
+                asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
+              }
+              const bool dep = odd & (off <= lane);
+              if (ballot(dep)) {
+                // bit 6: the lane has its own byte
+                int32_t code = dep ? lane - off : lane | 64;
+                do {
+                  code = bperm(code, code);
+                } while (ballot(code < 64));
+                v = (uint32_t)bperm(code, (int32_t)v);
+              }
+            } else {
+              v = lds[im < 0 ? lat : sp & RM];
+              if (x1 < total) e = entry_of(x1);
+            }
+            __builtin_amdgcn_wave_barrier();
+            ring[(op + x) & RM] = (uint8_t)v;
+            __builtin_amdgcn_wave_barrier();
+            if (x1 >= total) break;
+            x0 = x1;
+          }
+          op += total;
+          ip = at;
+          asm volatile("" : "+v"(ahead));  // arrived; what follows is stored without a wait
+          if (more) {
+            put_stage(have, ahead);
+            have += 256;
+          }
+          if (op >= flush_at) flush(op);
+          if (stopped) {
             general = true;
             break;
           }
-        } else {
-          general = stop >= 0;
         }
-        const int32_t own = __builtin_popcountll(ob);
-        const int32_t before = wave_inclusive_sum(own) - own;
-        for (int32_t x0 = 0; x0 < total; x0 += 2 * NT) {
-          // bit 15 and the byte, or the number of the source byte
-          uint32_t w[2] = {0x8000u, 0x8000u};
-          auto entry_of = [&](int32_t xw) -> uint64_t {  // the last sequence that starts at or before the byte
-            const int32_t q = xw >> 6;
-            const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), q) << 32) | rdlane((uint32_t)ob, q);
-            return tab[bits_below(m, (int32_t)rdlane((uint32_t)before, q))];
+      } else {
+        uint16_t *rec = reinterpret_cast<uint16_t *>(lds + G::kRecAt);
+        uint32_t *exits = reinterpret_cast<uint32_t *>(lds + G::kExitAt);
+        unsigned long long *cut = reinterpret_cast<unsigned long long *>(lds + G::kCutAt);
+        int32_t base = ip, entry = 0, buf = 0;
+        if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage)[tid] = ld_word(base, tid);
+        lds_barrier();
+        for (;;) {
+          const int32_t nbase = base + 64 * NW;
+          uint32_t ahead = 0;  // the next round's input, on its way until the end of this one
+          if (tid < G::kStageWords) ahead = ld_word(nbase, tid);
+          if (tid < G::kOut / 32) obits[tid] = 0;
+          if (tid == 0) *cut = ~0ull;
+          // headers
+          const int32_t st = RING + buf * G::kStage + (base & 3);
+          const uint32_t h = lds_u32(lds, st + tid);
+          const uint32_t hl = (h >> 4) & 15u, hm = h & 15u, lb = (h >> 8) & 255u;
+          const uint32_t lext = hl == 15 ? 1u : 0u;  // one literal length byte
+          const int32_t lit = (int32_t)(hl + (lext ? lb : 0u));
+          const int32_t src = tid + 1 + (int32_t)lext;  // first literal, from base
+          const uint32_t h2 = lds_u32(lds, st + min(src + lit, G::kStage - 8));
+          const int32_t hoff = (int32_t)(h2 & 0xffffu);
+          const uint32_t he = (h2 >> 16) & 255u;
+          const uint32_t ext = hm == 15 ? 1u : 0u;  // one match length byte
+          const int32_t len = lit + (int32_t)(hm + 4 + (ext ? he : 0u));
+          const int32_t adv = 3 + lit + (int32_t)(lext + ext);
+          // (bitwise: one vector compare chain, no branches)
+          const bool ok = (!(lext & (lb == 255)) & !(ext & (he == 255)) & (hoff >= 1) &
+                           (adv <= iend - base - tid)) != 0;
+          const uint64_t okm = ballot(ok);
+          // reach: bits 0..9 the lane the chain from here has got to (64 and more
+          // is a position of a later window; a start that is not ok leads to
+          // itself), bits 10..26 the output bytes and bits 27..31 the sequences on
+          // the way (at most 21 of 542 bytes)
+          uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 27) : (uint32_t)lane;
+          auto hop = [&]() {
+            const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
+            if ((way & 1023u) < 64) way = f + (way & ~1023u);
           };
-          auto source_of = [&](int32_t x, uint64_t en) -> uint32_t {
-            const uint32_t elo = (uint32_t)en;
-            const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
-            int32_t off = (int32_t)(elo >> 16);
-            const bool live = (im >= 0) & (x < total);
-            const bool far = live & (off > NEAR);
-            if (live & (im >= off)) {
-              // (im + 1/2) / off is at least 1/546 away from a whole number
-              const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
-              off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
-            }
-            const int32_t sp = x - off;  // source byte of a match, from op
-            const int32_t lat = st + x + (int32_t)(uint32_t)(en >> 32);
-            const int32_t rat = (op + sp) & RM, lm = im >> 31;
-            uint32_t v = lds[(lat & lm) | (rat & ~lm)];
-            if (far) {
-              v = dst[op + sp];
-              asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
-            }
-            return live & (sp >= x0) ? (uint32_t)(sp - x0) : 0x8000u | v;
+          uint64_t pass = 1ull << lane;  // the starts of the next eight hops
+          auto join = [&]() {
+            const uint32_t lo = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)pass);
+            const uint32_t hi = (uint32_t)bperm((int32_t)way, (int32_t)(uint32_t)(pass >> 32));
+            if ((way & 1023u) < 64) pass |= ((uint64_t)hi << 32) | lo;
           };
-          const int32_t xw = x0 + 64 * wave;
-          if (xw + NT < total) {
-            const uint64_t e0 = entry_of(xw), e1 = entry_of(xw + NT);
-            w[0] = source_of(xw + lane, e0);
-            w[1] = source_of(xw + NT + lane, e1);
-            rec[tid] = (uint16_t)w[0];
-            rec[NT + tid] = (uint16_t)w[1];
-          } else if (xw < total) {
-            w[0] = source_of(xw + lane, entry_of(xw));
-            rec[tid] = (uint16_t)w[0];
+          {
+            const uint32_t to = way & 1023u;
+            if (to < 64) pass |= 1ull << to;
           }
+          hop();
+          join();
+          hop();
+          join();
+          hop();
+          const uint32_t to8 = way & 1023u;
+          const uint32_t way8 = to8 == (uint32_t)lane ? 64u : to8;  // below 64: go on from there
+          hop();
+          hop();
+          exits[tid] = way + 64 * wave;  // positions from base
           lds_barrier();
+          // chain: a stop stays in its window, where no later step takes it up.
+          // Lane v of `at` and `past` is where window v is entered, and the bytes
+          // (17 bits) and sequences before it.
+          uint32_t ex[NW];
 #pragma unroll
-          for (int u = 0; u < 2; u++) {
-            uint16_t *mine = rec + NT * u + tid;
-            while (ballot(w[u] < 0x8000u)) {
-              // (one that has its byte reads it again)
-              w[u] = __hip_atomic_load(w[u] < 0x8000u ? rec + w[u] : mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              __hip_atomic_store(mine, (uint16_t)w[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            const int32_t x = x0 + NT * u + tid;
-            if (x < total) ring[(op + x) & RM] = (uint8_t)w[u];
+          for (int v = 0; v < NW; v++) ex[v] = exits[64 * v + lane];
+          uint32_t e = (uint32_t)entry, sum = 0;
+          uint32_t at = 0, past = 0;
+#pragma unroll
+          for (int v = 0; v < NW; v++) {
+            const uint32_t x = rdlane(ex[v], (int32_t)(e & 63u));
+            set_lane(at, v, e);
+            set_lane(past, v, sum);
+            const uint32_t y = (e >> 6) == (uint32_t)v ? x : e;
+            sum += y >> 10;
+            e = y & 1023u;
           }
-          if (x0 + 2 * NT >= total) {
-            asm volatile("" : "+v"(ahead));  // arrived, in every wavefront
-            if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage + (buf ^ 1) * G::kStage)[tid] = ahead;
+          asm("s_nop 1" : "+v"(at), "+v"(past));  // before lanes written in asm are read
+          const int32_t mine_at = (int32_t)rdlane(at, wave);
+          const uint32_t before_me = rdlane(past, wave);
+          const int32_t obase = (int32_t)(before_me & 0x1ffffu), kbase = (int32_t)(before_me >> 17);
+          int32_t total = (int32_t)(sum & 0x1ffffu);
+          int32_t stop = e < 64 * NW ? (int32_t)e : -1;
+          if (stop == entry) {  // the first sequence is not one for a round
+            ip = base + entry;
+            general = true;
+            break;
+          }
+          // walk
+          uint64_t starts = 0;
+          if (mine_at >> 6 == wave) {
+            int32_t l = mine_at & 63;
+            do {
+              starts |= ((uint64_t)rdlane((uint32_t)(pass >> 32), l) << 32) | rdlane((uint32_t)pass, l);
+              l = (int32_t)rdlane(way8, l);
+            } while (l < 64);
+            starts &= okm;
+          }
+          // scan
+          const bool mine = ((starts >> lane) & 1ull) != 0;
+          const int32_t oinc = obase + wave_inclusive_sum(mine ? len : 0);
+          const int32_t os = oinc - len;  // this sequence's first output byte, from op
+          if (mine) {
+            const bool hard = (oinc > oend - op) | (hoff > op + os + lit);
+            if (hard | (oinc > G::kOut)) {
+              atomicMin(cut, ((unsigned long long)tid << 32) | ((uint32_t)os << 1) | (hard ? 1u : 0u));
+            } else {
+              // table: byte x of the output is a literal below `os + lit`
+              tab[bits_below(starts, kbase)] =
+                  (uint64_t)((uint32_t)(os + lit) | ((uint32_t)hoff << 16)) | ((uint64_t)(uint32_t)(src - os) << 32);
+              const int32_t ob = (os - 1) & (G::kOut - 1);
+              atomicOr(obits + (ob >> 5), 1u << (ob & 31));
+            }
           }
           lds_barrier();
+          // output: lane q of a wavefront holds the bits of bytes 64 q .. 64 q + 63
+          // and the number of sequences that start before them
+          const uint64_t ob = reinterpret_cast<const uint64_t *>(obits)[lane & (G::kOut / 64 - 1)];
+          const uint64_t c = *cut;
+          const uint32_t clo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)c),
+                         chi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(c >> 32));
+          const bool is_cut = chi != ~0u;
+          if (is_cut) {
+            total = (int32_t)(clo >> 1);
+            stop = (int32_t)chi;
+            general = (clo & 1u) != 0;
+            if (total == 0) {  // the first sequence itself (never for its length alone)
+              ip = base + stop;
+              general = true;
+              break;
+            }
+          } else {
+            general = stop >= 0;
+          }
+          const int32_t own = __builtin_popcountll(ob);
+          const int32_t before = wave_inclusive_sum(own) - own;
+          for (int32_t x0 = 0; x0 < total; x0 += 2 * NT) {
+            // bit 15 and the byte, or the number of the source byte
+            uint32_t w[2] = {0x8000u, 0x8000u};
+            auto entry_of = [&](int32_t xw) -> uint64_t {  // the last sequence that starts at or before the byte
+              const int32_t q = xw >> 6;
+              const uint64_t m = ((uint64_t)rdlane((uint32_t)(ob >> 32), q) << 32) | rdlane((uint32_t)ob, q);
+              return tab[bits_below(m, (int32_t)rdlane((uint32_t)before, q))];
+            };
+            auto source_of = [&](int32_t x, uint64_t en) -> uint32_t {
+              const uint32_t elo = (uint32_t)en;
+              const int32_t im = x - (int32_t)(elo & 0xffffu);  // byte of the match, negative in the literals
+              int32_t off = (int32_t)(elo >> 16);
+              const bool live = (im >= 0) & (x < total);
+              const bool far = live & (off > NEAR);
+              if (live & (im >= off)) {
+                // (im + 1/2) / off is at least 1/546 away from a whole number
+                const int32_t turn = (int32_t)(((float)im + 0.5f) * __builtin_amdgcn_rcpf((float)off));
+                off = (int32_t)__umul24((uint32_t)off, (uint32_t)(turn + 1));
+              }
+              const int32_t sp = x - off;  // source byte of a match, from op
+              const int32_t lat = st + x + (int32_t)(uint32_t)(en >> 32);
+              const int32_t rat = (op + sp) & RM, lm = im >> 31;
+              uint32_t v = lds[(lat & lm) | (rat & ~lm)];
+              if (far) {
+                v = dst[op + sp];
+                asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
+              }
+              return live & (sp >= x0) ? (uint32_t)(sp - x0) : 0x8000u | v;
+            };
+            const int32_t xw = x0 + 64 * wave;
+            if (xw + NT < total) {
+              const uint64_t e0 = entry_of(xw), e1 = entry_of(xw + NT);
+              w[0] = source_of(xw + lane, e0);
+              w[1] = source_of(xw + NT + lane, e1);
+              rec[tid] = (uint16_t)w[0];
+              rec[NT + tid] = (uint16_t)w[1];
+            } else if (xw < total) {
+              w[0] = source_of(xw + lane, entry_of(xw));
+              rec[tid] = (uint16_t)w[0];
+            }
+            lds_barrier();
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+              uint16_t *mine = rec + NT * u + tid;
+              while (ballot(w[u] < 0x8000u)) {
+                // (one that has its byte reads it again)
+                const uint16_t *at = w[u] < 0x8000u ? rec + w[u] : mine;
+                w[u] = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(mine, (uint16_t)w[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              }
+              const int32_t x = x0 + NT * u + tid;
+              if (x < total) ring[(op + x) & RM] = (uint8_t)w[u];
+            }
+            if (x0 + 2 * NT >= total) {
+              asm volatile("" : "+v"(ahead));  // arrived, in every wavefront
+              if (tid < G::kStageWords) reinterpret_cast<uint32_t *>(stage + (buf ^ 1) * G::kStage)[tid] = ahead;
+            }
+            lds_barrier();
+          }
+          op += total;
+          if (op >= flush_at) flush(op);
+          if (stop >= 0) {
+            ip = base + stop;
+            if (general) break;
+            entry = stop;  // cut: the rest of the same positions
+            continue;
+          }
+          if (e >= 128 * NW) {  // past all of the next round
+            ip = base + (int32_t)e;
+            break;
+          }
+          base = nbase;
+          entry = (int32_t)e - 64 * NW;
+          buf ^= 1;
         }
-        op += total;
-        if (op >= flush_at) flush(op);
-        if (stop >= 0) {
-          ip = base + stop;
-          break;
-        }
-        if (e >= 128 * NW) {  // past all of the next round
-          ip = base + (int32_t)e;
-          break;
-        }
-        base = nbase;
-        entry = (int32_t)e - 64 * NW;
-        buf ^= 1;
       }
     }
     if (!general) continue;  // cut where the round's output was full
@@ -694,6 +709,13 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       if (NW > 1) drain();
       lds_barrier();
     };
+    // the next sequence has a second length byte: its literals', or its match's
+    // after literals without one (a round would stop at it at once)
+    auto long_next = [&]() -> bool {
+      if (ip + 20 > gb + 256) return false;
+      const uint32_t t = rbyte(ip), l = t >> 4;
+      return l == 15 ? rbyte(ip + 1) == 255u : (t & 15u) == 15 && rbyte(ip + 3 + (int32_t)l) == 255u;
+    };
     if (ip >= iend) { bad = 1; break; }
     look(ip);
     const uint32_t token = rbyte(ip);
@@ -751,6 +773,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             return (uint8_t)((j & 8 ? hi : lo) >> (8 * (j & 3)));
           },
           [&](int32_t) -> u32x4 { return w; });
+      general = NW > 1 && long_next();
       continue;
     }
     // kStep bytes a step: byte i of a step is byte (i mod off) of the `off`
@@ -782,6 +805,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       }
       op += ml;
     }
+    general = NW > 1 && long_next();
   }
   if (!bad && op != oend) bad = 7;
   if (!bad) {  // the slot is padded to 4 bytes at least

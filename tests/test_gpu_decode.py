@@ -373,6 +373,33 @@ def test_crafted_lz4_rounds(ctx, orc, plan, copies):
         at += len(want[i % 3])
 
 
+# (literals, offsets, match lengths): rounds cut at eight output bytes an input position, or just not; and sequences
+# with a second length byte one after the other, with and without ones between that rounds take
+DENSE_PLANS = {
+    "around_the_cut": ([(1, 3)], [(1, 20), (100, 250)], [(20, 60)]),
+    "always_cut": ([(0, 1)], [(1, 9), (300, 900)], [(200, 273)]),
+    "long_in_a_row": ([(0, 14), (270, 290)], [(1, 16), (200, 900)], [(274, 290), (600, 700)]),
+    "long_and_short": ([(0, 3), (12, 16), (268, 272)], [(1, 16), (200, 900)], [(4, 20), (272, 276)]),
+}
+
+
+@pytest.mark.parametrize("copies", [3, 1100, 2100])
+@pytest.mark.parametrize("plan", sorted(DENSE_PLANS))
+def test_crafted_lz4_dense_rounds(ctx, orc, plan, copies):
+    print(f"case: crafted lz4 dense rounds {plan} x {copies}", flush=True)
+    lits, offs, mls = DENSE_PLANS[plan]
+    c = ia.Context(clevel=5, filters=0)
+    chunks, want = [], []
+    for n in [41_001, 9_999, 50_003]:
+        rng = np.random.default_rng(zlib.crc32(plan.encode()) + n)
+        stream, raw = _craft_lz4(rng, n, lambda r: (_choice(r, lits), _choice(r, offs), _choice(r, mls)))
+        assert orc.lz4_decode(stream, n) == raw
+        chunks.append(_one_stream_chunk(c, stream, n))
+        want.append(raw)
+    got = ia.decode_chunks_flat(c, [chunks[i % 3] for i in range(copies)], sum(len(want[i % 3]) for i in range(copies)))
+    assert got == b"".join(want[i % 3] for i in range(copies))
+
+
 @pytest.mark.parametrize("copies", [3, 1100, 2100])
 def test_corrupt_stream_among_many(ctx, orc, copies):
     rng = np.random.default_rng(copies)
