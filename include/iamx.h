@@ -340,6 +340,9 @@ IAMX_API void iamx_graph_destroy(void *graph_exec);
  * copy itself when kernels were launched after the last snapshot) and resets
  * a non-zero word. */
 IAMX_API int iamx_status_snapshot(void);
+/* The status word's copy and `bytes` of device memory to the host, complete on
+ * return; through the buffer of iamx_host_direct where src is 16-byte aligned. */
+IAMX_API int iamx_result_out(void *dst, const void *src, size_t bytes);
 IAMX_API int iamx_decode_status(void);
 /* Status bit of a job table entry that points outside the buffers it was
  * given (the job is skipped); bits 1..7 are malformed LZ4 streams. */

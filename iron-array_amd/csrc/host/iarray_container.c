@@ -1518,8 +1518,7 @@ static void copy_out_task(void *v, int64_t i, int worker) {
 
 static ina_rc_t download(iarray_container_t *c, const void *d_src, void *dst, size_t bytes) {
   if (bytes < 4 * IAX_COPY_TASK) {
-    int e = iamx_status_snapshot(); /* read by the caller's status check without another launch */
-    if (!e) e = iamx_d2h(dst, d_src, bytes);
+    const int e = iamx_result_out(dst, d_src, bytes); /* with the status word for the caller's check */
     return e ? iax_dev_error(e, "download") : INA_SUCCESS;
   }
   const int64_t nt = (int64_t)((bytes + IAX_COPY_TASK - 1) / IAX_COPY_TASK);

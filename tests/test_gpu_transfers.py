@@ -21,6 +21,20 @@ def test_roundtrip_sizes(rows):
     assert np.array_equal(c.to_numpy(), a)
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1025, 4095, 4097, 65_536, 524_287, 524_288, 524_289])
+def test_small_results_to_host(n):
+    """float32 results of up to 2 MiB leave in one launch, 16 bytes a thread and
+    the last ones alone; larger ones through the pinned stages.  A smaller result
+    after a larger one shows none of its bytes."""
+    rng = np.random.default_rng(n)
+    ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
+    big = rng.integers(-9, 9, (1, 300_001)).astype(np.float32)
+    assert np.array_equal(ia.Container.from_numpy(ctx, big, (1, 300_001), (1, 4096)).to_numpy(), big)
+    a = rng.integers(-9, 9, (1, n)).astype(np.float32)
+    c = ia.Container.from_numpy(ctx, a, (1, n), (1, min(n, 4096)))
+    assert np.array_equal(c.to_numpy(), a)
+
+
 def test_blocks_reused_by_other_containers():
     """Containers freed and made in turn, each decoded while others live: a
     reused device block never shows another container's data."""
