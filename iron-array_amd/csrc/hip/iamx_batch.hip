@@ -6,8 +6,7 @@
 // sorts by decreasing K, so the longest tiles start first) and computes each
 // 128x128 tile of product p with the same MFMA tile code as k_gemm.  The grid
 // is sized to the resident-workgroup capacity of the GPU, so every workgroup
-// exits after the queue runs dry.  k_pack_batch re-shuffles every C block of
-// every product in one launch.
+// exits after the queue runs dry.
 #include "iamx_internal.h"
 
 namespace {
@@ -130,78 +129,6 @@ __global__ __launch_bounds__(256) void k_gemm_batch(const iamx_batch_prod_t *__r
   }
 }
 
-__device__ __forceinline__ uint64_t load_elem(const uint8_t *src, int ts, int64_t idx) {
-  return ts == 8 ? reinterpret_cast<const uint64_t *>(src)[idx] : reinterpret_cast<const uint32_t *>(src)[idx];
-}
-
-__device__ __forceinline__ uint64_t t8(uint64_t x) {
-  uint64_t t;
-  t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
-  x = x ^ t ^ (t << 7);
-  t = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
-  x = x ^ t ^ (t << 14);
-  t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
-  x = x ^ t ^ (t << 28);
-  return x;
-}
-
-// One workgroup per C block of any product: blk[2*i] = product, blk[2*i+1] =
-// block index inside that product (chunk-major, block-major).
-__global__ __launch_bounds__(256) void k_pack_batch(const iamx_batch_pack_t *__restrict__ packs,
-                                                    const int32_t *__restrict__ blk, const uint8_t *__restrict__ base_c,
-                                                    uint8_t *__restrict__ out) {
-  const iamx_batch_pack_t Q = packs[blk[2 * blockIdx.x]];
-  const iamx_tiling_t &t = Q.tiling;
-  const int64_t id = blk[2 * blockIdx.x + 1];
-  const int64_t nbpc = t.nblocks[0] * t.nblocks[1];
-  const int64_t nc = id / nbpc, nb = id % nbpc;
-  const int64_t ci0 = nc / t.nchunks[1], ci1 = nc % t.nchunks[1];
-  const int64_t bi0 = nb / t.nblocks[1], bi1 = nb % t.nblocks[1];
-  const int ts = t.typesize;
-  const int32_t cols = (int32_t)t.block[1];
-  const int32_t n = (int32_t)(t.block[0] * t.block[1]);
-  const int64_t r_in = bi0 * t.block[0], c_in = bi1 * t.block[1];
-  const int64_t gr0 = ci0 * t.chunk[0] + r_in, gc0 = ci1 * t.chunk[1] + c_in;
-  int64_t vr = t.chunk[0] - r_in;
-  if (t.shape[0] - gr0 < vr) vr = t.shape[0] - gr0;
-  int64_t vc = t.chunk[1] - c_in;
-  if (t.shape[1] - gc0 < vc) vc = t.shape[1] - gc0;
-  const uint8_t *src = base_c + Q.c_off_bytes;
-  const int64_t ld = t.shape[1];
-  uint8_t *o = out + Q.out_off + id * (int64_t)n * ts;
-  auto elem = [&](int32_t e) -> uint64_t {
-    const int32_t r = e / cols, c = e - (e / cols) * cols;
-    if (r >= vr || c >= vc) return 0;
-    return load_elem(src, ts, (gr0 + r) * ld + gc0 + c);
-  };
-  if (t.filter == IAMX_FILTER_BITSHUFFLE) {
-    const int32_t n8 = n - n % 8, rowlen = n8 / 8;
-    for (int32_t g = threadIdx.x; g < rowlen; g += blockDim.x) {
-      uint64_t v[8];
-      for (int i = 0; i < 8; i++) v[i] = elem(8 * g + i);
-      for (int j = 0; j < ts; j++) {
-        uint64_t x = 0;
-        for (int i = 0; i < 8; i++) x |= ((v[i] >> (8 * j)) & 0xffull) << (8 * i);
-        const uint64_t y = t8(x);
-        for (int k = 0; k < 8; k++) o[(int64_t)(8 * j + k) * rowlen + g] = (uint8_t)(y >> (8 * k));
-      }
-    }
-    for (int32_t e = n8 + threadIdx.x; e < n; e += blockDim.x) {
-      const uint64_t v = elem(e);
-      for (int j = 0; j < ts; j++) o[(int64_t)e * ts + j] = (uint8_t)(v >> (8 * j));
-    }
-    return;
-  }
-  const bool shuffled = t.filter == IAMX_FILTER_SHUFFLE;
-  for (int32_t e = threadIdx.x; e < n; e += blockDim.x) {
-    const uint64_t v = elem(e);
-    for (int j = 0; j < ts; j++) {
-      if (shuffled) o[(int64_t)j * n + e] = (uint8_t)(v >> (8 * j));
-      else o[(int64_t)e * ts + j] = (uint8_t)(v >> (8 * j));
-    }
-  }
-}
-
 }  // namespace
 
 extern "C" {
@@ -229,16 +156,6 @@ IAMX_API int iamx_gemm_batch(int dtype, const iamx_batch_prod_t *d_prods, const 
                 (const float *)base_a, (const float *)base_b, (float *)base_c);
   else
     return iamx::set_error(IAMX_EINVAL, "iamx_gemm_batch: dtype %d", dtype);
-  return IAMX_OK;
-}
-
-IAMX_API int iamx_pack_batch(const iamx_batch_pack_t *d_packs, const int32_t *d_blocks, int nblocks,
-                             const void *base_c, void *d_out) {
-  int rc = iamx::ensure_init();
-  if (rc) return rc;
-  if (nblocks <= 0) return IAMX_OK;
-  IAMX_LAUNCH("pack_batch", k_pack_batch, dim3(nblocks), dim3(256), 0, d_packs, d_blocks, (const uint8_t *)base_c,
-              (uint8_t *)d_out);
   return IAMX_OK;
 }
 

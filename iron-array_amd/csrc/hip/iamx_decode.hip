@@ -1,5 +1,5 @@
 // iamx_decode.hip -- Blosc2 block decode (LZ4 + un-shuffle / bit-un-shuffle)
-// and the C write-side block packing, for gfx950.
+// and the dense transpose, for gfx950.
 //
 // Decode is two launches:
 //   k_lz4_streams   one workgroup per LZ4 stream, of 8, 4 or 1 wavefronts by
@@ -16,12 +16,8 @@
 // chunks).
 #include "iamx_internal.h"
 
-
 namespace {
 
-using iamx::tr4;
-using iamx::transpose8;
-using iamx::u32_any;
 using iamx::u32x4;
 using iamx::u32x4_any;
 
@@ -572,7 +568,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
                 v = dst[op + sp];
                 asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
               }
-              return live & (sp >= x0) ? (uint32_t)(sp - x0) : 0x8000u | v;
+              return (live & (sp >= x0)) ? (uint32_t)(sp - x0) : 0x8000u | v;
             };
             const int32_t xw = x0 + 64 * wave;
             if (xw + NT < total) {
@@ -960,118 +956,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 1
   lz4_stream<NW>(job, scratch, status, lds);
 }
 
-__device__ __forceinline__ uint64_t load_elem(const uint8_t *src, int ts, int64_t idx) {
-  switch (ts) {
-    case 8: return reinterpret_cast<const uint64_t *>(src)[idx];
-    case 4: return reinterpret_cast<const uint32_t *>(src)[idx];
-    case 2: return reinterpret_cast<const uint16_t *>(src)[idx];
-    default: return src[idx];
-  }
-}
-
-// One workgroup per C block: gather the tile (zeros outside the valid extent),
-// apply the filter, write the block's bytes at (chunk * nblocks + block) * bsize.
-__global__ __launch_bounds__(256) void k_pack(iamx_tiling_t t, const uint8_t *__restrict__ src, int64_t ld,
-                                              uint8_t *__restrict__ out, int64_t id0) {
-  const int64_t nbpc = t.nblocks[0] * t.nblocks[1];
-  const int64_t id = id0 + blockIdx.x;
-  const int64_t nc = id / nbpc, nb = id % nbpc;
-  const int64_t ci0 = nc / t.nchunks[1], ci1 = nc % t.nchunks[1];
-  const int64_t bi0 = nb / t.nblocks[1], bi1 = nb % t.nblocks[1];
-  const int ts = t.typesize;
-  const int32_t rows = (int32_t)t.block[0], cols = (int32_t)t.block[1];
-  const int32_t n = rows * cols;
-  const int64_t r_in = bi0 * t.block[0], c_in = bi1 * t.block[1];
-  const int64_t gr0 = ci0 * t.chunk[0] + r_in, gc0 = ci1 * t.chunk[1] + c_in;
-  int64_t vr = t.chunk[0] - r_in;
-  if (t.shape[0] - gr0 < vr) vr = t.shape[0] - gr0;
-  int64_t vc = t.chunk[1] - c_in;
-  if (t.shape[1] - gc0 < vc) vc = t.shape[1] - gc0;
-  uint8_t *o = out + id * (int64_t)n * ts;
-  auto elem = [&](int32_t e) -> uint64_t {
-    const int32_t r = e / cols, c = e - (e / cols) * cols;
-    if (r >= vr || c >= vc) return 0;
-    return load_elem(src, ts, (gr0 + r) * ld + gc0 + c);
-  };
-  if (t.filter == IAMX_FILTER_BITSHUFFLE) {
-    const int32_t n8 = n - n % 8, rowlen = n8 / 8;
-    for (int32_t g = threadIdx.x; g < rowlen; g += blockDim.x) {
-      uint64_t v[8];
-      for (int i = 0; i < 8; i++) v[i] = elem(8 * g + i);
-      for (int j = 0; j < ts; j++) {
-        uint64_t x = 0;
-        for (int i = 0; i < 8; i++) x |= ((v[i] >> (8 * j)) & 0xffull) << (8 * i);
-        const uint64_t y = transpose8(x);
-        for (int k = 0; k < 8; k++) o[(int64_t)(8 * j + k) * rowlen + g] = (uint8_t)(y >> (8 * k));
-      }
-    }
-    for (int32_t e = n8 + threadIdx.x; e < n; e += blockDim.x) {
-      const uint64_t v = elem(e);
-      for (int j = 0; j < ts; j++) o[(int64_t)e * ts + j] = (uint8_t)(v >> (8 * j));
-    }
-    return;
-  }
-  const bool shuffled = t.filter == IAMX_FILTER_SHUFFLE && ts > 1;
-  if (shuffled && (ts == 4 || ts == 8)) {
-    // Four consecutive elements per thread, read together where they share a
-    // row inside the valid extent, one by one otherwise; their bytes j form
-    // 4 bytes of plane j (a 4x4 byte transpose per 4 planes), stored as one
-    // dword where it is aligned.
-    for (int32_t q = threadIdx.x; 4 * q < n; q += blockDim.x) {
-      const int32_t e0 = 4 * q;
-      const int32_t ne = min(4, n - e0);
-      const int32_t r = e0 / cols, c = e0 - r * cols;
-      uint32_t lo[4], hi[4] = {0, 0, 0, 0};
-      const int64_t idx = (gr0 + r) * ld + gc0 + c;
-      // vc counts valid columns from the block's first column to the chunk's
-      // (or array's) edge and can pass the block width: the four elements
-      // share a row only when they also end inside the block
-      if (ne == 4 && r < vr && c + 4 <= vc && c + 4 <= cols && ((uint64_t)(src + idx * ts) & 15) == 0) {
-        const IAMX_GLOBAL u32x4 *s = iamx::gptr<const u32x4>((uint64_t)(src + idx * ts));
-        const u32x4 a = s[0];
-        if (ts == 4) {
-          lo[0] = a.x; lo[1] = a.y; lo[2] = a.z; lo[3] = a.w;
-        } else {
-          const u32x4 b = s[1];
-          lo[0] = a.x; hi[0] = a.y; lo[1] = a.z; hi[1] = a.w;
-          lo[2] = b.x; hi[2] = b.y; lo[3] = b.z; hi[3] = b.w;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int32_t e = e0 + i, er = e / cols, ec = e - er * cols;
-          uint64_t v = 0;
-          if (i < ne && er < vr && ec < vc) v = load_elem(src, ts, (gr0 + er) * ld + gc0 + ec);
-          lo[i] = (uint32_t)v;
-          hi[i] = (uint32_t)(v >> 32);
-        }
-      }
-      uint32_t w[8];
-      tr4(lo[0], lo[1], lo[2], lo[3], w);
-      if (ts == 8) tr4(hi[0], hi[1], hi[2], hi[3], w + 4);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        if (j >= ts) continue;
-        uint8_t *d = o + (int64_t)j * n + e0;
-        if (ne == 4 && ((uint64_t)d & 3) == 0) {
-          *iamx::gptr<uint32_t>((uint64_t)d) = w[j];
-        } else {
-          for (int i = 0; i < ne; i++) d[i] = (uint8_t)(w[j] >> (8 * i));
-        }
-      }
-    }
-    return;
-  }
-  for (int32_t e = threadIdx.x; e < n; e += blockDim.x) {
-    const uint64_t v = elem(e);
-    if (shuffled) {
-      for (int j = 0; j < ts; j++) o[(int64_t)j * n + e] = (uint8_t)(v >> (8 * j));
-    } else {
-      for (int j = 0; j < ts; j++) o[(int64_t)e * ts + j] = (uint8_t)(v >> (8 * j));
-    }
-  }
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void k_transpose(int64_t rows, int64_t cols, const T *__restrict__ src,
                                                    T *__restrict__ dst) {
@@ -1136,29 +1020,6 @@ IAMX_API int iamx_decode(const iamx_lz4_job_t *d_lz4, int n_lz4, const iamx_bloc
   if (n_blocks > 0)
     rc = iamx::launch_unfilter(d_blocks, n_blocks, d_scratch, d_dst);
   return rc;
-}
-
-IAMX_API int iamx_pack_blocks_range(const iamx_tiling_t *t, const void *d_src, int64_t src_ld, void *d_out,
-                                    int64_t chunk_begin, int64_t chunk_end) {
-  int rc = iamx::ensure_init();
-  if (rc) return rc;
-  if (!t || t->typesize < 1 || t->typesize > 8 || t->block[0] <= 0 || t->block[1] <= 0)
-    return iamx::set_error(IAMX_EINVAL, "iamx_pack_blocks: bad tiling");
-  const int64_t nchunks = t->nchunks[0] * t->nchunks[1], nbpc = t->nblocks[0] * t->nblocks[1];
-  if (chunk_begin < 0 || chunk_end > nchunks || chunk_begin > chunk_end)
-    return iamx::set_error(IAMX_EINVAL, "iamx_pack_blocks: chunk range [%lld, %lld) outside [0, %lld)",
-                           (long long)chunk_begin, (long long)chunk_end, (long long)nchunks);
-  const int64_t nblk = (chunk_end - chunk_begin) * nbpc;
-  if (nblk == 0) return IAMX_OK;
-  if (nblk < 0 || nblk > INT32_MAX) return iamx::set_error(IAMX_EINVAL, "iamx_pack_blocks: bad block count");
-  IAMX_LAUNCH("pack_blocks", k_pack, dim3((unsigned)nblk), dim3(256), 0, *t, (const uint8_t *)d_src, src_ld,
-              (uint8_t *)d_out, chunk_begin * nbpc);
-  return IAMX_OK;
-}
-
-IAMX_API int iamx_pack_blocks(const iamx_tiling_t *t, const void *d_src, int64_t src_ld, void *d_out) {
-  if (!t) return iamx::set_error(IAMX_EINVAL, "iamx_pack_blocks: bad tiling");
-  return iamx_pack_blocks_range(t, d_src, src_ld, d_out, 0, t->nchunks[0] * t->nchunks[1]);
 }
 
 IAMX_API int iamx_transpose(int typesize, int64_t rows, int64_t cols, const void *d_src, void *d_dst) {

@@ -90,3 +90,60 @@ def test_pack_blocks_matches_numpy(dtype, shape, chunk, block, filt):
         h.iamx_free(d_out)
     bad = np.flatnonzero(got != want)
     assert bad.size == 0, f"{bad.size} bytes differ, first at {bad[:8].tolist()}"
+
+
+def _bitshuffled(raw, ts):
+    """Bit planes of the elements in groups of eight, the last ones as they are."""
+    n = raw.size // ts
+    n8 = n - n % 8
+    bits = np.unpackbits(raw[:n8 * ts].reshape(n8, ts), axis=1, bitorder="little")  # (element, bit)
+    return np.concatenate([np.packbits(bits.T, axis=1, bitorder="little").ravel(), raw[n8 * ts:]])
+
+
+# blocks of one part of eight elements a thread and just more, rows shorter than a set of four, odd lengths, chunks
+# that reach past the array
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.float32, np.float64])
+@pytest.mark.parametrize("shape,chunk,block", [
+    ((33, 1), (17, 1), (5, 1)),
+    ((40, 6), (40, 6), (13, 3)),
+    ((64, 70), (32, 64), (32, 64)),
+    ((131, 101), (100, 100), (41, 50)),
+    ((130, 257), (130, 150), (64, 65)),
+])
+@pytest.mark.parametrize("filt", [0, 1, 2], ids=["none", "shuffle", "bitshuffle"])
+def test_pack_blocks_parts(dtype, shape, chunk, block, filt):
+    print(f"case: pack parts {np.dtype(dtype).name} {shape} {chunk} {block} filter {filt}", flush=True)
+    rng = np.random.default_rng(sum(shape) + sum(block) + filt)
+    ts = np.dtype(dtype).itemsize
+    C = rng.integers(0, 256, (shape[0], shape[1] * ts)).astype(np.uint8).view(dtype)
+    want = _expected(C, chunk, block, 1 if filt == 1 and ts > 1 else 0)
+    bsize = block[0] * block[1] * ts
+    if filt == 2:
+        want = np.concatenate([_bitshuffled(want[i:i + bsize], ts) for i in range(0, want.size, bsize)])
+    h = ctypes.CDLL(ia.HIP_LIB_PATH)
+    h.iamx_malloc.restype = ctypes.c_void_p
+    h.iamx_malloc.argtypes = [ctypes.c_size_t]
+    h.iamx_free.argtypes = [ctypes.c_void_p]
+    h.iamx_h2d.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
+    h.iamx_d2h.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
+    h.iamx_pack_blocks.argtypes = [ctypes.POINTER(Tiling), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    assert h.iamx_init() == 0
+    t = Tiling()
+    for i in range(2):
+        t.shape[i], t.chunk[i], t.block[i] = shape[i], chunk[i], block[i]
+        t.nchunks[i] = _cdiv(shape[i], chunk[i])
+        t.nblocks[i] = _cdiv(chunk[i], block[i])
+    t.typesize, t.filter = ts, filt
+    d_src = h.iamx_malloc(C.nbytes + 64)
+    d_out = h.iamx_malloc(want.nbytes + 64)
+    try:
+        assert d_src and d_out
+        assert h.iamx_h2d(d_src, C.ctypes.data, C.nbytes) == 0
+        assert h.iamx_pack_blocks(ctypes.byref(t), d_src, shape[1], d_out) == 0
+        got = np.empty_like(want)
+        assert h.iamx_d2h(got.ctypes.data, d_out, got.nbytes) == 0
+    finally:
+        h.iamx_free(d_src)
+        h.iamx_free(d_out)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, f"{bad.size} bytes differ, first at {bad[:8].tolist()}"
