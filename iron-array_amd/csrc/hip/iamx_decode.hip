@@ -149,8 +149,8 @@ struct Lz4Geom<1> {
 // What bounds it where streams are few is the chain from round to round (about
 // 5200 cycles for 8 windows: header reads, 5 hops of pointer doubling, the
 // exits, the scans, the table, the sources), so its time falls with the windows
-// a round takes: a 250 KB bitshuffled float32 stream takes 443 us with one
-// wavefront, 205 with 4, 136 with 8; one sequence after the other, with 64
+// a round takes: a 250 KB bitshuffled float32 stream takes 451 us with one
+// wavefront, 205 with 4, 134 with 8; one sequence after the other, with 64
 // lanes copying each, took 783.  With four streams a CU it is vector issue (78%
 // of the cycles).  So a round's cost is its instructions and its waits:
 //  - LDS words at any byte offset are two aligned reads and a byte align; one
@@ -184,7 +184,7 @@ struct Lz4Geom<1> {
 // wavefront before a barrier that precedes the read.
 template <int NW>
 __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__restrict__ scratch, int *status,
-                                           uint8_t *lds) {
+                                           uint8_t *lds, int32_t ahead_at) {
   using G = Lz4Geom<NW>;
   constexpr int32_t NT = G::kThreads;
   constexpr int32_t RING = G::kRing, RM = RING - 1;
@@ -231,6 +231,20 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
     flushed = __builtin_amdgcn_readfirstlane(cur & ~15);
     flush_at = flushed + FLUSH_AT;
   };
+
+  // Wavefronts with more input left go first.  Streams that share a CU then end
+  // together, the long ones of unlike streams and all of equal ones, and none
+  // is left to decode with the CU to itself: 1024 exponent planes 426 to 366 us,
+  // 6400 of them 1733 to 1540; 1024 bitshuffled streams of 33 to 85 rounds 396
+  // to 340.
+  auto rank = [&](int32_t at) {
+    const int32_t left = iend - at;
+    if (left > ahead_at) __builtin_amdgcn_s_setprio(3);
+    else if (left > ahead_at >> 1) __builtin_amdgcn_s_setprio(2);
+    else if (left > ahead_at >> 2) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+  };
+  rank(ip);
 
   int bad = 0;
   bool general = false;
@@ -399,7 +413,10 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             put_stage(have, ahead);
             have += 256;
           }
-          if (op >= flush_at) flush(op);
+          if (op >= flush_at) {
+            flush(op);
+            rank(ip);
+          }
           if (stopped) {
             general = true;
             break;
@@ -601,7 +618,10 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
             lds_barrier();
           }
           op += total;
-          if (op >= flush_at) flush(op);
+          if (op >= flush_at) {
+            flush(op);
+            rank(base);
+          }
           if (stop >= 0) {
             ip = base + stop;
             if (general) break;
@@ -953,7 +973,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 1
     if (threadIdx.x == 0) atomicOr(status, 1 << 1);
     return;
   }
-  lz4_stream<NW>(job, scratch, status, lds);
+  // half the first job's input (the longest where they are sorted), or of a typical long one
+  const int32_t ahead_at = min(jobs[0].csize / 2, 24576);
+  lz4_stream<NW>(job, scratch, status, lds, ahead_at);
 }
 
 template <typename T>
@@ -980,22 +1002,25 @@ namespace iamx {
 // Wavefronts per stream, by how many streams a CU gets.  A stream's time is set
 // by its own chain of rounds, so few streams are spread over many wavefronts
 // each; many streams hide each other's waits, and one wavefront decodes a
-// sequence with the fewest instructions.  The lines are where a CU still holds
-// all of its streams at once (4 x 8 and 8 x 4 wavefronts).  Measured in us with
-// 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250 KB: 4 streams
-// 136 / 205 / 443, 1024 streams 306 / 352 / 667, 2048 streams 545 / 536 / 732,
-// 3072 streams - / 762 / 803, 4096 streams - / 913 / 914, 6400 streams with one
-// 1266; exponent planes of float32 (64 KB): 4 streams 219 / 383 / 875, 1024
-// streams 429 / 528 / 1027, 2048 streams 791 / 765 / 1113, 3072 streams - /
-// 1125 / 1204, 4096 streams - / 1412 / 1303; byte planes of 16 KB of float64:
-// 2048 streams 185 / 175 / 239, 3072 streams - / 250 / 258; short ones (700
-// bytes): 3072 streams - / 151 / 121.
+// sequence with the fewest instructions.  The first line is where a CU still
+// holds all of its streams at once with 8 wavefronts (4 x 8), the second where
+// 4 wavefronts, in one and a half loads of a CU (8 x 4), are overtaken.
+// Measured in us with 8 / 4 / 1 wavefronts on bitshuffled float32 streams of 250
+// KB: 4 streams 134 / 205 / 451, 1024 streams 290 / 332 / 606, 1280 streams 392
+// / 366, 2048 streams 521 / 471 / 675, 3072 streams - / 745 / 743, 4096 streams
+// - / 852 / 828, 6400 streams - / 1381 / 1076; exponent planes of float32 (64
+// KB): 4 streams 222 / 387 / 891, 1024 streams 371 / 500 / 1038, 1280 streams
+// 556 / 540, 2048 streams 706 / 658 / 1116, 3072 streams - / 1090 / 1194, 4096
+// streams - / 1267 / 1273, 6400 streams - / 2101 / 1550; a ragged matrix's
+// bitshuffled float64 streams: 3072 streams - / 510 / 1011, equal ones - / 282 /
+// 232; byte planes of 16 KB of float64: 3072 streams - / 244 / 255, 4096 streams
+// - / 292 / 275.
 int launch_lz4(const char *name, const iamx_lz4_job_t *d_lz4, int n_lz4, void *d_scratch, int64_t cap) {
   const int z = zstd_enabled() ? 1 : 0;
   if (n_lz4 <= 4 * g_num_cus)
     IAMX_LAUNCH(name, k_lz4_streams<8>, dim3(n_lz4), dim3(512), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
                 status_word(), z);
-  else if (n_lz4 <= 8 * g_num_cus)
+  else if (n_lz4 <= 12 * g_num_cus)
     IAMX_LAUNCH(name, k_lz4_streams<4>, dim3(n_lz4), dim3(256), 0, d_lz4, n_lz4, (uint8_t *)d_scratch, cap,
                 status_word(), z);
   else

@@ -400,6 +400,23 @@ def test_crafted_lz4_dense_rounds(ctx, orc, plan, copies):
     assert got == b"".join(want[i % 3] for i in range(copies))
 
 
+# more than 12 streams a CU: one wavefront each
+@pytest.mark.parametrize("plan", sorted({**ROUND_PLANS, **DENSE_PLANS}))
+def test_crafted_lz4_one_wavefront(ctx, orc, plan):
+    print(f"case: crafted lz4, one wavefront, {plan}", flush=True)
+    lits, offs, mls = {**ROUND_PLANS, **DENSE_PLANS}[plan]
+    c = ia.Context(clevel=5, filters=0)
+    chunks, want = [], []
+    for n in [31_001, 6_144, 30_003]:
+        rng = np.random.default_rng(zlib.crc32(plan.encode()) + n)
+        stream, raw = _craft_lz4(rng, n, lambda r: (_choice(r, lits), _choice(r, offs), _choice(r, mls)))
+        assert orc.lz4_decode(stream, n) == raw
+        chunks.append(_one_stream_chunk(c, stream, n))
+        want.append(raw)
+    got = ia.decode_chunks_flat(c, [chunks[i % 3] for i in range(3200)], sum(len(want[i % 3]) for i in range(3200)))
+    assert got == b"".join(want[i % 3] for i in range(3200))
+
+
 @pytest.mark.parametrize("copies", [3, 1100, 2100])
 def test_corrupt_stream_among_many(ctx, orc, copies):
     rng = np.random.default_rng(copies)
