@@ -105,7 +105,7 @@ struct Lz4Geom<1> {
   static constexpr int kThreads = 64;
   static constexpr int kRing = 4096;
   static constexpr int kOut = 1024;
-  static constexpr int kStep = 512;
+  static constexpr int kStep = 256;
   static constexpr int kStage = 1024;  // a ring, its first bytes repeated after its end
   static constexpr int kSeqs = 64;
   static constexpr int kTabAt = kRing + kStage + 16;
@@ -176,13 +176,25 @@ struct Lz4Geom<1> {
 // well, several wavefronts stay there (a bitshuffled float32 stream 136 to 133
 // us, one of a matrix's last rows 102 to 94; nothing with one wavefront).
 //
+// Many streams of one kind are all in the same place at once: bitshuffled ones
+// begin with their lowest planes, a literal run of half the stream, and wait for
+// HBM together, and then leave it idle while they decode rounds.  So with one
+// wavefront a stream that begins with a run of 8 KB or more, or is of 64 KB or
+// more compressed (SIDEWAYS), copies only what the ring has to hold of such a
+// run and moves the rest a little in every round: 4096 streams of an 8000^2
+// float64 matrix 320 to 303 us, 9216 of a 12000^2 float32 one 422 to 385, 10800
+// of normal float32 values in blocks of 100^2 275 to 221; nothing where streams
+// differ and overlap by themselves (20000^2 float32, 1290).  By the first run
+// alone the float64 ones took 342: some moved, some not.  In a body of its own:
+// other streams took 2 to 4% longer in one for both.
+//
 // Output bytes go to an LDS ring and reach the stream's scratch slot in
 // 16-byte stores whenever a quarter of the ring is pending.  An offset of more
 // than kNear reads the slot back from global memory: such a source is at least
 // 15/16 of the ring back, at most 5/16 of the ring is pending or was flushed
 // last, and the stores of the flush before that were waited for by every
 // wavefront before a barrier that precedes the read.
-template <int NW>
+template <int NW, bool SIDEWAYS = false>
 __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__restrict__ scratch, int *status,
                                            uint8_t *lds, int32_t ahead_at) {
   using G = Lz4Geom<NW>;
@@ -232,6 +244,38 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
     flush_at = flushed + FLUSH_AT;
   };
 
+  // SIDEWAYS: what is left of a long literal run is moved by the rounds after it,
+  // SIDE bytes each.  Bytes of the run, moved or not, are read from the input.
+  constexpr int32_t SIDE = 1024;
+  int32_t side_n = 0, side_src = 0, side_dst = 0;  // bytes left, from where, to where
+  int32_t run_at = 0, run_n = 0, run_in = 0;       // the run's output bytes, and input less output position
+  auto side_load = [&](int32_t i) -> u32x4 { return *(const IAMX_GLOBAL u32x4_any *)(sb + side_src + i); };
+  auto side_store = [&](int32_t i, u32x4 w) { *iamx::gptr<u32x4>((uint64_t)(dst + side_dst + i)) = w; };
+  auto side_finish = [&]() {
+    for (int32_t i = 16 * lane; i < side_n; i += 2 * SIDE) {
+      const bool two = i + SIDE < side_n;
+      const u32x4 a = side_load(i);
+      u32x4 b;
+      if (two) b = side_load(i + SIDE);
+      side_store(i, a);
+      if (two) side_store(i + SIDE, b);
+    }
+    side_n = 0;
+  };
+  // a byte that a flush wrote, or of the run; it has arrived
+  auto slot_byte = [&](int32_t at) -> uint32_t {
+    uint32_t v;
+    if (SIDEWAYS && run_n > 0) {
+      const bool in_run = (uint32_t)(at - run_at) < (uint32_t)run_n;
+      v = *(in_run ? sb + at + run_in : (const IAMX_GLOBAL uint8_t *)dst + at);
+      asm volatile("" : "+v"(v));
+    } else {
+      v = dst[at];
+      asm volatile("" : "+v"(v));
+    }
+    return v;
+  };
+
   // Wavefronts with more input left go first.  Streams that share a CU then end
   // together, the long ones of unlike streams and all of equal ones, and none
   // is left to decode with the CU to itself: 1024 exponent planes 426 to 366 us,
@@ -279,6 +323,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           const bool more = have - ip < 768;
           uint32_t ahead = 0;
           if (more) ahead = ld_word(have, lane);
+          u32x4 side;
+          if (SIDEWAYS && side_n > 0) side = side_load(16 * lane);
           if (lane < G::kOut / 32) obits[lane] = 0;
           // walk: the starts of up to three windows, listed by position
           int32_t n = 0, at = ip;  // sequences so far, the next one's position
@@ -383,10 +429,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
               if (x1 < total) e = entry_of(x1);
               // at most FLUSH_AT + kOut bytes are pending, so a far source was
               // flushed, by this wavefront's own stores
-              if (odd & (off > NEAR1)) {
-                v = dst[sp];
-                asm volatile("" : "+v"(v));  // arrived, here and not where the paths meet
-              }
+              if (odd & (off > NEAR1)) v = slot_byte(sp);  // arrived, here and not where the paths meet
               const bool dep = odd & (off <= lane);
               if (ballot(dep)) {
                 // bit 6: the lane has its own byte
@@ -412,6 +455,12 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           if (more) {
             put_stage(have, ahead);
             have += 256;
+          }
+          if (SIDEWAYS && side_n > 0) {
+            side_store(16 * lane, side);
+            side_src += SIDE;
+            side_dst += SIDE;
+            side_n -= SIDE;
           }
           if (op >= flush_at) {
             flush(op);
@@ -676,8 +725,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
     // goes out first, then whole 16-byte groups are stored to the slot, the
     // next groups' bytes asked for before the last ones are stored; the last
     // RING bytes also go to the ring.  byte_of and group_of give byte i and
-    // bytes i .. i + 15 of the n.
-    auto bulk = [&](int32_t n, auto byte_of, auto group_of) {
+    // bytes i .. i + 15 of the n; groups before g0 are left out.
+    auto bulk = [&](int32_t n, int32_t g0, auto byte_of, auto group_of) {
       flush(op);
       if (tid < op - flushed) dst[flushed + tid] = ring[(flushed + tid) & RM];
       lds_barrier();  // the ring is written below
@@ -706,8 +755,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         }
       };
       u32x4 wa, wb;
-      if (tid < ng) wa = group_of(head + 16 * tid);
-      for (int32_t g = tid; g < ng; g += 2 * NT) {
+      if (g0 + tid < ng) wa = group_of(head + 16 * (g0 + tid));
+      for (int32_t g = g0 + tid; g < ng; g += 2 * NT) {
         if (g + NT < ng) wb = group_of(head + 16 * (g + NT));
         group_store(g, wa);
         if (g + 2 * NT < ng) wa = group_of(head + 16 * (g + 2 * NT));
@@ -756,8 +805,20 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       } else {
         look(ip + lit);  // for what follows the run
         const IAMX_GLOBAL uint8_t *from = sb + ip;
+        int32_t g0 = 0;
+        if (SIDEWAYS && wide) {
+          const int32_t head = (16 - (op & 15)) & 15, before = (lit - RING - head) & ~(SIDE - 1);
+          if (before >= 4 * SIDE) {
+            side_finish();
+            side_n = run_n = before;
+            side_src = ip + head;
+            side_dst = run_at = op + head;
+            run_in = ip - op;
+            g0 = before >> 4;
+          }
+        }
         bulk(
-            lit, [&](int32_t i) -> uint8_t { return from[i]; },
+            lit, g0, [&](int32_t i) -> uint8_t { return from[i]; },
             [&](int32_t i) -> u32x4 { return *(const IAMX_GLOBAL u32x4_any *)(from + i); });
         ip += lit;
       }
@@ -782,7 +843,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
         w[t] = rdlane(b, 4 * t) | (rdlane(b, 4 * t + 1) << 8) | (rdlane(b, 4 * t + 2) << 16) | (rdlane(b, 4 * t + 3) << 24);
       const int32_t op0 = op;
       bulk(
-          ml,
+          ml, 0,
           [&](int32_t i) -> uint8_t {
             const int32_t j = (op0 + i) & 15;
             const uint32_t lo = j & 4 ? w.y : w.x, hi = j & 4 ? w.w : w.z;
@@ -792,6 +853,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
       general = NW > 1 && long_next();
       continue;
     }
+    if (SIDEWAYS && off > NEAR) side_finish();
     // kStep bytes a step: byte i of a step is byte (i mod off) of the `off`
     // bytes before the step
     {
@@ -825,6 +887,7 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
   }
   if (!bad && op != oend) bad = 7;
   if (!bad) {  // the slot is padded to 4 bytes at least
+    if (SIDEWAYS) side_finish();
     flush(oend);
     const int32_t p = flushed + 4 * tid;
     if (p < oend) dstw[p >> 2] = *reinterpret_cast<const uint32_t *>(ring + (p & RM));
@@ -975,6 +1038,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 1
   }
   // half the first job's input (the longest where they are sorted), or of a typical long one
   const int32_t ahead_at = min(jobs[0].csize / 2, 24576);
+  if constexpr (NW == 1) {  // long, or a literal run of 8 KB or more to begin with (32 length bytes of 255)
+    const uint8_t *in = reinterpret_cast<const uint8_t *>(job.src);
+    const int i = min((int)threadIdx.x, 32);
+    if (job.csize >= 65536 || (job.csize > 8192 && ballot(in[i] < (i ? 255 : 0xf0)) == 0)) {
+      lz4_stream<1, true>(job, scratch, status, lds, ahead_at);
+      return;
+    }
+  }
   lz4_stream<NW>(job, scratch, status, lds, ahead_at);
 }
 

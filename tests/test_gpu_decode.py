@@ -417,6 +417,36 @@ def test_crafted_lz4_one_wavefront(ctx, orc, plan):
     assert got == b"".join(want[i % 3] for i in range(3200))
 
 
+# streams that begin with a literal run of 8 KB or more, which a wavefront of its own moves beside the rounds, with
+# sources in the run, in its last 4 KB and after it; runs that follow before the first is moved, and long matches
+# that read it
+@pytest.mark.parametrize("copies", [3, 3200])
+@pytest.mark.parametrize("first", [8174, 8175, 8191, 12_299, 16_384, 40_001])
+def test_crafted_lz4_long_run_first(ctx, orc, first, copies):
+    print(f"case: crafted lz4 run of {first} first x {copies}", flush=True)
+    c = ia.Context(clevel=5, filters=0)
+    chunks, want = [], []
+    for n, every in [(first + 700, 10 ** 9), (first + 15_003, 10 ** 9), (first + 30_016, 200)]:
+        rng = np.random.default_rng(first + n)
+        at = [0]
+
+        def pick(r):
+            at[0] += 1
+            if at[0] == 1:
+                return first, int(r.integers(1, first)), 40
+            if at[0] % every == 0:
+                return int(r.integers(9000, 14_000)), int(r.integers(5000, 65_535)), int(r.integers(300, 5000))
+            return (_choice(r, [(0, 3), (0, 20)]), _choice(r, [(1, 80), (3900, 4200), (4200, 65_535)]),
+                    _choice(r, [(4, 30), (4, 270)]))
+
+        stream, raw = _craft_lz4(rng, n, pick)
+        assert orc.lz4_decode(stream, n) == raw
+        chunks.append(_one_stream_chunk(c, stream, n))
+        want.append(raw)
+    got = ia.decode_chunks_flat(c, [chunks[i % 3] for i in range(copies)], sum(len(want[i % 3]) for i in range(copies)))
+    assert got == b"".join(want[i % 3] for i in range(copies))
+
+
 @pytest.mark.parametrize("copies", [3, 1100, 2100])
 def test_corrupt_stream_among_many(ctx, orc, copies):
     rng = np.random.default_rng(copies)
