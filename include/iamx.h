@@ -33,6 +33,8 @@ enum {
 IAMX_API int iamx_init(void);
 IAMX_API const char *iamx_last_error(void);
 IAMX_API int iamx_device_info(char *name, int namelen, int *cus, char *arch, int archlen);
+/* iamx_free keeps blocks of up to 64 MiB (256 MiB in all) for later calls of
+ * iamx_malloc, once the device has finished the work queued before it. */
 IAMX_API void *iamx_malloc(size_t bytes);
 IAMX_API void iamx_free(void *dptr);
 IAMX_API int iamx_h2d(void *dst, const void *src, size_t bytes);
