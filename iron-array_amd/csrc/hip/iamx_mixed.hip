@@ -261,35 +261,40 @@ struct CrtMods {
 // most 52 bits, so a - m rint(a/m) is exact, and as the quotient is off by at
 // most one next to a half its magnitude is at most 128: only +128 needs
 // bringing back into an int8 (any residue of the class gives the exact product
-// modulo m, and 131071 products of 128^2 stay below 2^31).  6000x6000 operands
-// with 13 moduli read 0.29 GB and write 0.47 in 167 (A) and 260 us (B, through
-// the LDS tile); both ends brought back in FP64 took 229 and 281.  A tile kept
-// column by column in LDS measured the same (264).
+// modulo m, and 131071 products of 128^2 stay below 2^31).
+//
+// Bound by HBM: 6000x6000 operands with 13 moduli read 0.29 GB and write 0.47 in
+// 147 (A) and 170 us (B).  Both ends brought back in FP64 took 229 and 281; B
+// turned round through an LDS tile that the kernel for A held as well 167 and
+// 260.  What the stores of B's wavefronts cover decides: lines of 8 rows 170 us,
+// half lines of 16 rows 183, 16 bytes of 32 rows 237, of 64 rows 318.
+template <bool TRANS>
 __global__ __launch_bounds__(256) void k_residues_i8(const double *__restrict__ X, int64_t xr, int64_t xc,
-                                                     int64_t ldx, int trans, const int32_t *__restrict__ e, int scale,
+                                                     int64_t ldx, const int32_t *__restrict__ e, int scale,
                                                      const CrtMods mods, int8_t *__restrict__ planes, int64_t rows_p,
                                                      int64_t cols_p) {
   // a workgroup makes 32 plane rows x 128 plane columns (rows_p a multiple
-  // of 32, cols_p of 128); a thread 4 consecutive columns of 4 rows, stored
-  // as one dword per modulus
-  __shared__ double t[128][33];
+  // of 32, cols_p of 128).  A thread makes 4 consecutive columns of 4 rows, or
+  // where X lies the other way 16 consecutive columns of one row: a wavefront's
+  // 16-byte stores fill whole lines of 8 rows, its loads take 64 bytes of 16
+  // rows of X for each column.
+  constexpr int G = TRANS ? 16 : 4;
+  typedef uint32_t words __attribute__((ext_vector_type(G / 4)));
   const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = (int64_t)blockIdx.x * 128;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  if (trans) {
-    for (int i = ty; i < 128; i += 8) {
-      const int64_t xrow = c0 + i, xcol = r0 + tx;
-      t[i][tx] = (xrow < xr && xcol < xc) ? X[xrow * ldx + xcol] : 0.0;
-    }
-    __syncthreads();
-  }
+  const int wave = threadIdx.x >> 6;
+  const int tx = TRANS ? (threadIdx.x & 7) + 8 * wave : threadIdx.x & 31;
+  const int ty = TRANS ? (threadIdx.x >> 3) & 7 : threadIdx.x >> 5;
   const int64_t plane = rows_p * cols_p;
-  const int64_t c = c0 + 4 * tx;
-  for (int i = ty; i < 32; i += 8) {
+  const int64_t c = c0 + G * (TRANS ? ty : tx);
+  for (int i = TRANS ? tx : ty; i < 32; i += TRANS ? 32 : 8) {
     const int64_t r = r0 + i;
     if (r >= rows_p || c >= cols_p) continue;
-    const int er = r < (trans ? xc : xr) ? e[r] : 0;
-    double a[4];
-    if (!trans && r < xr && c + 4 <= xc) {  // inside: two 16-byte loads
+    const int er = r < (TRANS ? xc : xr) ? e[r] : 0;
+    double a[G];
+    if (TRANS) {
+#pragma unroll
+      for (int k = 0; k < G; k++) a[k] = c + k < xr && r < xc ? X[(c + k) * ldx + r] : 0.0;
+    } else if (r < xr && c + 4 <= xc) {  // inside: two 16-byte loads
       const double2_any *x = reinterpret_cast<const double2_any *>(X + r * ldx + c);
       const double2_any x0 = x[0], x1 = x[1];
       a[0] = x0.x;
@@ -298,21 +303,25 @@ __global__ __launch_bounds__(256) void k_residues_i8(const double *__restrict__ 
       a[3] = x1.y;
     } else {
 #pragma unroll
-      for (int k = 0; k < 4; k++)
-        a[k] = trans ? t[4 * tx + k][i] : ((r < xr && c + k < xc) ? X[r * ldx + c + k] : 0.0);
+      for (int k = 0; k < G; k++) a[k] = r < xr && c + k < xc ? X[r * ldx + c + k] : 0.0;
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) a[k] = rint(ldexp(a[k], scale - er));
+    for (int k = 0; k < G; k++) a[k] = rint(ldexp(a[k], scale - er));
     for (int l = 0; l < mods.n; l++) {
       const double m = (double)mods.m[l];
-      uint32_t word = 0;
+      words w;
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        int32_t res = (int32_t)fma(-m, rint(a[k] * mods.inv[l]), a[k]);
-        res -= res > 127 ? mods.m[l] : 0;
-        word |= (uint32_t)(uint8_t)res << (8 * k);
+      for (int g = 0; g < G / 4; g++) {
+        uint32_t word = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          int32_t res = (int32_t)fma(-m, rint(a[4 * g + k] * mods.inv[l]), a[4 * g + k]);
+          res -= res > 127 ? mods.m[l] : 0;
+          word |= (uint32_t)(uint8_t)res << (8 * k);
+        }
+        w[g] = word;
       }
-      *reinterpret_cast<uint32_t *>(planes + (int64_t)l * plane + r * cols_p + c) = word;
+      *reinterpret_cast<words *>(planes + (int64_t)l * plane + r * cols_p + c) = w;
     }
   }
 }
@@ -1064,8 +1073,8 @@ static int mixed_prepare_b(PrepB &pb, int slot, int form, int64_t N, int64_t K, 
                 dim3((unsigned)((N + 63) / 64), (unsigned)((K + kColSlab - 1) / kColSlab)), dim3(256), 0, Bd, K, N,
                 ldb, fb);
     IAMX_LAUNCH("ozaki_col_exp", k_col_exp_zero, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, fb, N);
-    IAMX_LAUNCH("ozaki_crt_residues_B", k_residues_i8, dim3((unsigned)(Kp / 128), (unsigned)(Np / 32)), dim3(256), 0,
-                Bd, K, N, ldb, 1, fb, q + 1, crt_mods(S), (int8_t *)ws, Np, Kp);
+    IAMX_LAUNCH("ozaki_crt_residues_B", k_residues_i8<true>, dim3((unsigned)(Kp / 128), (unsigned)(Np / 32)), dim3(256), 0,
+                Bd, K, N, ldb, fb, q + 1, crt_mods(S), (int8_t *)ws, Np, Kp);
     pb = PrepB{3, N, K, Np, Kp, S, ws, fb, true, p, q};
     return IAMX_OK;
   }
@@ -1157,8 +1166,8 @@ static int mixed_rows(const PrepB &pb, int form, int64_t M, const void *A, int64
     uint8_t *R = ws + rup((int64_t)(a_bytes + (size_t)Mp * 4), 256);
     const double *Ad = (const double *)A;
     IAMX_LAUNCH("ozaki_row_exp", k_row_exp, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, Ad, M, K, lda, ea);
-    IAMX_LAUNCH("ozaki_crt_residues_A", k_residues_i8, dim3((unsigned)(Kp / 128), (unsigned)(Mp / 32)), dim3(256), 0,
-                Ad, M, K, lda, 0, ea, pb.p + 1, crt_mods(n), (int8_t *)ws, Mp, Kp);
+    IAMX_LAUNCH("ozaki_crt_residues_A", k_residues_i8<false>, dim3((unsigned)(Kp / 128), (unsigned)(Mp / 32)), dim3(256), 0,
+                Ad, M, K, lda, ea, pb.p + 1, crt_mods(n), (int8_t *)ws, Mp, Kp);
     P.A = ws;
     P.lda = Kp;
     P.ldb = Kp;

@@ -227,6 +227,21 @@ def test_ozaki_crt_column_edges(N, moduli, monkeypatch):
         assert np.array_equal(c, a @ b), tile
 
 
+@pytest.mark.parametrize("K", [1, 15, 16, 17, 127, 129, 260])
+@pytest.mark.parametrize("N", [7, 9, 33])
+def test_ozaki_crt_depth_edges(K, N):
+    """B's residues take 16 rows of B a thread and 8 of its columns a wavefront:
+    exact integer products around both."""
+    ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
+    rng = np.random.default_rng(K + N)
+    a = rng.integers(-500, 501, (21, K)).astype(np.float64)
+    b = rng.integers(-500, 501, (K, N)).astype(np.float64)
+    ca = ia.Container.from_numpy(ctx, a, (21, K), (10, min(K, 40)))
+    cb = ia.Container.from_numpy(ctx, b, (K, N), (min(K, 40), N))
+    c = ia.matmul(ca, cb, (21, N), (10, N), precision=ia.OZAKI_CRT, slices=13).to_numpy()
+    assert np.array_equal(c, a @ b)
+
+
 def test_ozaki_exact_on_small_integers(orc):
     """Integers below 2^7 are one slice: every form must be exact."""
     ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
