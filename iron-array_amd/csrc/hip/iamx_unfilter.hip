@@ -399,8 +399,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
     if (J.nstreams == ts) return P.is_const[j] ? P.fill[j] : P.ptr[j][e];
     return P.is_const[0] ? P.fill[0] : P.ptr[0][(int64_t)j * n + e];
   };
+  // (a tile may name more than the block's n elements: those there are)
+  const int32_t wcols = shuffled ? min(J.vcols, cols) : J.vcols;
   for (int32_t r = blockIdx.y * (kThreads / 64) + threadIdx.x / 64; r < J.vrows; r += kThreads / 64 * gridDim.y) {
-    for (int32_t c = threadIdx.x % 64; c < J.vcols; c += 64) {
+    for (int32_t c = threadIdx.x % 64; c < wcols; c += 64) {
+      if ((int64_t)r * cols + c >= n) break;
       const int32_t e = r * cols + c;
       uint64_t v = 0;
       if (shuffled) {
