@@ -37,6 +37,28 @@ def test_unfilter_shapes(case, dt, filters):
     assert c.transpose().to_numpy().tobytes() == np.ascontiguousarray(a.T).tobytes()
 
 
+
+# unfiltered and bit-shuffled blocks in a stream a byte of the elements: whole groups of eight and not, groups of four
+# elements across a stream's end, streams and blocks of one byte throughout, blocks of fewer than four elements
+@pytest.mark.parametrize("split", [ia.ALWAYS_SPLIT, ia.NEVER_SPLIT], ids=["split", "one"])
+@pytest.mark.parametrize("filters", [ia.COMP_SHUFFLE, ia.COMP_BITSHUFFLE, 0], ids=["bytes", "bits", "none"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,block", [((96, 64), (32, 32)), ((70, 66), (35, 22)), ((60, 63), (20, 21)),
+                                         ((5, 9000), (5, 4104)), ((2017, 8), (2017, 8)), ((24, 26), (1, 2)),
+                                         ((33, 40), (3, 1)), ((520, 528), (8, 8))])
+def test_unfilter_split_streams(shape, block, dt, filters, split):
+    print(f"case: unfilter {shape} blocks {block} {np.dtype(dt).name} filters {filters} split {split}", flush=True)
+    rng = np.random.default_rng(shape[0] + block[0])
+    a = rng.standard_normal(shape).astype(dt)
+    a[: shape[0] // 3] = np.round(a[: shape[0] // 3])
+    a[shape[0] // 2:, : shape[1] // 2] = np.frombuffer(b"\x2a" * 8, dt)[0]
+    a[-1:] = 0
+    ctx = ia.Context(clevel=5, filters=filters, splitmode=split)
+    c = ia.Container.from_numpy(ctx, a, shape, block)
+    assert c.to_numpy().tobytes() == a.tobytes()
+    assert c.transpose().to_numpy().tobytes() == np.ascontiguousarray(a.T).tobytes()
+
+
 class _Job(ctypes.Structure):
     """iamx_block_job_t"""
     _fields_ = [("src", ctypes.c_uint64 * 8), ("kind", ctypes.c_uint8 * 8), ("fill", ctypes.c_uint8 * 8),
