@@ -20,6 +20,8 @@
 // sum is the same whichever workgroup forms it).  Row sums land in
 // partial[block column][row]; a second launch adds the block columns in
 // order, so y is bit-identical run to run.
+#include <algorithm>
+
 #include "iamx_internal.h"
 
 namespace {
@@ -314,8 +316,12 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
   const int32_t n8 = filter == IAMX_FILTER_BITSHUFFLE ? n - n % 8 : n;
   const int32_t rowlen = n8 / 8;
   // this workgroup's share of the block's rows
-  const int32_t rfirst = (int32_t)((int64_t)vrows * blockIdx.y / gridDim.y);
-  const int32_t rlast = (int32_t)((int64_t)vrows * (blockIdx.y + 1) / gridDim.y);
+  int32_t rfirst = 0, rlast = vrows;
+  if (gridDim.y > 1) {
+    const uint32_t y = blockIdx.y, each = (uint32_t)vrows / gridDim.y, more = (uint32_t)vrows % gridDim.y;
+    rfirst = (int32_t)(y * each + min(y, more));
+    rlast = rfirst + (int32_t)(each + (y < more ? 1 : 0));
+  }
   if (rfirst >= rlast) return;
   if (bits && J.nstreams == 1 && S.ptr[0] != nullptr && cols >= 32 && n8 >= 32 && ts == (int)sizeof(T)) {
     quad_path<T>(S.ptr[0], n, n8, rowlen, cols, rfirst, rlast, vcols, xs, p0, p1, partial + (int64_t)bcol * M, row0, M);
@@ -373,6 +379,7 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
     return;
   }
 
+  const bool plain = !bits && !split_planes && ts == (int)sizeof(T);
   for (int32_t ra = rfirst; ra < rlast; ra += rows_per_win) {
     const int32_t rb = min(rlast, ra + rows_per_win);
     const int32_t g0 = (ra * cols) / 8, g1 = (rb * cols - 1) / 8;  // groups [g0, g1]
@@ -380,7 +387,28 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const iamx_block_job_t *__re
     for (int32_t g = g0 + tid; g <= g1; g += 256) {
       const int32_t e0 = 8 * g;
       uint64_t v[8];
-      if (bits && e0 + 8 <= n8) {
+      // unfiltered elements of one stream, all eight there: wide loads at any
+      // address (byte by byte 12 wavefronts a CU evict one another's lines: a
+      // 4096^2 float64 matrix 407 us, so 40)
+      const IAMX_GLOBAL uint8_t *at = nullptr;
+      if (plain && e0 + 8 <= n) {
+        const int32_t ne = one_stream ? n * ts : neblock;
+        const int32_t s = one_stream ? 0 : e0 * ts / ne, o = e0 * ts - s * ne;
+        if (S.ptr[s] && o + 8 * ts <= ne) at = S.ptr[s] + o;
+      }
+      if (at) {
+#pragma unroll
+        for (int h = 0; h < (int)sizeof(T) / 2; h++) {
+          const u32x4_any w = *(const IAMX_GLOBAL u32x4_any *)(at + 16 * h);
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            const int k = 4 * h + t;  // word k of the eight elements
+            if (sizeof(T) == 4) v[k] = w[t];
+            else if (k & 1) v[k / 2] |= (uint64_t)w[t] << 32;
+            else v[k / 2] = w[t];
+          }
+        }
+      } else if (bits && e0 + 8 <= n8) {
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = 0;
         for (int j = 0; j < ts; j++) {
@@ -467,7 +495,7 @@ __global__ __launch_bounds__(256) void k_zero_words(uint32_t *__restrict__ p, in
 // check every job against them (IAMX_STATUS_RANGE).
 int gemv_fused_launch(int dtype, const iamx_lz4_job_t *d_lz4, int n_lz4, const iamx_block_job_t *d_blocks,
                       const int32_t *d_blk_rc, int n_blocks, int nbc, const void *x, void *y, int64_t M, int64_t K,
-                      int64_t cap, void *d_scratch, void *d_partial, const uint8_t *d_xzero = nullptr) {
+                      int64_t cap, void *d_scratch, void *d_partial, int64_t block, const uint8_t *d_xzero = nullptr) {
   if (n_lz4 > 0) {
     const int rc = iamx::launch_lz4("lz4_streams_gemv", d_lz4, n_lz4, d_scratch, cap);
     if (rc) return rc;
@@ -475,9 +503,13 @@ int gemv_fused_launch(int dtype, const iamx_lz4_job_t *d_lz4, int n_lz4, const i
   const dim3 rgrid((unsigned)((M + 255) / 256));
   int *st = iamx::status_word();
   // enough workgroups for 4 a CU (what the LDS holds), up to 16 to a block: the
-  // four 250x250 blocks of a 500x500 matrix took 36 us with one each
-  const int share = n_blocks >= 4 * iamx::g_num_cus ? 1 : (4 * iamx::g_num_cus + n_blocks - 1) / n_blocks;
-  const dim3 bgrid((unsigned)n_blocks, (unsigned)(share < 16 ? share : 16));
+  // four 250x250 blocks of a 500x500 matrix took 36 us with one each.  None has
+  // less than 4096 elements, 128 groups of 32 for its 256 threads: below that its
+  // own way in costs more than it takes over (float64 blocks of 70^2 22 us shared
+  // by 11, 11.6 by one; of 125^2 64 by 8, 57 by 3)
+  const int64_t want = ((int64_t)4 * iamx::g_num_cus + n_blocks - 1) / n_blocks;
+  const int64_t share = std::max<int64_t>(std::min<int64_t>({want, block / 4096, 16}), 1);
+  const dim3 bgrid((unsigned)n_blocks, (unsigned)share);
   if (dtype == 0) {
     IAMX_LAUNCH("gemv_fused_f64", k_gemv_fused<double>, bgrid, dim3(256), 0, d_blocks, d_blk_rc, n_blocks,
                 (const double *)x, (const uint8_t *)d_scratch, (double *)d_partial, M, K, nbc, cap, st, d_xzero);
@@ -540,10 +572,9 @@ IAMX_API int iamx_gemv_fused(int dtype, const iamx_lz4_job_t *d_lz4, int n_lz4, 
   int rc = iamx::ensure_init();
   if (rc) return rc;
   if (bs1 > kMaxCols) return iamx::set_error(IAMX_EINVAL, "iamx_gemv_fused: block width %d > %d", bs1, kMaxCols);
-  (void)bs0;
   if (n_blocks <= 0 || nbc <= 0) return iamx::set_error(IAMX_EINVAL, "iamx_gemv_fused: no blocks");
   return gemv_fused_launch(dtype, d_lz4, n_lz4, d_blocks, d_blk_rc, n_blocks, nbc, x, y, M, INT64_MAX, INT64_MAX,
-                           d_scratch, d_partial);
+                           d_scratch, d_partial, (int64_t)bs0 * bs1);
 }
 
 IAMX_API int iamx_opt_gemv_fused(int dtype, const iamx_lz4_job_t *d_lz4, int n_lz4, const iamx_block_job_t *d_blocks,
@@ -551,11 +582,10 @@ IAMX_API int iamx_opt_gemv_fused(int dtype, const iamx_lz4_job_t *d_lz4, int n_l
                                  void *y, int64_t M, void *d_scratch, void *d_partial, const uint8_t *d_xzero) {
   int rc = iamx::ensure_init();
   if (rc) return rc;
-  (void)bs0;
   if (bs1 > kMaxCols) return iamx::set_error(IAMX_EINVAL, "iamx_opt_gemv_fused: block width %d > %d", bs1, kMaxCols);
   if (n_blocks <= 0 || nbc <= 0 || !d_xzero) return iamx::set_error(IAMX_EINVAL, "iamx_opt_gemv_fused: no blocks");
   return gemv_fused_launch(dtype, d_lz4, n_lz4, d_blocks, d_blk_rc, n_blocks, nbc, x, y, M, INT64_MAX, INT64_MAX,
-                           d_scratch, d_partial, d_xzero);
+                           d_scratch, d_partial, (int64_t)bs0 * bs1, d_xzero);
 }
 
 IAMX_API int64_t iamx_gemv_fused_noalloc_limit(void) { return (int64_t)kNoAllocBytes; }
@@ -564,7 +594,6 @@ IAMX_API int iamx_gemv_fused_noalloc(int dtype, const iamx_lz4_job_t *d_lz4, int
                                      const iamx_block_job_t *d_blocks, const int32_t *d_blk_rc, int n_blocks, int nbc,
                                      int bs0, int bs1, const void *x, int64_t K, void *y, int64_t M,
                                      int64_t scratch_bytes) {
-  (void)bs0;
   if (!iamx::initialized()) return iamx::set_error(IAMX_EINVAL, "iamx_gemv_fused_noalloc: call iamx_init first");
   if (dtype != 0 && dtype != 1) return iamx::set_error(IAMX_EINVAL, "iamx_gemv_fused_noalloc: dtype %d", dtype);
   if (bs1 > kMaxCols || bs1 < 1)
@@ -587,7 +616,7 @@ IAMX_API int iamx_gemv_fused_noalloc(int dtype, const iamx_lz4_job_t *d_lz4, int
   IAMX_LAUNCH("gemv_noalloc_clear", k_zero_words, dim3((unsigned)((pn + 1023) / 1024 < 4096 ? (pn + 1023) / 1024 : 4096)),
               dim3(256), 0, (uint32_t *)(base + poff), pn);
   return gemv_fused_launch(dtype, d_lz4, n_lz4, d_blocks, d_blk_rc, n_blocks, nbc, x, y, M, K, scratch_bytes, base,
-                           base + poff);
+                           base + poff, (int64_t)bs0 * bs1);
 }
 
 }  // extern "C"

@@ -38,3 +38,25 @@ def test_gemv_block_shapes_exact(case, dt, filters):
     cx = ia.Container.from_numpy(ctx, x, (chunks[1],), (blocks[1],))
     y = ia.matmul(cA, cx, (chunks[0],), (blocks[0],)).to_numpy()
     assert np.array_equal(y, (A.astype(np.float64) @ x.astype(np.float64)).astype(dt))
+
+
+# unfiltered blocks read eight elements at once, in one stream and in one a byte (whose ends fall inside groups of
+# eight, or do not), and few blocks of just under, at and over two workgroups' work
+@pytest.mark.parametrize("split", [ia.ALWAYS_SPLIT, ia.NEVER_SPLIT], ids=["split", "one"])
+@pytest.mark.parametrize("filters", [ia.COMP_SHUFFLE, ia.COMP_BITSHUFFLE, 0], ids=["bytes", "bits", "none"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,block", [((40, 37), (20, 15)), ((64, 64), (32, 32)), ((126, 130), (63, 65)),
+                                         ((128, 128), (64, 64)), ((91, 90), (91, 90)), ((90, 92), (90, 91)),
+                                         ((270, 9), (135, 9)), ((200, 7), (100, 7))])
+def test_gemv_unfiltered_and_shared_blocks(shape, block, dt, filters, split):
+    print(f"case: gemv {shape} blocks {block} {np.dtype(dt).name} filters {filters} split {split}", flush=True)
+    rng = np.random.default_rng(shape[0] * 1009 + block[1])
+    A = (rng.integers(-9, 10, shape) * 0.25).astype(dt)
+    A[: shape[0] // 3] *= 2.0 ** 20
+    A[-1] = 0
+    x = rng.integers(-4, 5, shape[1]).astype(dt)
+    ctx = ia.Context(clevel=5, filters=filters, splitmode=split)
+    cA = ia.Container.from_numpy(ctx, A, shape, block)
+    cx = ia.Container.from_numpy(ctx, x, (shape[1],), (block[1],))
+    y = ia.matmul(cA, cx, (shape[0],), (block[0],)).to_numpy()
+    assert np.array_equal(y, (A.astype(np.float64) @ x.astype(np.float64)).astype(dt))
