@@ -34,7 +34,8 @@ IAMX_API int iamx_init(void);
 IAMX_API const char *iamx_last_error(void);
 IAMX_API int iamx_device_info(char *name, int namelen, int *cus, char *arch, int archlen);
 /* iamx_free keeps blocks of up to 64 MiB (256 MiB in all) for later calls of
- * iamx_malloc, once the device has finished the work queued before it. */
+ * iamx_malloc, once the device has finished the work queued before it; they go
+ * back when an allocation here or of a workspace fails. */
 IAMX_API void *iamx_malloc(size_t bytes);
 IAMX_API void iamx_free(void *dptr);
 IAMX_API int iamx_h2d(void *dst, const void *src, size_t bytes);
@@ -80,7 +81,8 @@ IAMX_API int iamx_use_stream(int side);
 IAMX_API void *iamx_upload_host(int stage, size_t bytes);
 IAMX_API int iamx_upload(int stage, void *d_dst, size_t bytes);
 IAMX_API int iamx_upload_release(int stage);
-/* hipMemGetInfo of the library's device */
+/* hipMemGetInfo of the library's device; the blocks that iamx_free keeps count
+ * as free */
 IAMX_API int iamx_mem_info(size_t *free_bytes, size_t *total_bytes);
 /* Scratch that lives until iamx_shutdown; grown (never shrunk) on demand.
  * Each slot is independent of the others. */

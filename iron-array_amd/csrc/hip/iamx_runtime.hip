@@ -184,7 +184,7 @@ static Workspace g_ws[IAMX_WORKSPACES];
 // 20-300 us.  A block is kept only after the device has finished everything
 // queued before its free (what hipFree waits for too), so its next owner may
 // use it on any stream.  All are given back at shutdown, and when an allocation
-// fails.
+// of a block or a workspace fails; until then they count as free memory.
 constexpr size_t kKeepBytes = (size_t)256 << 20, kKeepBlock = (size_t)64 << 20;
 static std::mutex g_blocks_mu;
 static std::unordered_map<void *, size_t> g_live_blocks;  // sizes of the blocks handed out
@@ -203,6 +203,19 @@ static void release_kept() {
   for (auto &b : g_kept_blocks) (void)hipFree(b.second);
   g_kept_blocks.clear();
   g_kept_bytes = 0;
+}
+
+// hipMalloc, once more without the kept blocks (g_blocks_mu held); null if it fails
+static void *device_alloc(size_t bytes) {
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess && g_kept_bytes) {
+    release_kept();
+    e = hipMalloc(&p, bytes);
+  }
+  if (e == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 }  // namespace iamx
@@ -239,13 +252,8 @@ IAMX_API void *iamx_malloc(size_t bytes) {
     g_kept_blocks.erase(kept);
     return p;
   }
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess && g_kept_bytes) {
-    release_kept();
-    e = hipMalloc(&p, want);
-  }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  p = device_alloc(want);
+  if (!p) {
     set_error(IAMX_ENOMEM, "hipMalloc(%zu) failed", bytes);
     return nullptr;
   }
@@ -529,6 +537,10 @@ IAMX_API int iamx_mem_info(size_t *free_bytes, size_t *total_bytes) {
   if (rc) return rc;
   size_t f = 0, t = 0;
   IAMX_HIP_CHECK(hipMemGetInfo(&f, &t));
+  {
+    std::lock_guard<std::mutex> lk(g_blocks_mu);
+    f += g_kept_bytes;
+  }
   if (free_bytes) *free_bytes = f;
   if (total_bytes) *total_bytes = t;
   return IAMX_OK;
@@ -545,8 +557,11 @@ IAMX_API void *iamx_workspace(int slot, size_t bytes) {
     w.bytes = 0;
   }
   size_t want = bytes + bytes / 8 + 4096;
-  if (hipMalloc(&w.ptr, want) != hipSuccess) {
-    w.ptr = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(g_blocks_mu);
+    w.ptr = device_alloc(want);
+  }
+  if (!w.ptr) {
     set_error(IAMX_ENOMEM, "workspace %d: hipMalloc(%zu) failed", slot, want);
     return nullptr;
   }
