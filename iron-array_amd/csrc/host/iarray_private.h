@@ -149,14 +149,6 @@ void iax_parallel_for(int nthreads, int64_t n, iax_task_fn fn, void *ctx);
 double iax_now(void);
 /* Order LZ4 decode jobs by compressed size, largest first. */
 void iax_sort_lz4_jobs(iamx_lz4_job_t *jobs, int64_t n);
-/* Download `total` bytes of d_src into the pinned staging buffer in pieces
- * and run fn(ctx, task, worker) for each of `ntasks` tasks as soon as the
- * piece holding its bytes (up to task_end[task]) has landed, so the copy of
- * later pieces overlaps the work on earlier ones.  *host receives the
- * staging buffer (owned by the device runtime). */
-ina_rc_t iax_download_pipelined(const void *d_src, size_t total, const int64_t *task_end, int64_t ntasks,
-                                int nthreads, iax_task_fn fn, void *ctx, uint8_t **host);
-
 /* Device work that fills part of a buffer before it is downloaded: enqueue
  * (asynchronously) what produces the bytes of tasks [t0, t1) of panel k;
  * returns an iamx error code. */

@@ -76,3 +76,30 @@ def test_kept_blocks_are_given_back_to_an_allocation(fake_device, what):
     assert {what}
     assert fake.fake_device_used() <= 1024 * MB
     """)
+
+
+RESULT = """
+    def result(rows):
+        a = np.zeros((rows, 65536 // 4), np.float32)
+        c = ia.Container.from_numpy(ia.Context(clevel=0, filters=0), a, (min(rows, 64), a.shape[1]), (8, 4096))
+        return c.to_numpy().view(np.uint32).ravel()  # the device image: nothing wrote over the numbers it began with
+"""
+
+
+@pytest.mark.parametrize("rows", [32, 33, 1023, 1024, 1025, 1536, 1537, 2048, 4000])
+def test_results_of_any_size_pin_a_bounded_ring(fake_device, rows):
+    """64 KiB a row: one piece, all slots of the ring, one more, and rings full."""
+    fake_device(RESULT + f"""
+    fake.fake_limits(4096 * MB, 4096 * MB)
+    got = result({rows})
+    assert np.array_equal(got, np.arange(got.size, dtype=np.uint32))
+    assert fake.fake_pinned_peak() < 120 * MB
+    """)
+
+
+def test_result_without_pinned_memory_for_the_ring(fake_device):
+    fake_device(RESULT + """
+    fake.fake_limits(4096 * MB, 50 * MB)  # two upload stages of 16 MiB and a little more
+    got = result(2048)
+    assert np.array_equal(got, np.arange(got.size, dtype=np.uint32))
+    """)

@@ -53,3 +53,14 @@ def test_blocks_reused_by_other_containers():
         a, c = live[int(rng.integers(0, len(live)))]
         p = ia.matmul(c, c, a.shape, (min(a.shape[0], 64),) * 2)
         assert np.array_equal(p.to_numpy(), a @ a)
+
+
+@pytest.mark.parametrize("rows", [32_767, 32_768, 32_769, 49_160, 70_001])
+def test_results_through_the_ring(rows):
+    """Results of just under, at and over the 64 MiB of the ring of pinned pieces, and some halves more."""
+    rng = np.random.default_rng(rows)
+    a = rng.integers(-2 ** 62, 2 ** 62, (rows, 256))
+    ctx = ia.Context(clevel=0, filters=0)
+    c = ia.Container.from_numpy(ctx, a, (min(rows, 4096), 256), (64, 256))
+    for _ in range(2):
+        assert np.array_equal(c.to_numpy(), a)
