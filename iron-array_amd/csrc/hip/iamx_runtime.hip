@@ -324,6 +324,7 @@ IAMX_API void *iamx_host_buffer(size_t bytes) {
   }
   const size_t want = bytes + bytes / 8 + 4096;
   if (hipHostMalloc(&g_host_buf, want, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch reports it
     g_host_buf = nullptr;
     set_error(IAMX_ENOMEM, "hipHostMalloc(%zu) failed", want);
     return nullptr;
@@ -350,6 +351,7 @@ IAMX_API void *iamx_host_direct(size_t bytes, void **dev) {
     }
     const size_t want = bytes + bytes / 8 + 4096;
     if (hipHostMalloc(&g_direct_buf, want, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
       g_direct_buf = nullptr;
       set_error(IAMX_ENOMEM, "hipHostMalloc(%zu, mapped) failed", want);
       return nullptr;
@@ -496,6 +498,7 @@ IAMX_API void *iamx_upload_host(int stage, size_t bytes) {
   }
   const size_t want = bytes + bytes / 8 + 4096;
   if (hipHostMalloc(&g_up_host[stage], want, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
     g_up_host[stage] = nullptr;
     set_error(IAMX_ENOMEM, "hipHostMalloc(%zu) failed", want);
     return nullptr;

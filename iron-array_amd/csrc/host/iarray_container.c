@@ -338,9 +338,11 @@ ina_rc_t iax_materialize(iarray_container_t *c) {
 /* ---- uploads ---------------------------------------------------------------------------------- *
  * Host pieces to their places behind one device address, through the two
  * pinned upload stages: the host threads fill one stage while the other is
- * copied, and the library stream waits for the copies.  Copying the pieces
- * into one pageable buffer and from there took 2.4 ms for the 30 MB of a
- * 2000x2000 float64 product; the host link carries them in 0.55. */
+ * copied.  Both the library stream and, before it returns, the host wait for the
+ * copies (any stream may read them then); where a stage cannot be had the
+ * pieces are copied from where they are.  Copying the pieces into one pageable
+ * buffer and from there took 2.4 ms for the 30 MB of a 2000x2000 float64
+ * product; the host link carries them in 0.55. */
 #define IAX_UPLOAD_PIECE ((size_t)16 << 20)
 #define IAX_COPY_TASK ((size_t)512 << 10)
 
@@ -385,8 +387,8 @@ int iax_upload(void *d_dst, const iax_piece_t *pieces, int64_t n, int nthreads) 
     int64_t j = i;
     while (j < nt && t[j].off + t[j].len - t[i].off <= stage_bytes) j++;
     uint8_t *h = (uint8_t *)iamx_upload_host(stage, stage_bytes);
-    if (!h) {
-      e = IAMX_ENOMEM;
+    if (!h) { /* no pinned stage: from the pieces themselves */
+      for (; i < nt && !e; i++) e = iamx_h2d((uint8_t *)d_dst + t[i].off, t[i].src, t[i].len);
       break;
     }
     copy_ctx_t x = {t + i, h, t[i].off};
@@ -1502,8 +1504,7 @@ static int64_t nitems(const iarray_container_t *c) {
  * so).  The ring bounds what a result of any size pins.  Results that fit it
  * come in pieces of 4 MiB, larger ones of 16 MiB, whose copies leave fewer gaps
  * on the link (1 GiB 28 ms by 4 MiB, 20.4 so).  A caller's buffer is always good
- * enough: where the ring cannot
- * be had it is copied to directly. */
+ * enough: where the ring cannot be had it is copied to directly. */
 #define IAX_DOWN_RING ((size_t)64 << 20)
 #define IAX_DOWN_SLOTS 16
 

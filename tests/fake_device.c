@@ -19,6 +19,9 @@ void fake_limits(size_t device, size_t pinned) {
 size_t fake_device_used(void) { return dev_used; }
 size_t fake_pinned_peak(void) { return pin_peak; }
 
+static __thread hipError_t last = hipSuccess;
+static hipError_t error(hipError_t e) { return last = e; }
+
 static void *take(size_t n, size_t *used, size_t limit) {
   pthread_mutex_lock(&mu);
   size_t *p = *used + n <= limit ? aligned_alloc(4096, ((n + 4095) & ~(size_t)4095) + 4096) : NULL;
@@ -39,13 +42,13 @@ static void give(void *v, size_t *used) {
 }
 
 hipError_t hipMalloc(void **p, size_t n) {
-  if (!(*p = take(n, &dev_used, dev_limit))) return hipErrorOutOfMemory;
+  if (!(*p = take(n, &dev_used, dev_limit))) return error(hipErrorOutOfMemory);
   for (size_t i = 0; i < n / 4; i++) ((unsigned *)*p)[i] = (unsigned)i;
   return hipSuccess;
 }
 hipError_t hipFree(void *p) { return give(p, &dev_used), hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) {
-  return (*p = take(n, &pin_used, pin_limit)) ? hipSuccess : hipErrorOutOfMemory;
+  return (*p = take(n, &pin_used, pin_limit)) ? hipSuccess : error(hipErrorOutOfMemory);
 }
 hipError_t hipHostFree(void *p) { return give(p, &pin_used), hipSuccess; }
 hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned flags) { return *d = h, hipSuccess; }
@@ -70,7 +73,10 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int d) {
   return hipSuccess;
 }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = last;
+  return last = hipSuccess, e;
+}
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 static char symbol[1 << 20];
 hipError_t hipGetSymbolAddress(void **p, const void *s) { return *p = symbol, hipSuccess; }

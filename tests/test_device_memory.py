@@ -20,6 +20,7 @@ def fake_device(tmp_path_factory):
                            "-o", so, os.path.join(HERE, "fake_device.c")])
     head = textwrap.dedent(f"""
         import ctypes, sys
+        sys.path.insert(0, {HERE!r})
         sys.path.insert(0, {os.path.join(os.path.dirname(HERE), "iron-array_amd")!r})
         fake = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
         fake.fake_limits.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
@@ -102,4 +103,28 @@ def test_result_without_pinned_memory_for_the_ring(fake_device):
     fake.fake_limits(4096 * MB, 50 * MB)  # two upload stages of 16 MiB and a little more
     got = result(2048)
     assert np.array_equal(got, np.arange(got.size, dtype=np.uint32))
+    """)
+
+
+@pytest.mark.parametrize("pinned", [1, 10, 20, 1024])
+@pytest.mark.parametrize("rows", [1, 40, 512, 700])
+def test_uploads_with_and_without_pinned_stages(fake_device, rows, pinned):
+    """The blocks of a container stored raw, of 64 KiB to 44 MiB, read back from
+    the device addresses that its plan names, with no stage, one of two, and both."""
+    fake_device(f"""
+    from test_zz_no_alloc import DevicePlan
+    class Job(ctypes.Structure):
+        _fields_ = [("src", ctypes.c_uint64 * 8), ("rest", ctypes.c_uint8 * 64)]
+    fake.fake_limits(4096 * MB, {pinned} * MB)
+    rng = np.random.default_rng(1)
+    a = rng.integers(0, 2 ** 62, ({rows}, 8192))
+    c = ia.Container.from_numpy(ia.Context(clevel=0, filters=0), a, (min({rows}, 16), 8192), (1, 8192))
+    p = DevicePlan()
+    assert ia.lib().iarray_container_device_plan(c.ptr, ctypes.cast(ctypes.byref(p), ctypes.c_void_p)) == 0
+    jobs = (Job * p.n_blocks).from_address(p.blocks)
+    assert p.n_blocks == {rows}
+    for i in range({rows}):
+        got = np.frombuffer((ctypes.c_uint8 * 65536).from_address(jobs[i].src[0]), np.int64)
+        assert np.array_equal(got, a[i]), i
+    c.to_numpy()  # launches and their error checks, after the allocations that failed
     """)
