@@ -149,6 +149,11 @@ typedef struct iamx_block_job_s {
 
 IAMX_API int iamx_decode(const iamx_lz4_job_t *d_lz4, int n_lz4, const iamx_block_job_t *d_blocks, int n_blocks,
                          void *d_scratch, void *d_dst);
+/* The streams of a table of BloscLZ jobs only (any other flags
+ * IAMX_STATUS_CODEC).  iamx_decode and iamx_gemv_fused decode such jobs too,
+ * beside LZ4 ones; for more than 12 streams a CU of them alone this is faster,
+ * and those are then called with n_lz4 = 0. */
+IAMX_API int iamx_decode_blosclz(const iamx_lz4_job_t *d_jobs, int n_jobs, void *d_scratch);
 
 /* ---- GEMM / GEMV -------------------------------------------------------------
  * Replaces the per-C-block cblas_?gemm of the gemm branch

@@ -560,6 +560,8 @@ void iax_sort_lz4_jobs(iamx_lz4_job_t *jobs, int64_t n) {
 static size_t place_plan(jobs_t *j, iax_plan_t *plan, uint8_t *d_base, size_t off, iax_piece_t *pieces) {
   iax_sort_lz4_jobs(j->lz4, j->n_lz4);
   plan->n_lz4 = (int)j->n_lz4;
+  plan->blosclz = j->n_lz4 > 0;
+  for (int64_t i = 0; i < j->n_lz4 && plan->blosclz; i++) plan->blosclz = j->lz4[i].codec == IAMX_CODEC_BLOSCLZ;
   plan->n_blocks = (int)j->n_blk;
   plan->scratch_bytes = j->scratch;
   const void *src[3] = {j->lz4, j->blk, j->rc4};
@@ -575,6 +577,11 @@ static size_t place_plan(jobs_t *j, iax_plan_t *plan, uint8_t *d_base, size_t of
   plan->d_blocks = (iamx_block_job_t *)(d_base + at[1]);
   plan->d_blk_rc = (int32_t *)(d_base + at[2]);
   return off;
+}
+
+int iax_plan_streams(const iax_plan_t *p, void *d_scratch, int *n_lz4) {
+  *n_lz4 = p->blosclz ? 0 : p->n_lz4;
+  return p->blosclz ? iamx_decode_blosclz(p->d_lz4, p->n_lz4, d_scratch) : 0;
 }
 
 /* Device addresses inside the arena were planned relative to its start. */
@@ -859,7 +866,8 @@ ina_rc_t iax_decode_dense(iarray_container_t *c, void *d_dst, int scratch_slot) 
   if (INA_FAILED(rc)) return rc;
   void *scratch = iamx_workspace(scratch_slot, (size_t)c->plan.scratch_bytes + 16);
   if (!scratch) return iax_dev_error(IAMX_ENOMEM, "decode scratch");
-  int e = iamx_decode(c->plan.d_lz4, c->plan.n_lz4, c->plan.d_blocks, c->plan.n_blocks, scratch, d_dst);
+  int n_lz4, e = iax_plan_streams(&c->plan, scratch, &n_lz4);
+  if (!e) e = iamx_decode(c->plan.d_lz4, n_lz4, c->plan.d_blocks, c->plan.n_blocks, scratch, d_dst);
   if (e) return iax_dev_error(e, "decode");
   return INA_SUCCESS;
 }
@@ -932,7 +940,8 @@ static ina_rc_t decode_transposed(iarray_container_t *v, iarray_container_t *bas
   }
   void *scratch = iamx_workspace(0, (size_t)p->scratch_bytes + 16);
   if (!scratch) return iax_dev_error(IAMX_ENOMEM, "decode scratch");
-  int e = iamx_decode(p->d_lz4, p->n_lz4, v->d_tblocks, p->n_blocks, scratch, dst);
+  int n_lz4, e = iax_plan_streams(p, scratch, &n_lz4);
+  if (!e) e = iamx_decode(p->d_lz4, n_lz4, v->d_tblocks, p->n_blocks, scratch, dst);
   if (e) return iax_dev_error(e, "decode");
   return INA_SUCCESS;
 }
@@ -1927,7 +1936,8 @@ INA_API(ina_rc_t) iarray_decode_chunks_flat(iarray_context_t *ctx, int64_t nchun
   }
   if (INA_SUCCEED(rc)) {
     void *scratch = iamx_workspace(0, (size_t)plan.scratch_bytes + 16);
-    int e = scratch ? iamx_decode(plan.d_lz4, plan.n_lz4, plan.d_blocks, plan.n_blocks, scratch, d_out) : IAMX_ENOMEM;
+    int n_lz4, e = scratch ? iax_plan_streams(&plan, scratch, &n_lz4) : IAMX_ENOMEM;
+    if (!e) e = iamx_decode(plan.d_lz4, n_lz4, plan.d_blocks, plan.n_blocks, scratch, d_out);
     if (!e) e = iamx_d2h(out, d_out, (size_t)nbytes_total);
     if (e) rc = iax_dev_error(e, "flat decode");
     if (INA_SUCCEED(rc)) rc = check_decode_status();

@@ -399,12 +399,14 @@ static ina_rc_t run_gemv(iarray_container_t *a, iarray_container_t *x, iarray_co
       iax_operand_forget(6);
       void *partial = iamx_workspace(6, pbytes + 16);
       if (!scratch || !partial) return iax_dev_error(IAMX_ENOMEM, "gemv scratch");
+      int n_lz4 = 0;
       if (!e) e = iamx_memset(partial, 0, pbytes);
+      if (!e && p->n_blocks > 0) e = iax_plan_streams(p, scratch, &n_lz4);
       if (!e && p->n_blocks > 0 && d_xzero)
-        e = iamx_opt_gemv_fused(dt, p->d_lz4, p->n_lz4, p->d_blocks, p->d_blk_rc, p->n_blocks, (int)p->nbcols,
+        e = iamx_opt_gemv_fused(dt, p->d_lz4, n_lz4, p->d_blocks, p->d_blk_rc, p->n_blocks, (int)p->nbcols,
                                 (int)a->block[0], (int)a->block[1], dx, dy, M, scratch, partial, d_xzero);
       else if (!e && p->n_blocks > 0)
-        e = iamx_gemv_fused(dt, p->d_lz4, p->n_lz4, p->d_blocks, p->d_blk_rc, p->n_blocks, (int)p->nbcols,
+        e = iamx_gemv_fused(dt, p->d_lz4, n_lz4, p->d_blocks, p->d_blk_rc, p->n_blocks, (int)p->nbcols,
                             (int)a->block[0], (int)a->block[1], dx, dy, M, scratch, partial);
       else if (!e)
         e = iamx_memset(dy, 0, (size_t)(M * a->itemsize));

@@ -25,6 +25,7 @@ struct iarray_context_s {
 typedef struct iax_plan_s {
   iamx_lz4_job_t *d_lz4;
   int n_lz4;
+  int blosclz; /* every stream is a BloscLZ one */
   iamx_block_job_t *d_blocks;
   int n_blocks;
   int32_t *d_blk_rc; /* (row0, col0, block column, 0) per block job, for the fused GEMV */
@@ -168,6 +169,9 @@ typedef struct {
   size_t off, len;
 } iax_piece_t;
 int iax_upload(void *d_dst, const iax_piece_t *pieces, int64_t n, int nthreads);
+/* Decodes the streams that have a pass of their own; *n_lz4 is how many are left
+ * for the entry point that follows.  Returns an iamx error code. */
+int iax_plan_streams(const iax_plan_t *p, void *d_scratch, int *n_lz4);
 /* Decode the whole (base) container into a dense row-major device buffer of
  * shape (shape0, shape1) with leading dimension shape1. */
 ina_rc_t iax_decode_dense(iarray_container_t *c, void *d_dst, int scratch_slot);

@@ -708,3 +708,41 @@ def test_zlib_chunks_are_refused(ctx):
     assert chunk[2] >> 5 == 3
     with pytest.raises(ia.IArrayError, match="codec format 3 has no GPU decoder"):
         ia.decode_chunks_flat(ctx, [chunk], len(raw))
+
+
+# ---- containers of BloscLZ streams alone: more than 12 streams a CU have a pass of their own ---------------------
+@pytest.mark.parametrize("copies", [3, 3200])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_blosclz_alone(orc, dt, copies):
+    """decode_chunks_flat, to_numpy, the transposed view and the fused GEMV of
+    operands whose chunks c-blosc 1.21 wrote with BloscLZ, few streams and many
+    (integer data: exact); a chunk cut short among them is an error."""
+    b = _libblosc()
+    if b is None:
+        pytest.skip("c-blosc 1.21 not present")
+    print(f"case: blosclz alone {np.dtype(dt).name} x {copies}", flush=True)
+    rng = np.random.default_rng(copies)
+    isz = np.dtype(dt).itemsize
+    ctx = ia.Context(clevel=5, filters=ia.COMP_SHUFFLE)
+    one = np.repeat(rng.integers(-20, 21, (48, 20, 6)), 5, axis=2).astype(dt)  # planes of runs
+    one[:, 3] = 7
+    chunks = [_cblosc_compress(b, b"blosclz", one[i].tobytes(), 5, 1, isz, 600 * isz) for i in range(48)]
+    pick = [i % 48 for i in range(copies)]
+    flat = ia.decode_chunks_flat(ctx, [chunks[i] for i in pick], copies * 600 * isz)
+    assert flat == b"".join(one[i].tobytes() for i in pick)
+    a = np.concatenate([one[i] for i in pick])
+    c = ia.Container.from_chunks(ctx, dt, a.shape, (20, 30), (20, 30), [chunks[i] for i in pick])
+    assert np.array_equal(c.to_numpy(), a)
+    assert np.array_equal(c.transpose().to_numpy(), a.T)
+    x = rng.integers(-5, 6, 30).astype(dt)
+    y = ia.matmul(c, ia.Container.from_numpy(ctx, x, (30,), (30,)), (20,), (20,)).to_numpy()
+    assert np.array_equal(y, a @ x)
+    short = bytearray(_cblosc_compress(b, b"blosclz", np.full((20, 30), 7, dt).tobytes(), 5, 1, isz, 600 * isz))
+    at = struct.unpack("<i", short[16:20])[0]
+    for _ in range(isz - 1):
+        at += 4 + struct.unpack("<i", short[at:at + 4])[0]
+    cs = struct.unpack("<i", short[at:at + 4])[0]
+    assert at + 4 + cs == len(short) and 1 < cs < 600
+    short[at:at + 4] = struct.pack("<i", cs - 1)  # the last stream lacks its last byte
+    with pytest.raises(ia.IArrayError):
+        ia.decode_chunks_flat(ctx, [chunks[i] for i in pick[:-1]] + [bytes(short)], copies * 600 * isz)
