@@ -125,8 +125,8 @@ struct Lz4Geom<1> {
 //            + t.  Sequences of at most 269 literals and 273 match bytes (one
 //            length byte each) inside the stream are decoded by rounds (`ok`).
 //   reach    each wavefront follows the sequences of its 64-position window
-//            from all 64 starts at once, by pointer doubling (at most 21
-//            hops): where the chain leaves the window or stops at a sequence
+//            from all 64 starts at once, by pointer doubling (at most 22
+//            hops, at 0, 3, .. 63): where the chain leaves the window or stops at a sequence
 //            that is not ok, and how many sequences and output bytes it
 //            passes.  None of this needs to know where the window is entered.
 //   chain    the windows' exits are then followed from the round's entry, one
@@ -189,11 +189,14 @@ struct Lz4Geom<1> {
 // other streams took 2 to 4% longer in one for both.
 //
 // Output bytes go to an LDS ring and reach the stream's scratch slot in
-// 16-byte stores whenever a quarter of the ring is pending.  An offset of more
-// than kNear reads the slot back from global memory: such a source is at least
-// 15/16 of the ring back, at most 5/16 of the ring is pending or was flushed
-// last, and the stores of the flush before that were waited for by every
-// wavefront before a barrier that precedes the read.
+// 16-byte stores whenever a quarter of the ring (FLUSH_AT) is pending.  An offset
+// of more than NEAR reads the slot back from global memory.  With several
+// wavefronts such a source must lie before the last flush, whose stores alone may
+// still be on their way: those of the flush before it were waited for by every
+// wavefront before a barrier that precedes the read.  It does: a round begins
+// with less than FLUSH_AT bytes pending, the last flush wrote at most FLUSH_AT +
+// kOut, and the byte that reads is at most kOut past the round's first, so NEAR
+// has to be twice FLUSH_AT + kOut or more (15/16 of the ring against 12/16).
 template <int NW, bool SIDEWAYS = false>
 __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__restrict__ scratch, int *status,
                                            uint8_t *lds, int32_t ahead_at) {
@@ -202,6 +205,8 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
   constexpr int32_t RING = G::kRing, RM = RING - 1;
   constexpr int32_t NEAR = RING - G::kStep;
   constexpr int32_t FLUSH_AT = RING / 4;
+  static_assert(NW == 1 || NEAR >= 2 * (FLUSH_AT + G::kOut), "a far source was stored before the last flush");
+  static_assert(G::kStep <= G::kOut, "and by the general path");
   uint8_t *ring = lds;
   uint8_t *stage = lds + RING;
   uint64_t *tab = reinterpret_cast<uint64_t *>(lds + G::kTabAt);
@@ -504,7 +509,9 @@ __device__ __forceinline__ void lz4_stream(const iamx_lz4_job_t job, uint8_t *__
           // reach: bits 0..9 the lane the chain from here has got to (64 and more
           // is a position of a later window; a start that is not ok leads to
           // itself), bits 10..26 the output bytes and bits 27..31 the sequences on
-          // the way (at most 21 of 542 bytes)
+          // the way (at most 22 of 542 bytes; over all windows kSeqs of them)
+          static_assert((64 + 2) / 3 < 32 && G::kSeqs * kSeqOut < 1 << 17, "they fit their fields");
+          static_assert(63 + kSeqIn + 64 * (NW - 1) < 1024, "and the position");
           uint32_t way = ok ? (uint32_t)(lane + adv) | ((uint32_t)len << 10) | (1u << 27) : (uint32_t)lane;
           auto hop = [&]() {
             const uint32_t f = (uint32_t)bperm((int32_t)way, (int32_t)way);
