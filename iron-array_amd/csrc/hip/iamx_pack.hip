@@ -168,6 +168,11 @@ __device__ __forceinline__ void pack_bits(const Tile &b, uint8_t *o, int32_t row
 // planes 41 to 19).  A 3001 x 2503 float32 product in blocks of 128^2 45 to 16
 // us, 4096^2 in blocks of 256^2 58 to 24, 300 x 170 float64 18.6 to 6.7; two
 // groups of 48 ragged products 56 to 14 us each.
+//
+// WIDE: elements of 4 and 8 bytes.  Other sizes, element by element, are bound by
+// the wavefronts there are: in one kernel with the wide paths they took up to 38%
+// longer (4096^2 2-byte elements, unfiltered, in blocks of 50^2 64 us, 46 alone).
+template <bool WIDE>
 __device__ __forceinline__ void pack_part(const iamx_tiling_t &t, const uint8_t *src, int64_t ld, uint8_t *o,
                                           int64_t id, int part, int parts) {
   const Tile b = tile_of(t, src, ld, id);
@@ -176,9 +181,9 @@ __device__ __forceinline__ void pack_part(const iamx_tiling_t &t, const uint8_t 
   if (t.filter == IAMX_FILTER_BITSHUFFLE) {
     const int32_t n8 = b.n - b.n % 8, rowlen = n8 / 8;
     for (int64_t g = first; g < rowlen; g += step) {
-      if (ts == 4) {
+      if (WIDE && ts == 4) {
         pack_bits<4>(b, o, rowlen, (int32_t)g);
-      } else if (ts == 8) {
+      } else if (WIDE) {
         pack_bits<8>(b, o, rowlen, (int32_t)g);
       } else {
         uint64_t v[8];
@@ -198,9 +203,9 @@ __device__ __forceinline__ void pack_part(const iamx_tiling_t &t, const uint8_t 
     return;
   }
   const bool shuffled = t.filter == IAMX_FILTER_SHUFFLE && ts > 1;
-  if (ts == 4) {
+  if (WIDE && ts == 4) {
     pack_bytes<4>(b, shuffled, o, first, step);
-  } else if (ts == 8) {
+  } else if (WIDE) {
     pack_bytes<8>(b, shuffled, o, first, step);
   } else {
     for (int64_t e = first; e < b.n; e += step) {
@@ -212,10 +217,11 @@ __device__ __forceinline__ void pack_part(const iamx_tiling_t &t, const uint8_t 
 
 // Workgroups (x, y): block id0 + x of C, part y; block `id`'s bytes go to
 // out + id * bsize.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void k_pack(iamx_tiling_t t, const uint8_t *__restrict__ src, int64_t ld,
                                               uint8_t *__restrict__ out, int64_t id0) {
   const int64_t id = id0 + blockIdx.x;
-  pack_part(t, src, ld, out + id * (t.block[0] * t.block[1] * t.typesize), id, blockIdx.y, gridDim.y);
+  pack_part<WIDE>(t, src, ld, out + id * (t.block[0] * t.block[1] * t.typesize), id, blockIdx.y, gridDim.y);
 }
 
 // The C blocks of any product: blk[2*i] = product, blk[2*i+1] = block index
@@ -225,9 +231,12 @@ __global__ __launch_bounds__(256) void k_pack_batch(const iamx_batch_pack_t *__r
                                                     uint8_t *__restrict__ out) {
   const iamx_batch_pack_t Q = packs[blk[2 * blockIdx.x]];
   const int64_t id = blk[2 * blockIdx.x + 1];
-  pack_part(Q.tiling, base_c + Q.c_off_bytes, Q.tiling.shape[1],
-            out + Q.out_off + id * (Q.tiling.block[0] * Q.tiling.block[1] * Q.tiling.typesize), id, blockIdx.y,
-            gridDim.y);
+  const iamx_tiling_t &t = Q.tiling;
+  uint8_t *o = out + Q.out_off + id * (t.block[0] * t.block[1] * t.typesize);
+  if (t.typesize == 4 || t.typesize == 8)
+    pack_part<true>(t, base_c + Q.c_off_bytes, t.shape[1], o, id, blockIdx.y, gridDim.y);
+  else
+    pack_part<false>(t, base_c + Q.c_off_bytes, t.shape[1], o, id, blockIdx.y, gridDim.y);
 }
 
 }  // namespace
@@ -248,8 +257,13 @@ IAMX_API int iamx_pack_blocks_range(const iamx_tiling_t *t, const void *d_src, i
   if (nblk == 0) return IAMX_OK;
   if (nblk < 0 || nblk > INT32_MAX) return iamx::set_error(IAMX_EINVAL, "iamx_pack_blocks: bad block count");
   const int64_t parts = (t->block[0] * t->block[1] + 8 * 256 - 1) / (8 * 256);  // eight elements a thread
-  IAMX_LAUNCH("pack_blocks", k_pack, dim3((unsigned)nblk, (unsigned)(parts < 1024 ? parts : 1024)), dim3(256), 0, *t,
-              (const uint8_t *)d_src, src_ld, (uint8_t *)d_out, chunk_begin * nbpc);
+  const dim3 grid((unsigned)nblk, (unsigned)(parts < 1024 ? parts : 1024));
+  if (t->typesize == 4 || t->typesize == 8)
+    IAMX_LAUNCH("pack_blocks", k_pack<true>, grid, dim3(256), 0, *t, (const uint8_t *)d_src, src_ld, (uint8_t *)d_out,
+                chunk_begin * nbpc);
+  else
+    IAMX_LAUNCH("pack_blocks", k_pack<false>, grid, dim3(256), 0, *t, (const uint8_t *)d_src, src_ld, (uint8_t *)d_out,
+                chunk_begin * nbpc);
   return IAMX_OK;
 }
 
