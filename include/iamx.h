@@ -104,7 +104,7 @@ IAMX_API double iamx_prof_span_ms(void); /* first start .. last stop since reset
 /* ---- Blosc2 block decode --------------------------------------------------
  * Replaces the decode inside blosc2_getitem_ctx (src/linalg/iarray_gemm.c:259,
  * src/linalg/iarray_gemv.c:194) and caterva_get_slice_buffer
- * (src/iarray_container.c:704,730): LZ4 streams are decoded by one wavefront
+ * (src/iarray_container.c:704,730): LZ4 streams are decoded by one workgroup
  * each into scratch, then every block is un-shuffled / bit-un-shuffled and
  * written into its tile of a dense row-major destination (edge-trimmed). */
 typedef struct iamx_lz4_job_s {

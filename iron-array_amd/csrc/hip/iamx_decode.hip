@@ -146,13 +146,16 @@ struct Lz4Geom<1> {
 //            source written in the same step is a lower byte: the threads
 //            leave their byte, or the number of their source byte, in LDS and
 //            follow the numbers until they find a byte.
-// What bounds it where streams are few is the chain from round to round (about
-// 5200 cycles for 8 windows: header reads, 5 hops of pointer doubling, the
-// exits, the scans, the table, the sources), so its time falls with the windows
-// a round takes: a 250 KB bitshuffled float32 stream takes 451 us with one
-// wavefront, 205 with 4, 134 with 8; one sequence after the other, with 64
-// lanes copying each, took 783.  With four streams a CU it is vector issue (78%
-// of the cycles).  So a round's cost is its instructions and its waits:
+// What bounds it where streams are few is the chain from round to round (header
+// reads, 5 hops of pointer doubling, the exits, the scans, the table, the
+// sources), so its time falls with the windows a round takes: a 250 KB
+// bitshuffled float32 stream takes 451 us with one wavefront, 205 with 4, 134
+// with 8; one sequence after the other, with 64 lanes copying each, took 783.
+// With four streams of 8 wavefronts a CU it is vector issue: the vector
+// instructions of 1024 exponent planes fill 91% of their wavefronts' life at four
+// cycles each.  With 25 of one wavefront (6400 bitshuffled streams) a wavefront
+// waits 65% of its life, for LDS and for HBM, and issues 23%.  So a round's cost
+// is its instructions and its waits:
 //  - LDS words at any byte offset are two aligned reads and a byte align; one
 //    misaligned read a lane took 522 us where this takes 424 (1024 exponent
 //    planes of 64 KB of float32).
@@ -1114,7 +1117,11 @@ namespace iamx {
 // streams - / 1267 / 1273, 6400 streams - / 2101 / 1550; a ragged matrix's
 // bitshuffled float64 streams: 3072 streams - / 510 / 1011, equal ones - / 282 /
 // 232; byte planes of 16 KB of float64: 3072 streams - / 244 / 255, 4096 streams
-// - / 292 / 275.
+// - / 292 / 275.  So around the second line the count alone does not decide:
+// streams of unlike length want more wavefronts than equal ones, by up to twice
+// the time, and the jobs' sizes do not tell the two apart (lines at 24 streams a
+// CU, or four wavefronts for the longest 12 a CU, won 10 to 40% on the one and
+// lost as much on the other).
 int launch_lz4(const char *name, const iamx_lz4_job_t *d_lz4, int n_lz4, void *d_scratch, int64_t cap) {
   const int z = zstd_enabled() ? 1 : 0;
   if (n_lz4 <= 4 * g_num_cus)
